@@ -174,6 +174,17 @@ int sopht_vorticity_stretching_flux_3d(int dtype, void* const flux[3], const int
                                        const void* const velocity[3],
                                        const int64_t* velocity_strides, int64_t nz, int64_t ny,
                                        int64_t nx, double prefactor, void* stream);
+/* gen_vorticity_stretching_timestep_{euler_forward,ssprk3}_pyst_kernel_3d —
+ * .../vorticity_stretching_timestep_3d.py:10-158. scheme 0 (Euler): flux = p (w . grad) u,
+ * w += flux; mid may be NULL. scheme 1 (SSPRK3): three stages, the last with prefactor p_last;
+ * mid keeps the mid-step field and flux the last stage's flux. One pass over memory when the
+ * cells of every field are adjacent along x and no written field overlaps another operand. */
+int sopht_vorticity_stretching_timestep_3d(int dtype, int scheme, void* const w[3],
+                                           const int64_t* w_strides, const void* const u[3],
+                                           const int64_t* u_strides, void* const flux[3],
+                                           const int64_t* flux_strides, void* const mid[3],
+                                           const int64_t* mid_strides, int64_t nz, int64_t ny,
+                                           int64_t nx, double p, double p_last, void* stream);
 
 /* ---------------------------------------------------------------- free-space Poisson */
 

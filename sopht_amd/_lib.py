@@ -80,6 +80,8 @@ SIGNATURES = {
     "sopht_passive_transport_step_3d": [_i, _i, _p3, _p3, _p3, _i64, _i64, _i64, _d, _d, _vp],
     "sopht_velocity_abs_sum_max_3d": [_i, _p3, _i64, _vp, _vp, _i64, _vp, _vp],
     "sopht_vorticity_stretching_flux_3d": [_i, _p3, _pi64, _p3, _pi64, _p3, _pi64, _i64, _i64, _i64, _d, _vp],
+    "sopht_vorticity_stretching_timestep_3d": [
+        _i, _i, _p3, _pi64, _p3, _pi64, _p3, _pi64, _vp, _vp, _i64, _i64, _i64, _d, _d, _vp],
     "sopht_poisson3d_create": [_i, _i64, _i64, _i64, _d, _vp, C.POINTER(_vp)],
     "sopht_poisson3d_solve": [_vp, _vp, _pi64, _vp, _pi64, _vp],
     "sopht_poisson3d_vector_solve": [_vp, _p3, _pi64, _p3, _pi64, _vp],

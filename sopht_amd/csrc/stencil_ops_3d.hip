@@ -9,6 +9,7 @@
 #include <mutex>
 
 #include "common.h"
+#include "row_march.h"
 
 namespace sopht {
 
@@ -552,8 +553,10 @@ int eno3_adjoint_impl(void* field_adj, const int64_t* fas, void* const vel_adj[3
       s);
 }
 
+constexpr int kStretchChunk = 16;
+
 template <typename T>
-int stretching_impl(void* const flux[3], const int64_t* fs, const void* const w[3],
+int stretching_general(void* const flux[3], const int64_t* fs, const void* const w[3],
                     const int64_t* ws, const void* const u[3], const int64_t* us, int64_t nz,
                     int64_t ny, int64_t nx, T p, hipStream_t s) {
   View3<T> o0 = make_view<T>(flux[0], fs), o1 = make_view<T>(flux[1], fs), o2 = make_view<T>(flux[2], fs);
@@ -584,6 +587,86 @@ int stretching_impl(void* const flux[3], const int64_t* fs, const void* const w[
         o2(z, y, x) = T(0);
       },
       s);
+}
+
+// The row-vector kernel where the rows allow it (cells adjacent along x, at least one vector
+// per row, outputs apart from the velocity), else one thread per cell.
+template <typename T>
+int stretching_impl(void* const flux[3], const int64_t* fs, const void* const w[3],
+                    const int64_t* ws, const void* const u[3], const int64_t* us, int64_t nz,
+                    int64_t ny, int64_t nx, T p, hipStream_t s) {
+  bool rows = row_box_ok<T>(nz, ny, nx) && row_strides_ok(fs, nz, ny, nx) && row_strides_ok(ws, nz, ny, nx) &&
+              row_strides_ok(us, nz, ny, nx);
+  if (!rows) return stretching_general<T>(flux, fs, w, ws, u, us, nz, ny, nx, p, s);
+  const RowGeo g = row_geo<T>(nz, ny, nx, kStretchChunk);
+  k_stretch_rows<T, 0><<<row_blocks(g), kRowThreads, 0, s>>>(g, rows3<T>(u, us), rows3<T>(w, ws), Rows3<T>{},
+                                                            rows3<T>(flux, fs), Rows3<T>{}, p, p);
+  SOPHT_CHECK_LAUNCH();
+  return SOPHT_OK;
+}
+
+template <typename T>
+int axpby(void* out, const int64_t* os, const void* a, const int64_t* as, const void* b, const int64_t* bs,
+          int64_t nz, int64_t ny, int64_t nx, T ta, T tb, hipStream_t s) {
+  View3<T> o = make_view<T>(out, os), x1 = make_view<T>(a, as), x2 = make_view<T>(b, bs);
+  return launch_box(
+      0, 0, 0, nz, ny, nx,
+      [=] __device__(int64_t z, int64_t y, int64_t x) { o(z, y, x) = ta * x1(z, y, x) + tb * x2(z, y, x); }, s);
+}
+
+// Euler (scheme 0) and SSPRK3 (scheme 1) stretching steps. One pass where the row-vector
+// kernel takes the fields and none of the fields it writes meets another operand; otherwise
+// the sequence of fluxes, sums and axpbys of the reference, which reads and writes in its order.
+template <typename T>
+int stretching_step_impl(int scheme, void* const w[3], const int64_t* ws, const void* const u[3],
+                         const int64_t* us, void* const flux[3], const int64_t* fs, void* const mid[3],
+                         const int64_t* ms, int64_t nz, int64_t ny, int64_t nx, T p, T p_last, hipStream_t s) {
+  bool rows = row_box_ok<T>(nz, ny, nx) && row_strides_ok(fs, nz, ny, nx) && row_strides_ok(ws, nz, ny, nx) &&
+              row_strides_ok(us, nz, ny, nx) && (scheme == 0 || row_strides_ok(ms, nz, ny, nx));
+  for (int a = 0; rows && a < 3; ++a)
+    for (int b = 0; rows && b < 3; ++b) {
+      auto meet = [&](const void* q, const int64_t* qs, const void* r, const int64_t* rs) {
+        return fields_meet<T>(q, qs, r, rs, nz, ny, nx);
+      };
+      rows = !meet(w[a], ws, u[b], us) && !meet(w[a], ws, flux[b], fs) && !meet(flux[a], fs, u[b], us);
+      if (a != b) rows = rows && !meet(w[a], ws, w[b], ws) && !meet(flux[a], fs, flux[b], fs);
+      if (scheme == 1)
+        rows = rows && !meet(mid[a], ms, w[b], ws) && !meet(mid[a], ms, u[b], us) && !meet(mid[a], ms, flux[b], fs) &&
+               (a == b || !meet(mid[a], ms, mid[b], ms));
+    }
+  if (rows) {
+    const RowGeo g = row_geo<T>(nz, ny, nx, kStretchChunk);
+    const void* const wc[3] = {w[0], w[1], w[2]};
+    if (scheme == 0)
+      k_stretch_rows<T, 1><<<row_blocks(g), kRowThreads, 0, s>>>(g, rows3<T>(u, us), rows3<T>(wc, ws), rows3<T>(w, ws),
+                                                                rows3<T>(flux, fs), Rows3<T>{}, p, p);
+    else
+      k_stretch_rows<T, 2><<<row_blocks(g), kRowThreads, 0, s>>>(g, rows3<T>(u, us), rows3<T>(wc, ws), rows3<T>(w, ws),
+                                                                rows3<T>(flux, fs), rows3<T>(mid, ms), p, p_last);
+    SOPHT_CHECK_LAUNCH();
+    return SOPHT_OK;
+  }
+  int rc = SOPHT_OK;
+  auto add = [&](void* const o[3], const int64_t* os, const void* const a[3], const int64_t* as, T ta,
+                 const void* const b[3], const int64_t* bs, T tb) {
+    for (int c = 0; c < 3 && !rc; ++c) rc = axpby<T>(o[c], os, a[c], as, b[c], bs, nz, ny, nx, ta, tb, s);
+  };
+  auto stage = [&](void* const v[3], const int64_t* vs, T q) {
+    if (!rc) rc = stretching_impl<T>(flux, fs, v, vs, u, us, nz, ny, nx, q, s);
+  };
+  stage(w, ws, p);
+  if (scheme == 0) {
+    add(w, ws, w, ws, T(1), flux, fs, T(1));
+    return rc;
+  }
+  add(mid, ms, w, ws, T(1), flux, fs, T(1));
+  stage(mid, ms, p);
+  add(mid, ms, mid, ms, T(1), flux, fs, T(1));
+  add(mid, ms, w, ws, T(0.75), mid, ms, T(0.25));
+  stage(mid, ms, p_last);
+  add(mid, ms, mid, ms, T(1), flux, fs, T(1));
+  add(w, ws, w, ws, T(1.0 / 3.0), mid, ms, T(2.0 / 3.0));
+  return rc;
 }
 
 
@@ -882,6 +965,17 @@ int sopht_vorticity_stretching_flux_3d(int dtype, void* const flux[3], const int
                                        int64_t ny, int64_t nx, double p, void* stream) {
   REQUIRE_GRID(nz, ny, nx);
   DISPATCH(dtype, stretching_impl<T>(flux, fs, w, ws, u, us, nz, ny, nx, T(p), as_stream(stream)));
+}
+
+int sopht_vorticity_stretching_timestep_3d(int dtype, int scheme, void* const w[3], const int64_t* ws,
+                                           const void* const u[3], const int64_t* us, void* const flux[3],
+                                           const int64_t* fs, void* const mid[3], const int64_t* ms, int64_t nz,
+                                           int64_t ny, int64_t nx, double p, double p_last, void* stream) {
+  REQUIRE_GRID(nz, ny, nx);
+  SOPHT_REQUIRE(scheme == 0 || scheme == 1, "scheme must be 0 (Euler) or 1 (SSPRK3)");
+  SOPHT_REQUIRE(scheme == 0 || (mid != nullptr && ms != nullptr), "SSPRK3 needs a mid-step field");
+  DISPATCH(dtype, stretching_step_impl<T>(scheme, w, ws, u, us, flux, fs, mid, ms, nz, ny, nx, T(p), T(p_last),
+                                          as_stream(stream)));
 }
 
 int sopht_laplacian_filter_3d(int dtype, int filter_order, int filter_type, void* field,

@@ -603,15 +603,20 @@ def gen_vorticity_stretching_timestep_euler_forward_pyst_kernel_3d(
     num_threads: bool | int = False,
     fixed_grid_size: tuple[int, int, int] | bool = False,
 ) -> Callable:
-    """``vorticity_stretching_timestep_3d.py:10-55``."""
-    flux = gen_vorticity_stretching_flux_pyst_kernel_3d(real_t)
-    add = gen_elementwise_sum_pyst_kernel_3d(real_t, field_type="vector")
+    """``vorticity_stretching_timestep_3d.py:10-55``: flux into its buffer, then
+    ``vorticity += flux``, in one pass."""
+    tag = L.dtype_tag(real_t)
 
     def vorticity_stretching_timestep_euler_forward_pyst_kernel_3d(
         vorticity_field, velocity_field, vorticity_stretching_flux_field, dt_by_2_dx: float
     ) -> None:
-        flux(vorticity_stretching_flux_field, vorticity_field, velocity_field, dt_by_2_dx)
-        add(vorticity_field, vorticity_field, vorticity_stretching_flux_field)
+        nz, ny, nx = _shape3(vorticity_field)
+        f = vorticity_stretching_flux_field
+        L.call("sopht_vorticity_stretching_timestep_3d", tag, 0, L.comps(vorticity_field),
+               L.strides3(vorticity_field[0]), L.comps(velocity_field), L.strides3(velocity_field[0]),
+               L.comps(f), L.strides3(f[0]), None, None, nz, ny, nx, float(dt_by_2_dx),
+               float(dt_by_2_dx), L.stream_ptr())
+        L.written(vorticity_field, f)
 
     return vorticity_stretching_timestep_euler_forward_pyst_kernel_3d
 
@@ -624,23 +629,19 @@ def gen_vorticity_stretching_timestep_ssprk3_pyst_kernel_3d(
 ) -> Callable:
     """``vorticity_stretching_timestep_3d.py:58-158`` (both mid-step views alias
     ``midstep_buffer_vector_field``; third stage prefactor ``dt_by_2_dx * 0.5``)."""
-    flux = gen_vorticity_stretching_flux_pyst_kernel_3d(real_t)
-    add = gen_elementwise_sum_pyst_kernel_3d(real_t, field_type="vector")
-    saxpby = gen_elementwise_saxpby_pyst_kernel_3d(real_t, field_type="vector")
+    tag = L.dtype_tag(real_t)
     m = midstep_buffer_vector_field
 
     def vorticity_stretching_timestep_ssprk3_pyst_kernel_3d(
         vorticity_field, velocity_field, vorticity_stretching_flux_field, dt_by_2_dx: float
     ) -> None:
+        nz, ny, nx = _shape3(vorticity_field)
         f = vorticity_stretching_flux_field
-        flux(f, vorticity_field, velocity_field, dt_by_2_dx)
-        add(m, vorticity_field, f)
-        flux(f, m, velocity_field, dt_by_2_dx)
-        add(m, m, f)
-        saxpby(m, vorticity_field, m, 0.75, 0.25)
-        flux(f, m, velocity_field, dt_by_2_dx * 0.5)
-        add(m, m, f)
-        saxpby(vorticity_field, vorticity_field, m, 1.0 / 3.0, 2.0 / 3.0)
+        L.call("sopht_vorticity_stretching_timestep_3d", tag, 1, L.comps(vorticity_field),
+               L.strides3(vorticity_field[0]), L.comps(velocity_field), L.strides3(velocity_field[0]),
+               L.comps(f), L.strides3(f[0]), L.comps(m), L.strides3(m[0]), nz, ny, nx,
+               float(dt_by_2_dx), float(dt_by_2_dx * 0.5), L.stream_ptr())
+        L.written(vorticity_field, m, f)
 
     return vorticity_stretching_timestep_ssprk3_pyst_kernel_3d
 

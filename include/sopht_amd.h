@@ -154,6 +154,20 @@ int sopht_advection_flux_conservative_eno3_3d(int dtype, void* flux, const int64
                                               const int64_t* velocity_strides, int64_t nz,
                                               int64_t ny, int64_t nx, double inv_dx,
                                               void* stream);
+/* The same flux stored instead of added: flux = E on [2:-2]^3, 0 elsewhere. The flux field must
+ * not overlap the field or the velocity. */
+int sopht_advection_flux_conservative_eno3_set_3d(int dtype, void* flux, const int64_t* flux_strides,
+                                                  const void* field, const int64_t* field_strides,
+                                                  const void* const velocity[3],
+                                                  const int64_t* velocity_strides, int64_t nz,
+                                                  int64_t ny, int64_t nx, double inv_dx, void* stream);
+/* gen_advection_timestep_euler_forward_conservative_eno3_pyst_kernel_3d —
+ * .../advection_timestep_3d.py:12-99: per component (ncomp 1 or 3) flux = E with prefactor
+ * inv_dx (the caller's -dt/dx), 0 on the border, then field += flux. */
+int sopht_advection_timestep_euler_forward_conservative_eno3_3d(
+    int dtype, int ncomp, void* const field[3], const int64_t* field_strides, void* flux,
+    const int64_t* flux_strides, const void* const velocity[3], const int64_t* velocity_strides,
+    int64_t nz, int64_t ny, int64_t nx, double inv_dx, void* stream);
 
 /* Adjoint of gen_advection_flux_conservative_eno3_pyst_kernel_3d
  * (.../advection_flux_3d.py:12-233; the reference has no adjoint): the transpose of the flux
@@ -161,6 +175,13 @@ int sopht_advection_flux_conservative_eno3_3d(int dtype, void* flux, const int64
  * [2:-2]^3, accumulates field_adj += J_field^T flux_adj and velocity_adj[c] += J_u_c^T flux_adj
  * over the whole grid. Either output may be NULL. Deterministic (gather, no atomics). */
 int sopht_advection_flux_conservative_eno3_adjoint_3d(
+    int dtype, void* field_adj, const int64_t* field_adj_strides, void* const velocity_adj[3],
+    const int64_t* velocity_adj_strides, const void* flux_adj, const int64_t* flux_adj_strides,
+    const void* field, const int64_t* field_strides, const void* const velocity[3],
+    const int64_t* velocity_strides, int64_t nz, int64_t ny, int64_t nx, double inv_dx,
+    void* stream);
+/* The same transpose stored into the outputs (which need not be initialised) instead of added. */
+int sopht_advection_flux_conservative_eno3_adjoint_set_3d(
     int dtype, void* field_adj, const int64_t* field_adj_strides, void* const velocity_adj[3],
     const int64_t* velocity_adj_strides, const void* flux_adj, const int64_t* flux_adj_strides,
     const void* field, const int64_t* field_strides, const void* const velocity[3],

@@ -77,9 +77,15 @@ SIGNATURES = {
         _i, _vp, _pi64, _vp, _pi64, _p3, _pi64, _i64, _i64, _i64, _d, _vp],
     "sopht_advection_flux_conservative_eno3_adjoint_3d": [
         _i, _vp, _pi64, _vp, _pi64, _vp, _pi64, _vp, _pi64, _p3, _pi64, _i64, _i64, _i64, _d, _vp],
+    "sopht_advection_flux_conservative_eno3_adjoint_set_3d": [
+        _i, _vp, _pi64, _vp, _pi64, _vp, _pi64, _vp, _pi64, _p3, _pi64, _i64, _i64, _i64, _d, _vp],
     "sopht_passive_transport_step_3d": [_i, _i, _p3, _p3, _p3, _i64, _i64, _i64, _d, _d, _vp],
     "sopht_velocity_abs_sum_max_3d": [_i, _p3, _i64, _vp, _vp, _i64, _vp, _vp],
     "sopht_vorticity_stretching_flux_3d": [_i, _p3, _pi64, _p3, _pi64, _p3, _pi64, _i64, _i64, _i64, _d, _vp],
+    "sopht_advection_flux_conservative_eno3_set_3d": [
+        _i, _vp, _pi64, _vp, _pi64, _p3, _pi64, _i64, _i64, _i64, _d, _vp],
+    "sopht_advection_timestep_euler_forward_conservative_eno3_3d": [
+        _i, _i, _p3, _pi64, _vp, _pi64, _p3, _pi64, _i64, _i64, _i64, _d, _vp],
     "sopht_vorticity_stretching_timestep_3d": [
         _i, _i, _p3, _pi64, _p3, _pi64, _p3, _pi64, _vp, _vp, _i64, _i64, _i64, _d, _d, _vp],
     "sopht_poisson3d_create": [_i, _i64, _i64, _i64, _d, _vp, C.POINTER(_vp)],
@@ -218,6 +224,11 @@ def comps(v):
     stride, without building the component views)."""
     base, step = v.data_ptr(), v.stride(0) * v.element_size()
     return _p3(base, base + step, base + 2 * step)
+
+
+def first(t):
+    """The pointer of a scalar field as the first of three components."""
+    return _p3(t.data_ptr(), 0, 0)
 
 
 def require_device_tensor(t, real_t, name, ndim=None):

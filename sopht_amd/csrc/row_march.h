@@ -2,12 +2,15 @@
 //
 // A thread owns a 16-byte vector of V neighbouring cells of one row (V = 4 FP32, 2 FP64) and
 // walks a chunk of z planes; the z neighbours stay in registers and the x neighbours come from
-// the adjacent lanes. The vectors of a plane are dealt to the threads in row order without
-// gaps, so any row length keeps every lane busy: 170 cells are 43 vectors, and the next row
-// starts at the next lane. The last vector of a row ends at the row's last cell; where the row
-// length is no multiple of V it overlaps its neighbour by `skip` cells, which it computes but
-// does not store. Rows need no alignment beyond the element's: gfx950 loads 16 bytes from any
-// 4-byte address.
+// the adjacent lanes. The vectors of a plane are dealt to the lanes in row order without gaps,
+// so any row length keeps the lanes busy: 170 cells are 43 vectors, and the next row starts at
+// the next lane. A wavefront takes 62 vectors; its first and last lane read the vectors beside
+// them for their neighbours and store nothing, which replaces scalar loads at its ends.
+// Rows need no alignment beyond the element's (gfx950 loads 16 bytes from any 4-byte address).
+// Where the row length is no multiple of V, the row's last vector reads up to V - 1 elements
+// past the row's end: into the rows behind it, whose values are not used. The last row of the
+// last plane has none behind it, and no vector is read there beyond its end: the operators'
+// stencils never reach it from a cell they write, and pointwise operands use rload_own.
 #pragma once
 
 #include <cstdlib>
@@ -18,6 +21,7 @@ namespace sopht {
 namespace {
 
 constexpr int kRowThreads = 256;
+constexpr int kRowLanes = 62;  // lanes of a wavefront that own a column
 
 template <typename T>
 struct RowVec {
@@ -73,16 +77,17 @@ struct RowGeo {
   int chunk;   // planes per workgroup
 };
 
-// The column of this thread. Threads past the last column repeat it (act = false), so that
-// every lane takes part in the lane shifts.
-template <typename T>
+// The column of this lane; lanes outside the plane repeat its first or last one and own no
+// cell. H is the operator's reach: stencil operands are read around the row yl, which is the
+// own row where the operator writes inside values and the nearest such row elsewhere, so that
+// every row read exists.
+template <typename T, int H>
 struct RowCol {
   static constexpr int V = RowVec<T>::V;
-  int x, y, ym, yp, z0, z1;
-  bool yin;            // the row is inside in y
-  bool edge_l, edge_r; // the adjacent lane does not hold the adjacent vector
-  unsigned own, inner; // cells to store; those inside in x
-  int nx;
+  int x, y, yl, z0, z1;
+  bool tail;            // the row's vector that holds cells past its end, on the last row
+  bool yin;             // rows the operator writes inside values to
+  unsigned own, inner;  // cells to store; those inside in x
 
   __device__ __forceinline__ RowCol(const RowGeo& g) {
     // contiguous runs of workgroups per XCD, so that rows shared by neighbouring workgroups
@@ -93,35 +98,37 @@ struct RowCol {
     const int tile = item % g.tiles;
     z0 = (item / g.tiles) * g.chunk;
     z1 = z0 + g.chunk < g.nz ? z0 + g.chunk : g.nz;
-    int col = tile * kRowThreads + int(threadIdx.x);
-    const int cols = g.nv * g.ny;
-    const bool act = col < cols;
-    col = act ? col : cols - 1;
-    y = col / g.nv;
-    const int xv = col - y * g.nv;
-    nx = g.nx;
-    x = xv * V < nx - V ? xv * V : nx - V;
-    const int skip = xv * V - x;
-    yin = y > 0 && y < g.ny - 1;
-    ym = y > 0 ? y - 1 : 0;
-    yp = y < g.ny - 1 ? y + 1 : y;
     const int lane = int(threadIdx.x) & 63;
-    edge_l = lane == 0 || skip != 0 || !act;
-    edge_r = lane == 63 || x + 2 * V > nx || !act;
-    own = act ? (RowVec<T>::kAll >> skip) << skip : 0u;
-    inner = 0;
+    int col = (tile * (kRowThreads / 64) + (int(threadIdx.x) >> 6)) * kRowLanes + lane - 1;
+    const int cols = g.nv * g.ny;
+    const bool act = lane > 0 && lane <= kRowLanes && col < cols;
+    col = col < 0 ? 0 : (col < cols ? col : cols - 1);
+    y = col / g.nv;
+    x = (col - y * g.nv) * V;
+    yin = y >= H && y < g.ny - H;
+    yl = y < H ? H : (y < g.ny - H ? y : g.ny - H - 1);
+    tail = x + V > g.nx && y == g.ny - 1;
+    own = inner = 0;
 #pragma unroll
-    for (int k = 0; k < V; ++k) inner |= (x + k > 0 && x + k < nx - 1) ? 1u << k : 0u;
-  }
-  // The cells left and right of the vector v read from row (row points at the field's cell
-  // x = 0); unspecified outside the grid.
-  __device__ __forceinline__ void nbrs(rvec<T> v, const T* row, T& left, T& right) const {
-    left = from_prev_lane(v[V - 1]);
-    right = from_next_lane(v[0]);
-    if (edge_l && x > 0) left = row[x - 1];
-    if (edge_r && x + V < nx) right = row[x + V];
+    for (int k = 0; k < V; ++k) {
+      own |= act && x + k < g.nx ? 1u << k : 0u;
+      inner |= x + k >= H && x + k < g.nx - H ? 1u << k : 0u;
+    }
   }
 };
+
+// A pointwise operand at the lane's own cells of plane z (p points at the first of them).
+template <typename T, int H>
+__device__ __forceinline__ rvec<T> rload_own(const RowCol<T, H>& c, const RowGeo& g, const T* p, int z) {
+  if (c.tail && z == g.nz - 1) {
+    rvec<T> v = {};
+#pragma unroll
+    for (int k = 0; k < RowVec<T>::V; ++k)
+      if (c.x + k < g.nx) v[k] = p[k];
+    return v;
+  }
+  return rload(p);
+}
 
 // Workgroups for the columns of an (nz, ny, nx) box. Chunks start at `most` planes and are
 // halved (down to 2) while there are fewer than four workgroups per CU: a chunk's first planes
@@ -133,26 +140,28 @@ inline RowGeo row_geo(int64_t nz, int64_t ny, int64_t nx, int most) {
   g.ny = int(ny);
   g.nx = int(nx);
   g.nv = ceil_div(nx, RowVec<T>::V);
-  g.tiles = ceil_div(int64_t(g.nv) * ny, kRowThreads);
+  g.tiles = ceil_div(int64_t(g.nv) * ny, kRowLanes * (kRowThreads / 64));
   g.chunk = most;
   while (g.chunk > 2 && int64_t(g.tiles) * ceil_div(nz, g.chunk) < 1024) g.chunk /= 2;
   return g;
 }
 inline unsigned row_blocks(const RowGeo& g) { return unsigned(int64_t(g.tiles) * ceil_div(g.nz, g.chunk)); }
 
-// Whether the row-vector kernels take a field: cells adjacent along x, non-negative row and
-// plane strides, 32-bit offsets, and rows of at least one vector.
+// Whether the row-vector kernels take a field: cells adjacent along x, rows and planes that
+// do not overlap, and 32-bit offsets.
 inline bool row_strides_ok(const int64_t* s, int64_t nz, int64_t ny, int64_t nx) {
   constexpr int64_t lim = int64_t(1) << 31;
-  return s[2] == 1 && s[0] >= 0 && s[1] >= 0 && s[0] < lim && s[1] < lim &&
+  return s[2] == 1 && s[0] >= nx && s[1] >= nx && s[0] < lim && s[1] < lim &&
+         (s[0] >= (ny - 1) * s[1] + nx || s[1] >= (nz - 1) * s[0] + nx) &&
          (nz - 1) * s[0] + (ny - 1) * s[1] + nx < lim;
 }
-template <typename T>
+// ... and a box: one with cells the operator (of reach H) writes inside values to, and with
+// vectors and workgroups that 32 bits count.
+template <typename T, int H>
 inline bool row_box_ok(int64_t nz, int64_t ny, int64_t nx) {
-  constexpr int64_t lim = int64_t(1) << 31;
-  return nx >= RowVec<T>::V && nz < lim && ny < lim && nx < lim &&
-         ceil_div(nx, RowVec<T>::V) * ny < lim - kRowThreads &&
-         int64_t(ceil_div(int64_t(ceil_div(nx, RowVec<T>::V)) * ny, kRowThreads)) * ceil_div(nz, 2) < lim;
+  constexpr int64_t lim = int64_t(1) << 30;
+  return nz > 2 * H && ny > 2 * H && nx > 2 * H && nx >= RowVec<T>::V && nz < lim && ny < lim && nx < lim &&
+         nz * ny < lim && ny * nx < lim && nz * (ny * nx) / RowVec<T>::V < 62 * lim;
 }
 inline RowStrides row_strides(const int64_t* s) { return RowStrides{int(s[1]), int(s[0])}; }
 
@@ -199,34 +208,33 @@ __global__ void __launch_bounds__(kRowThreads)
                    T p, T p_last) {
   constexpr int V = RowVec<T>::V;
   using vec = rvec<T>;
-  const RowCol<T> c(g);
-  const int ur = c.y * u.s.y, urm = c.ym * u.s.y, urp = c.yp * u.s.y;
+  const RowCol<T, 1> c(g);
+  const int ur = c.yl * u.s.y + c.x, wr = c.y * w.s.y + c.x;
   vec um[3], uc[3];
   {
     const int zm = c.z0 > 0 ? c.z0 - 1 : 0;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      um[a] = rload(u.p[a] + zm * u.s.z + ur + c.x);
-      uc[a] = rload(u.p[a] + c.z0 * u.s.z + ur + c.x);
+      um[a] = rload(u.p[a] + zm * u.s.z + ur);
+      uc[a] = rload(u.p[a] + c.z0 * u.s.z + ur);
     }
   }
   for (int z = c.z0; z < c.z1; ++z) {
-    const int zp = z < g.nz - 1 ? z + 1 : z;
+    const bool plane = z > 0 && z < g.nz - 1;
     vec wv[3], up[3], grad[3][3];  // grad[a][axis]: difference of u_a along x, y, z
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      const T* ua = u.p[a] + z * u.s.z;
-      up[a] = rload(u.p[a] + zp * u.s.z + ur + c.x);
-      wv[a] = rload(w.p[a] + z * w.s.z + c.y * w.s.y + c.x);
-      grad[a][1] = rload(ua + urp + c.x) - rload(ua + urm + c.x);
+      const T* ua = u.p[a] + z * u.s.z + ur;
+      up[a] = z < g.nz - 1 ? rload(ua + u.s.z) : uc[a];
+      wv[a] = rload_own(c, g, w.p[a] + z * w.s.z + wr, z);
+      grad[a][1] = plane ? rload(ua + u.s.y) - rload(ua - u.s.y) : vec{};
       grad[a][2] = up[a] - um[a];
-      T left, right;
-      c.nbrs(uc[a], ua + ur, left, right);
+      const T left = from_prev_lane(uc[a][V - 1]), right = from_next_lane(uc[a][0]);
 #pragma unroll
       for (int k = 0; k < V; ++k)
         grad[a][0][k] = (k < V - 1 ? uc[a][k < V - 1 ? k + 1 : k] : right) - (k > 0 ? uc[a][k > 0 ? k - 1 : k] : left);
     }
-    const bool zin = c.yin && z > 0 && z < g.nz - 1;
+    const bool zin = c.yin && plane;
     auto stage = [&](const vec* v, T q, vec* f) {
 #pragma unroll
       for (int a = 0; a < 3; ++a)
@@ -238,9 +246,10 @@ __global__ void __launch_bounds__(kRowThreads)
     };
     vec f[3], m[3], o[3];
     stage(wv, p, f);
-    if constexpr (SCHEME >= 1)
+    if constexpr (SCHEME >= 1) {
 #pragma unroll
       for (int a = 0; a < 3; ++a) o[a] = m[a] = wv[a] + f[a];
+    }
     if constexpr (SCHEME == 2) {
       stage(m, p, f);
 #pragma unroll
@@ -259,6 +268,235 @@ __global__ void __launch_bounds__(kRowThreads)
       if constexpr (SCHEME == 2) rstore(mid.p[a] + z * mid.s.z + c.y * mid.s.y + c.x, m[a], c.own);
       um[a] = uc[a];
       uc[a] = up[a];
+    }
+  }
+}
+
+// ------------------------------------------------------------------ ENO3 advection flux
+
+// The flux through the face between cells 0 and 1 of one axis (advection_flux_3d.py:12-233):
+// g = field * velocity at cells -1 .. 2, u the velocity at cells 0 and 1. A cell's front face
+// is its upper neighbour's back face, with the same upwind choice and the same terms, so each
+// face is formed once.
+template <typename T>
+__device__ __forceinline__ T eno3_face(T gm, T g0, T g1, T gp, T u0, T u1) {
+  const T c13 = T(1.0 / 3.0), c56 = T(5.0 / 6.0), c16 = T(1.0 / 6.0);
+  const bool up = u0 > -u1;
+  return c13 * (up ? g1 : g0) + c56 * (up ? g0 : g1) - c16 * (up ? gm : gp);
+}
+
+// ENO3 conservative advection flux on [2:-2]^3: added to the flux field, or (SET) stored with
+// zeros on the border cells, which spares the clearing and the read of the flux field.
+// A thread forms V + 1 x faces, two rows of y faces and one plane of z faces per plane of V
+// cells; its 13 16-byte loads per plane (field rows y-2..y+2, u_y rows y-2..y+2, u_x, u_z and
+// the field two planes up) come mostly from L1 and L2, and their rate bounds it.
+// 150 x 201 x 230 FP32, storing: 36 us (3.8 TB/s of 5 words per cell) against 94 us with one
+// cell per thread plus 7 us for the clearing.
+template <typename T, bool SET>
+__global__ void __launch_bounds__(kRowThreads)
+    k_eno3_rows(RowGeo g, T* flux, RowStrides os, const T* f, RowStrides fs, Rows3<const T> u, T inv_dx) {
+  constexpr int V = RowVec<T>::V;
+  using vec = rvec<T>;
+  const RowCol<T, 2> c(g);
+  const int fr = c.yl * fs.y + c.x, ur = c.yl * u.s.y + c.x, orow = c.y * os.y + c.x;
+  // planes with a flux: those of the chunk inside [2, nz - 2)
+  const int za = c.z0 < 2 ? 2 : c.z0, zb = c.z1 < g.nz - 2 ? c.z1 : g.nz - 2;
+  if (SET) {
+    for (int z = c.z0; z < c.z1; ++z)
+      if (z < za || z >= zb) rstore(flux + z * os.z + orow, vec{}, c.own);
+  }
+  if (za >= zb) return;  // the same for the whole workgroup
+  // along z: the field at z, z+1; u_z at z, z+1; their products at z-1, z, z+1; the back face
+  vec f0 = rload(f + za * fs.z + fr), f1 = rload(f + (za + 1) * fs.z + fr);
+  vec w0 = rload(u.p[2] + za * u.s.z + ur), w1 = rload(u.p[2] + (za + 1) * u.s.z + ur);
+  vec gm, g0 = f0 * w0, g1 = f1 * w1, back;
+  {
+    const vec wm = rload(u.p[2] + (za - 1) * u.s.z + ur);
+    gm = rload(f + (za - 1) * fs.z + fr) * wm;
+    const vec gmm = rload(f + (za - 2) * fs.z + fr) * rload(u.p[2] + (za - 2) * u.s.z + ur);
+#pragma unroll
+    for (int k = 0; k < V; ++k) back[k] = eno3_face<T>(gmm[k], gm[k], g0[k], g1[k], wm[k], w0[k]);
+  }
+  const unsigned mask = c.yin ? c.own & c.inner : 0u;
+  for (int z = za; z < zb; ++z) {
+    const T* fz = f + z * fs.z + fr;
+    const T* uxz = u.p[0] + z * u.s.z + ur;
+    const T* uyz = u.p[1] + z * u.s.z + ur;
+    T* oz = flux + z * os.z + orow;
+    const vec f2 = rload(fz + 2 * fs.z), w2 = rload(u.p[2] + (z + 2) * u.s.z + ur);
+    const vec ux = rload(uxz);
+    vec uy[5], gy[5];
+#pragma unroll
+    for (int r = 0; r < 5; ++r) uy[r] = rload(uyz + (r - 2) * u.s.y);
+#pragma unroll
+    for (int r = 0; r < 5; ++r) gy[r] = (r == 2 ? f0 : rload(fz + (r - 2) * fs.y)) * uy[r];
+    vec acc = {};
+    if (!SET) acc = rload_own(c, g, static_cast<const T*>(oz), z);
+    {  // x faces -1/2 .. V - 1/2 of the vector
+      const vec gx = f0 * ux;
+      T e[V + 4], v[V + 2];  // products at cells -2 .. V + 1, velocities at -1 .. V
+      e[0] = from_prev_lane(gx[V - 2]);
+      e[1] = from_prev_lane(gx[V - 1]);
+      e[V + 2] = from_next_lane(gx[0]);
+      e[V + 3] = from_next_lane(gx[1]);
+      v[0] = from_prev_lane(ux[V - 1]);
+      v[V + 1] = from_next_lane(ux[0]);
+#pragma unroll
+      for (int k = 0; k < V; ++k) {
+        e[k + 2] = gx[k];
+        v[k + 1] = ux[k];
+      }
+      T face[V + 1];
+#pragma unroll
+      for (int k = 0; k <= V; ++k) face[k] = eno3_face<T>(e[k], e[k + 1], e[k + 2], e[k + 3], v[k], v[k + 1]);
+#pragma unroll
+      for (int k = 0; k < V; ++k) {
+        acc[k] = acc[k] + inv_dx * face[k + 1];
+        acc[k] = acc[k] - inv_dx * face[k];
+      }
+    }
+    const vec g2 = f2 * w2;
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+      acc[k] = acc[k] + inv_dx * eno3_face<T>(gy[1][k], gy[2][k], gy[3][k], gy[4][k], uy[2][k], uy[3][k]);
+      acc[k] = acc[k] - inv_dx * eno3_face<T>(gy[0][k], gy[1][k], gy[2][k], gy[3][k], uy[1][k], uy[2][k]);
+      const T front = eno3_face<T>(gm[k], g0[k], g1[k], g2[k], w0[k], w1[k]);
+      acc[k] = acc[k] + inv_dx * front;
+      acc[k] = acc[k] - inv_dx * back[k];
+      back[k] = front;
+    }
+    if (SET) {
+#pragma unroll
+      for (int k = 0; k < V; ++k) acc[k] = mask >> k & 1u ? acc[k] : T(0);
+      rstore(oz, acc, c.own);
+    } else {
+      rstore(oz, acc, mask);
+    }
+    gm = g0;
+    g0 = g1;
+    g1 = g2;
+    f0 = f1;
+    f1 = f2;
+    w0 = w1;
+    w1 = w2;
+  }
+}
+
+// Transpose of the ENO3 flux along one axis with the upwind choices frozen at the velocity, at
+// cell m: a and u are the flux adjoint (0 where the forward writes nothing) and the axis'
+// velocity at cells m - 2 .. m + 2. The flux at a cell is its front face minus its back face,
+// so face (i, i + 1) carries d = a(i) - a(i + 1), and the faces m - 2 .. m + 1 read cell m.
+template <typename T>
+__device__ __forceinline__ T eno3_gather(const T* a, const T* u) {
+  const T c13 = T(1.0 / 3.0), c56 = T(5.0 / 6.0), c16 = T(1.0 / 6.0);
+  const T lo = !(u[0] > -u[1]) ? a[0] - a[1] : T(0);
+  const T hi = u[3] > -u[4] ? a[3] - a[4] : T(0);
+  return (u[1] > -u[2] ? c13 : c56) * (a[1] - a[2]) + (u[2] > -u[3] ? c56 : c13) * (a[2] - a[3]) - c16 * (lo + hi);
+}
+
+// The transpose on a whole box: gbar_axis as above where the forward flux reads the cell along
+// that axis, then field_adj (+)= sum_axis gbar_axis u_axis, vel_adj[axis] (+)= gbar_axis field.
+// SET stores instead of adding, which spares the outputs' clearing and their read (4 of 13
+// words per cell). A gather: no atomics, the same bits on every run.
+// Bound by memory: 150 x 201 x 230 FP32, storing, 52 us (4.8 TB/s of 9 words per cell) against
+// 148 us with one cell per thread, each weighing the 15 fluxes that read it, plus 19 us of clearing.
+template <typename T, bool SET>
+__global__ void __launch_bounds__(kRowThreads)
+    k_eno3_adjoint_rows(RowGeo g, T* fa, RowStrides fas, Rows3<T> va, const T* a, RowStrides as, const T* f,
+                        RowStrides fs, Rows3<const T> u, T inv_dx) {
+  constexpr int V = RowVec<T>::V;
+  using vec = rvec<T>;
+  const RowCol<T, 2> c(g);
+  const int ar = c.yl * as.y + c.x, ur = c.yl * u.s.y + c.x;
+  // a plane of the flux adjoint, 0 where the forward writes no plane
+  auto a_plane = [&](int q) -> vec {
+    return q >= 2 && q < g.nz - 2 ? rload(a + q * as.z + ar) : vec{};
+  };
+  auto u_plane = [&](int q) -> vec {  // u_z, read where a face of the forward reads it
+    const int p = q < 1 ? 1 : (q < g.nz - 1 ? q : g.nz - 2);
+    return rload(u.p[2] + p * u.s.z + ur);
+  };
+  vec az[5], uz[5];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    az[k + 1] = a_plane(c.z0 - 2 + k);
+    uz[k + 1] = u_plane(c.z0 - 2 + k);
+  }
+  // rows y - 2 .. y + 2: the flux adjoint is 0 outside [2, ny - 2); the velocity rows are
+  // clamped into the grid (a clamped row's faces carry d = 0)
+  int arow[5], urow[5];
+  bool ain[5];
+#pragma unroll
+  for (int r = 0; r < 5; ++r) {
+    const int y = c.y + r - 2;
+    ain[r] = y >= 2 && y < g.ny - 2;
+    arow[r] = (y < 2 ? 2 : (y < g.ny - 2 ? y : g.ny - 3)) * as.y + c.x;
+    urow[r] = (y < 1 ? 1 : (y < g.ny - 1 ? y : g.ny - 2)) * u.s.y + c.x;
+  }
+  for (int z = c.z0; z < c.z1; ++z) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      az[k] = az[k + 1];
+      uz[k] = uz[k + 1];
+    }
+    az[4] = a_plane(z + 2);
+    uz[4] = u_plane(z + 2);
+    vec gb[3] = {{}, {}, {}};
+    if (z >= 2 && z < g.nz - 2) {  // the same for the whole workgroup
+      vec ay[5], uy[5];
+#pragma unroll
+      for (int r = 0; r < 5; ++r) {
+        uy[r] = rload(u.p[1] + z * u.s.z + urow[r]);
+        ay[r] = r == 2 ? az[2] : rload(a + z * as.z + arow[r]);
+      }
+      const vec ux = rload(u.p[0] + z * u.s.z + ur);
+      T e[V + 4], v[V + 4];
+#pragma unroll
+      for (int k = 0; k < V; ++k) {
+        e[k + 2] = c.inner >> k & 1u ? az[2][k] : T(0);
+        v[k + 2] = ux[k];
+      }
+      e[0] = from_prev_lane(e[V]);
+      e[1] = from_prev_lane(e[V + 1]);
+      v[0] = from_prev_lane(v[V]);
+      v[1] = from_prev_lane(v[V + 1]);
+      e[V + 2] = from_next_lane(e[2]);
+      e[V + 3] = from_next_lane(e[3]);
+      v[V + 2] = from_next_lane(v[2]);
+      v[V + 3] = from_next_lane(v[3]);
+      if (c.x == 0) e[0] = e[1] = T(0);  // the lane before holds another row's end
+#pragma unroll
+      for (int k = 0; k < V; ++k) {
+        if (c.yin) gb[0][k] = inv_dx * eno3_gather<T>(e + k, v + k);
+        const T ac[5] = {ain[0] ? ay[0][k] : T(0), ain[1] ? ay[1][k] : T(0), ain[2] ? ay[2][k] : T(0),
+                         ain[3] ? ay[3][k] : T(0), ain[4] ? ay[4][k] : T(0)};
+        const T uc[5] = {uy[0][k], uy[1][k], uy[2][k], uy[3][k], uy[4][k]};
+        if (c.inner >> k & 1u) gb[1][k] = inv_dx * eno3_gather<T>(ac, uc);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+      const T ac[5] = {az[0][k], az[1][k], az[2][k], az[3][k], az[4][k]};
+      const T uc[5] = {uz[0][k], uz[1][k], uz[2][k], uz[3][k], uz[4][k]};
+      if (c.yin && (c.inner >> k & 1u)) gb[2][k] = inv_dx * eno3_gather<T>(ac, uc);
+    }
+    if (fa) {
+      T* o = fa + z * fas.z + c.y * fas.y + c.x;
+      vec r = {};
+#pragma unroll
+      for (int ax = 0; ax < 3; ++ax) r += gb[ax] * rload_own(c, g, u.p[ax] + z * u.s.z + c.y * u.s.y + c.x, z);
+      if (!SET) r += rload_own(c, g, static_cast<const T*>(o), z);
+      rstore(o, r, c.own);
+    }
+    if (va.p[0]) {
+      const vec fv = rload_own(c, g, f + z * fs.z + c.y * fs.y + c.x, z);
+#pragma unroll
+      for (int ax = 0; ax < 3; ++ax) {
+        T* o = va.p[ax] + z * va.s.z + c.y * va.s.y + c.x;
+        vec r = gb[ax] * fv;
+        if (!SET) r += rload_own(c, g, static_cast<const T*>(o), z);
+        rstore(o, r, c.own);
+      }
     }
   }
 }

@@ -347,10 +347,10 @@ __device__ __forceinline__ T eno3_cell(const T* f, int64_t fo, Strides3 fs, cons
   return acc;
 }
 
-// The same flux marching z: a thread owns one (y, x) column of kEnoZc planes and keeps f
-// and u_z at z-2..z+2 in registers, so the z terms cost two loads per cell instead of nine.
-// The x and y terms are read as in eno3_cell, and every expression is the same, so the
-// results are the same bits.
+// The same flux for fields whose cells are not adjacent along x (k_eno3_rows takes the others):
+// a thread owns one (y, x) column of kEnoZc planes and keeps f and u_z at z-2..z+2 in
+// registers, so the z terms cost two loads per cell instead of nine. The x and y terms are read
+// as in eno3_cell, and every expression is the same, so the results are the same bits.
 constexpr int kEnoZc = 16;
 
 template <typename T>
@@ -411,11 +411,32 @@ __global__ void __launch_bounds__(kEnoTx* kEnoTy)
   }
 }
 
+constexpr int kEnoChunk = 16;
+
+template <typename T>
+bool eno3_rows_ok(const int64_t* fs, const int64_t* is, const int64_t* vs, int64_t nz, int64_t ny, int64_t nx) {
+  return row_box_ok<T, 2>(nz, ny, nx) && row_strides_ok(fs, nz, ny, nx) && row_strides_ok(is, nz, ny, nx) &&
+         row_strides_ok(vs, nz, ny, nx);
+}
+
+template <typename T, bool SET>
+int eno3_rows(void* flux, const int64_t* fs, const void* field, const int64_t* is, const void* const vel[3],
+              const int64_t* vs, int64_t nz, int64_t ny, int64_t nx, T inv_dx, hipStream_t s) {
+  const RowGeo g = row_geo<T>(nz, ny, nx, kEnoChunk);
+  k_eno3_rows<T, SET><<<row_blocks(g), kRowThreads, 0, s>>>(g, static_cast<T*>(flux), row_strides(fs),
+                                                          static_cast<const T*>(field), row_strides(is),
+                                                          rows3<T>(vel, vs), inv_dx);
+  SOPHT_CHECK_LAUNCH();
+  return SOPHT_OK;
+}
+
 template <typename T>
 int eno3_impl(void* flux, const int64_t* fs, const void* field, const int64_t* is,
               const void* const vel[3], const int64_t* vs, int64_t nz, int64_t ny, int64_t nx,
               T inv_dx, hipStream_t s) {
   if (nz <= 4 || ny <= 4 || nx <= 4) return SOPHT_OK;
+  if (eno3_rows_ok<T>(fs, is, vs, nz, ny, nx))
+    return eno3_rows<T, false>(flux, fs, field, is, vel, vs, nz, ny, nx, inv_dx, s);
   const Strides3 os3 = strides_of(fs), is3 = strides_of(is), vs3 = strides_of(vs);
   T* o = static_cast<T*>(flux);
   const T* f = static_cast<const T*>(field);
@@ -438,6 +459,39 @@ int eno3_impl(void* flux, const int64_t* fs, const void* field, const int64_t* i
         o[oo] = eno3_cell<T>(f, is3.at(z, y, x), is3, u, vs3.at(z, y, x), vs3, o[oo], inv_dx);
       },
       s);
+}
+
+// flux = the ENO3 flux on [2:-2]^3, 0 elsewhere.
+template <typename T>
+int eno3_set_impl(void* flux, const int64_t* fs, const void* field, const int64_t* is,
+                  const void* const vel[3], const int64_t* vs, int64_t nz, int64_t ny, int64_t nx,
+                  T inv_dx, hipStream_t s) {
+  bool apart = true;
+  for (int a = 0; a < 3; ++a) apart = apart && !fields_meet<T>(flux, fs, vel[a], vs, nz, ny, nx);
+  if (apart && eno3_rows_ok<T>(fs, is, vs, nz, ny, nx) && !fields_meet<T>(flux, fs, field, is, nz, ny, nx))
+    return eno3_rows<T, true>(flux, fs, field, is, vel, vs, nz, ny, nx, inv_dx, s);
+  View3<T> o = make_view<T>(flux, fs);
+  int rc = launch_box(
+      0, 0, 0, nz, ny, nx, [=] __device__(int64_t z, int64_t y, int64_t x) { o(z, y, x) = T(0); }, s);
+  return rc ? rc : eno3_impl<T>(flux, fs, field, is, vel, vs, nz, ny, nx, inv_dx, s);
+}
+
+// field += flux after the flux has been cleared and filled, component by component through
+// one scalar flux field (advection_timestep_3d.py:12-99).
+template <typename T>
+int eno3_step_impl(int ncomp, void* const field[3], const int64_t* is, void* flux, const int64_t* fs,
+                   const void* const vel[3], const int64_t* vs, int64_t nz, int64_t ny, int64_t nx,
+                   T inv_dx, hipStream_t s) {
+  for (int c = 0; c < ncomp; ++c) {
+    int rc = eno3_set_impl<T>(flux, fs, field[c], is, vel, vs, nz, ny, nx, inv_dx, s);
+    if (rc) return rc;
+    View3<T> f = make_view<T>(field[c], is), o = make_view<T>(flux, fs);
+    rc = launch_box(
+        0, 0, 0, nz, ny, nx,
+        [=] __device__(int64_t z, int64_t y, int64_t x) { f(z, y, x) = f(z, y, x) + o(z, y, x); }, s);
+    if (rc) return rc;
+  }
+  return SOPHT_OK;
 }
 
 // Weight of g[c + o] in the ENO3 flux at c along one axis (front face minus back face), for
@@ -519,11 +573,26 @@ template <typename T>
 int eno3_adjoint_impl(void* field_adj, const int64_t* fas, void* const vel_adj[3],
                       const int64_t* vas, const void* flux_adj, const int64_t* as,
                       const void* field, const int64_t* is, const void* const vel[3],
-                      const int64_t* vs, int64_t nz, int64_t ny, int64_t nx, T inv_dx,
+                      const int64_t* vs, int64_t nz, int64_t ny, int64_t nx, T inv_dx, bool set,
                       hipStream_t s) {
-  if (nz <= 4 || ny <= 4 || nx <= 4) return SOPHT_OK;
   const bool has_f = field_adj != nullptr, has_v = vel_adj != nullptr;
   if (!has_f && !has_v) return SOPHT_OK;
+  const bool rows = row_box_ok<T, 2>(nz, ny, nx) && row_strides_ok(as, nz, ny, nx) &&
+                    row_strides_ok(is, nz, ny, nx) && row_strides_ok(vs, nz, ny, nx) &&
+                    (!has_f || row_strides_ok(fas, nz, ny, nx)) && (!has_v || row_strides_ok(vas, nz, ny, nx));
+  if (set && !rows) {  // clear, then add
+    int rc = SOPHT_OK;
+    auto clear = [&](void* p, const int64_t* st) {
+      View3<T> o = make_view<T>(p, st);
+      if (!rc)
+        rc = launch_box(
+            0, 0, 0, nz, ny, nx, [=] __device__(int64_t z, int64_t y, int64_t x) { o(z, y, x) = T(0); }, s);
+    };
+    if (has_f) clear(field_adj, fas);
+    for (int a = 0; has_v && a < 3; ++a) clear(vel_adj[a], vas);
+    if (rc) return rc;
+  }
+  if (nz <= 4 || ny <= 4 || nx <= 4) return SOPHT_OK;
   const int64_t zero3[3] = {0, 0, 0};
   const Strides3 fas3 = strides_of(has_f ? fas : zero3), vas3 = strides_of(has_v ? vas : zero3);
   const Strides3 as3 = strides_of(as), is3 = strides_of(is), us3 = strides_of(vs);
@@ -536,6 +605,16 @@ int eno3_adjoint_impl(void* field_adj, const int64_t* fas, void* const vel_adj[3
   const T* u0 = static_cast<const T*>(vel[0]);
   const T* u1 = static_cast<const T*>(vel[1]);
   const T* u2 = static_cast<const T*>(vel[2]);
+  if (rows) {
+    const RowGeo g = row_geo<T>(nz, ny, nx, kEnoChunk);
+    Rows3<T> va{};
+    if (has_v) va = rows3<T>(vel_adj, vas);
+    auto* kernel = set ? k_eno3_adjoint_rows<T, true> : k_eno3_adjoint_rows<T, false>;
+    kernel<<<row_blocks(g), kRowThreads, 0, s>>>(g, fa, has_f ? row_strides(fas) : RowStrides{0, 0}, va, a,
+                                                row_strides(as), f, row_strides(is), rows3<T>(vel, vs), inv_dx);
+    SOPHT_CHECK_LAUNCH();
+    return SOPHT_OK;
+  }
   if (eno3_grid_fits(nz, ny)) {
     dim3 grid(unsigned(ceil_div(nx, kEnoTx)), unsigned(ceil_div(ny, kEnoTy)), unsigned(nz));
     k_eno3_adjoint<T><<<grid, dim3(kEnoTx, kEnoTy), 0, s>>>(fa, fas3, va0, va1, va2, vas3, a, as3, f,
@@ -595,7 +674,7 @@ template <typename T>
 int stretching_impl(void* const flux[3], const int64_t* fs, const void* const w[3],
                     const int64_t* ws, const void* const u[3], const int64_t* us, int64_t nz,
                     int64_t ny, int64_t nx, T p, hipStream_t s) {
-  bool rows = row_box_ok<T>(nz, ny, nx) && row_strides_ok(fs, nz, ny, nx) && row_strides_ok(ws, nz, ny, nx) &&
+  bool rows = row_box_ok<T, 1>(nz, ny, nx) && row_strides_ok(fs, nz, ny, nx) && row_strides_ok(ws, nz, ny, nx) &&
               row_strides_ok(us, nz, ny, nx);
   if (!rows) return stretching_general<T>(flux, fs, w, ws, u, us, nz, ny, nx, p, s);
   const RowGeo g = row_geo<T>(nz, ny, nx, kStretchChunk);
@@ -621,7 +700,7 @@ template <typename T>
 int stretching_step_impl(int scheme, void* const w[3], const int64_t* ws, const void* const u[3],
                          const int64_t* us, void* const flux[3], const int64_t* fs, void* const mid[3],
                          const int64_t* ms, int64_t nz, int64_t ny, int64_t nx, T p, T p_last, hipStream_t s) {
-  bool rows = row_box_ok<T>(nz, ny, nx) && row_strides_ok(fs, nz, ny, nx) && row_strides_ok(ws, nz, ny, nx) &&
+  bool rows = row_box_ok<T, 1>(nz, ny, nx) && row_strides_ok(fs, nz, ny, nx) && row_strides_ok(ws, nz, ny, nx) &&
               row_strides_ok(us, nz, ny, nx) && (scheme == 0 || row_strides_ok(ms, nz, ny, nx));
   for (int a = 0; rows && a < 3; ++a)
     for (int b = 0; rows && b < 3; ++b) {
@@ -945,18 +1024,54 @@ int sopht_advection_flux_conservative_eno3_3d(int dtype, void* flux, const int64
                                as_stream(stream)));
 }
 
-int sopht_advection_flux_conservative_eno3_adjoint_3d(
+int sopht_advection_flux_conservative_eno3_set_3d(int dtype, void* flux, const int64_t* fs, const void* field,
+                                                  const int64_t* is, const void* const vel[3], const int64_t* vs,
+                                                  int64_t nz, int64_t ny, int64_t nx, double inv_dx, void* stream) {
+  REQUIRE_GRID(nz, ny, nx);
+  DISPATCH(dtype, eno3_set_impl<T>(flux, fs, field, is, vel, vs, nz, ny, nx, T(inv_dx), as_stream(stream)));
+}
+
+int sopht_advection_timestep_euler_forward_conservative_eno3_3d(int dtype, int ncomp, void* const field[3],
+                                                                const int64_t* is, void* flux, const int64_t* fs,
+                                                                const void* const vel[3], const int64_t* vs,
+                                                                int64_t nz, int64_t ny, int64_t nx, double inv_dx,
+                                                                void* stream) {
+  REQUIRE_GRID(nz, ny, nx);
+  SOPHT_REQUIRE(ncomp == 1 || ncomp == 3, "ncomp must be 1 or 3");
+  DISPATCH(dtype, eno3_step_impl<T>(ncomp, field, is, flux, fs, vel, vs, nz, ny, nx, T(inv_dx), as_stream(stream)));
+}
+
+static int eno3_adjoint_call(
     int dtype, void* field_adj, const int64_t* fas, void* const velocity_adj[3],
     const int64_t* vas, const void* flux_adj, const int64_t* as, const void* field,
     const int64_t* is, const void* const vel[3], const int64_t* vs, int64_t nz, int64_t ny,
-    int64_t nx, double inv_dx, void* stream) {
+    int64_t nx, double inv_dx, int set,
+    void* stream) {
   REQUIRE_GRID(nz, ny, nx);
   SOPHT_REQUIRE(field_adj == nullptr || fas != nullptr, "field_adj needs its strides");
   SOPHT_REQUIRE(velocity_adj == nullptr || (vas != nullptr && velocity_adj[0] != nullptr &&
                                             velocity_adj[1] != nullptr && velocity_adj[2] != nullptr),
                 "velocity_adj needs three components and their strides");
   DISPATCH(dtype, eno3_adjoint_impl<T>(field_adj, fas, velocity_adj, vas, flux_adj, as, field, is,
-                                       vel, vs, nz, ny, nx, T(inv_dx), as_stream(stream)));
+                                       vel, vs, nz, ny, nx, T(inv_dx), set != 0, as_stream(stream)));
+}
+
+int sopht_advection_flux_conservative_eno3_adjoint_3d(
+    int dtype, void* field_adj, const int64_t* fas, void* const velocity_adj[3],
+    const int64_t* vas, const void* flux_adj, const int64_t* as, const void* field,
+    const int64_t* is, const void* const vel[3], const int64_t* vs, int64_t nz, int64_t ny,
+    int64_t nx, double inv_dx, void* stream) {
+  return eno3_adjoint_call(dtype, field_adj, fas, velocity_adj, vas, flux_adj, as, field, is, vel, vs, nz, ny, nx,
+                           inv_dx, 0, stream);
+}
+
+int sopht_advection_flux_conservative_eno3_adjoint_set_3d(
+    int dtype, void* field_adj, const int64_t* fas, void* const velocity_adj[3],
+    const int64_t* vas, const void* flux_adj, const int64_t* as, const void* field,
+    const int64_t* is, const void* const vel[3], const int64_t* vs, int64_t nz, int64_t ny,
+    int64_t nx, double inv_dx, void* stream) {
+  return eno3_adjoint_call(dtype, field_adj, fas, velocity_adj, vas, flux_adj, as, field, is, vel, vs, nz, ny, nx,
+                           inv_dx, 1, stream);
 }
 
 int sopht_vorticity_stretching_flux_3d(int dtype, void* const flux[3], const int64_t* fs,

@@ -481,6 +481,19 @@ def gen_advection_flux_conservative_eno3_pyst_kernel_3d(
     return advection_flux_conservative_eno3_pyst_kernel_3d
 
 
+def _eno3_adjoint(entry, tag, field_adj, velocity_adj, flux_adj, field, velocity, inv_dx):
+    nz, ny, nx = _shape3(field)
+    L.call(entry, tag, L.ptr(field_adj),
+           L.strides3(field_adj) if field_adj is not None else None,
+           L.comps(velocity_adj) if velocity_adj is not None else None,
+           L.strides3(velocity_adj[0]) if velocity_adj is not None else None,
+           L.ptr(flux_adj), L.strides3(flux_adj), L.ptr(field), L.strides3(field),
+           L.comps(velocity), L.strides3(velocity[0]), nz, ny, nx, float(inv_dx),
+           L.stream_ptr())
+    written = [t for t in (field_adj, velocity_adj) if t is not None]
+    L.written(*written)
+
+
 def gen_advection_flux_conservative_eno3_adjoint_kernel_3d(real_t: type) -> Callable:
     """Transpose of the ENO3 flux above (``advection_flux_3d.py:12-233``; the reference has no
     adjoint), with each face's upwind stencil choice frozen at ``velocity``.
@@ -494,16 +507,8 @@ def gen_advection_flux_conservative_eno3_adjoint_kernel_3d(real_t: type) -> Call
     def advection_flux_conservative_eno3_adjoint_kernel_3d(
         field_adj, velocity_adj, flux_adj, field, velocity, inv_dx: float
     ) -> None:
-        nz, ny, nx = _shape3(field)
-        L.call("sopht_advection_flux_conservative_eno3_adjoint_3d", tag, L.ptr(field_adj),
-               L.strides3(field_adj) if field_adj is not None else None,
-               L.comps(velocity_adj) if velocity_adj is not None else None,
-               L.strides3(velocity_adj[0]) if velocity_adj is not None else None,
-               L.ptr(flux_adj), L.strides3(flux_adj), L.ptr(field), L.strides3(field),
-               L.comps(velocity), L.strides3(velocity[0]), nz, ny, nx, float(inv_dx),
-               L.stream_ptr())
-        written = [t for t in (field_adj, velocity_adj) if t is not None]
-        L.written(*written)
+        _eno3_adjoint("sopht_advection_flux_conservative_eno3_adjoint_3d", tag, field_adj, velocity_adj,
+                      flux_adj, field, velocity, inv_dx)
 
     return advection_flux_conservative_eno3_adjoint_kernel_3d
 
@@ -518,15 +523,17 @@ def eno3_advection_flux(field, velocity, inv_dx: float):
     import torch
 
     real_t = np.float32 if field.dtype == torch.float32 else np.float64
-    forward_kernel = gen_advection_flux_conservative_eno3_pyst_kernel_3d(real_t)
-    adjoint_kernel = gen_advection_flux_conservative_eno3_adjoint_kernel_3d(real_t)
+    tag = L.dtype_tag(real_t)
 
     class _ENO3Flux(torch.autograd.Function):
         @staticmethod
         def forward(ctx, f, u):
             f, u = f.contiguous(), u.contiguous()
-            flux = torch.zeros_like(f)
-            forward_kernel(flux, f, u, inv_dx)
+            flux = torch.empty_like(f)
+            nz, ny, nx = _shape3(f)
+            L.call("sopht_advection_flux_conservative_eno3_set_3d", tag, L.ptr(flux), L.strides3(flux),
+                   L.ptr(f), L.strides3(f), L.comps(u), L.strides3(u[0]), nz, ny, nx, float(inv_dx),
+                   L.stream_ptr())
             ctx.save_for_backward(f, u)
             return flux
 
@@ -534,10 +541,11 @@ def eno3_advection_flux(field, velocity, inv_dx: float):
         def backward(ctx, grad_flux):
             f, u = ctx.saved_tensors
             grad_flux = grad_flux.contiguous()
-            gf = torch.zeros_like(f) if ctx.needs_input_grad[0] else None
-            gu = torch.zeros_like(u) if ctx.needs_input_grad[1] else None
+            gf = torch.empty_like(f) if ctx.needs_input_grad[0] else None
+            gu = torch.empty_like(u) if ctx.needs_input_grad[1] else None
             if gf is not None or gu is not None:
-                adjoint_kernel(gf, gu, grad_flux, f, u, inv_dx)
+                _eno3_adjoint("sopht_advection_flux_conservative_eno3_adjoint_set_3d", tag, gf, gu, grad_flux, f, u,
+                              inv_dx)
             return gf, gu
 
     return _ENO3Flux.apply(field, velocity)
@@ -552,16 +560,19 @@ def gen_advection_timestep_euler_forward_conservative_eno3_pyst_kernel_3d(
     """``advection_timestep_3d.py:12-99``: zero flux, ENO3 flux with ``inv_dx=-dt_by_dx``,
     ``field += flux`` (per component for vectors)."""
     _check_field_type(field_type)
-    set_val = gen_set_fixed_val_pyst_kernel_3d(real_t)
-    flux_kernel = gen_advection_flux_conservative_eno3_pyst_kernel_3d(real_t)
-    add = gen_elementwise_sum_pyst_kernel_3d(real_t)
+    tag = L.dtype_tag(real_t)
+
+    def step(ncomp, fields, field, advection_flux, velocity, dt_by_dx):
+        nz, ny, nx = _shape3(field)
+        L.call("sopht_advection_timestep_euler_forward_conservative_eno3_3d", tag, ncomp, fields,
+               L.strides3(field), L.ptr(advection_flux), L.strides3(advection_flux), L.comps(velocity),
+               L.strides3(velocity[0]), nz, ny, nx, float(-dt_by_dx), L.stream_ptr())
+        L.written(field, advection_flux)
 
     def advection_timestep_euler_forward_conservative_eno3_pyst_kernel_3d(
         field, advection_flux, velocity, dt_by_dx: float
     ) -> None:
-        set_val(field=advection_flux, fixed_val=0)
-        flux_kernel(advection_flux=advection_flux, field=field, velocity=velocity, inv_dx=-dt_by_dx)
-        add(sum_field=field, field_1=field, field_2=advection_flux)
+        step(1, L.first(field), field, advection_flux, velocity, dt_by_dx)
 
     if field_type == "scalar":
         return advection_timestep_euler_forward_conservative_eno3_pyst_kernel_3d
@@ -569,10 +580,7 @@ def gen_advection_timestep_euler_forward_conservative_eno3_pyst_kernel_3d(
     def vector_field_advection_timestep_euler_forward_conservative_eno3_pyst_kernel_3d(
         vector_field, advection_flux, velocity, dt_by_dx: float
     ) -> None:
-        for i in range(3):
-            advection_timestep_euler_forward_conservative_eno3_pyst_kernel_3d(
-                vector_field[i], advection_flux, velocity, dt_by_dx
-            )
+        step(3, L.comps(vector_field), vector_field, advection_flux, velocity, dt_by_dx)
 
     return vector_field_advection_timestep_euler_forward_conservative_eno3_pyst_kernel_3d
 

@@ -98,3 +98,54 @@ def test_stretching_step_with_one_buffer_for_flux_and_midstep(dev, real_t):
     bound = 2 * 30 * float(np.finfo(real_t).eps) * 16
     np.testing.assert_allclose(to_host(wd), r, atol=bound, rtol=0)
     np.testing.assert_allclose(to_host(bd), buf, atol=bound, rtol=0)
+
+
+@pytest.mark.parametrize("shape", [(5, 5, 5), (6, 5, 6), (9, 7, 37), (36, 6, 66), (7, 5, 1031), (40, 12, 256)])
+def test_eno3_flux_and_step(dev, real_t, shape):
+    rng = np.random.default_rng(13)
+    f = rng.uniform(-1, 1, shape).astype(real_t)
+    u = rng.uniform(-1, 1, (3, *shape)).astype(real_t)
+    one = np.ones_like(f)
+    p = real_t(0.25)
+    f64, u64 = f.astype(np.float64), u.astype(np.float64)
+    # six faces of at most 4/3 each, four roundings a face and one an addition
+    bound = 2 * 6 * 5 * float(np.finfo(real_t).eps) * 2
+    ref = np.ones(shape)
+    S.advection_flux_conservative_eno3(ref, f64, u64, float(p))
+    kernel = spne().gen_advection_flux_conservative_eno3_pyst_kernel_3d(real_t)
+    both(lambda o, i: kernel(o[0], i[0], i[1], p), [one], [f, u], dev, [ref], bound)
+    flux = np.zeros(shape)
+    S.advection_flux_conservative_eno3(flux, f64, u64, -float(p))
+    step = spne().gen_advection_timestep_euler_forward_conservative_eno3_pyst_kernel_3d(real_t)
+    both(lambda o, i: step(o[0], o[1], i[0], p), [f, one], [u], dev, [f64 + flux, flux], bound)
+    w = rng.uniform(-1, 1, (3, *shape)).astype(real_t)
+    fluxes = np.zeros((3, *shape))
+    for c in range(3):
+        S.advection_flux_conservative_eno3(fluxes[c], w[c].astype(np.float64), u64, -float(p))
+    step3 = spne().gen_advection_timestep_euler_forward_conservative_eno3_pyst_kernel_3d(real_t, field_type="vector")
+    both(lambda o, i: step3(o[0], o[1], i[0], p), [w, one], [u], dev, [w.astype(np.float64) + fluxes, fluxes[2]], bound)
+    flux = spne().eno3_advection_flux(to_dev(f, dev), to_dev(u, dev), float(p))
+    np.testing.assert_allclose(to_host(flux), ref - 1, atol=bound, rtol=0)
+
+
+@pytest.mark.parametrize("shape", [(5, 5, 5), (6, 5, 6), (9, 7, 37), (36, 6, 66), (7, 5, 1031), (40, 12, 256)])
+def test_eno3_adjoint(dev, real_t, shape):
+    rng = np.random.default_rng(14)
+    f = rng.uniform(-1, 1, shape).astype(real_t)
+    u = rng.uniform(-1, 1, (3, *shape)).astype(real_t)
+    a = rng.uniform(-1, 1, shape).astype(real_t)
+    p = 0.25
+    # four weighted differences of at most 2 along each axis, then three products: about
+    # 12 roundings of values up to 3
+    bound = 2 * 12 * float(np.finfo(real_t).eps) * 3
+    fr, ur = np.zeros(shape), np.zeros((3, *shape))
+    S.advection_flux_conservative_eno3_adjoint(fr, ur, *(x.astype(np.float64) for x in (a, f, u)), p)
+    kernel = spne().gen_advection_flux_conservative_eno3_adjoint_kernel_3d(real_t)
+    both(lambda o, i: kernel(o[0], o[1], i[0], i[1], i[2], p), [np.ones_like(f), np.ones_like(u)], [a, f, u], dev,
+         [1 + fr, 1 + ur], bound)
+    both(lambda o, i: kernel(None, o[0], i[0], i[1], i[2], p), [np.ones_like(u)], [a, f, u], dev, [1 + ur], bound)
+    fd, ud = to_dev(f, dev).requires_grad_(), to_dev(u, dev).requires_grad_()
+    flux = spne().eno3_advection_flux(fd, ud, p)
+    flux.backward(to_dev(a, dev))
+    np.testing.assert_allclose(to_host(fd.grad), fr, atol=bound, rtol=0)
+    np.testing.assert_allclose(to_host(ud.grad), ur, atol=bound, rtol=0)

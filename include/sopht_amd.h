@@ -77,6 +77,11 @@ int sopht_diffusion_flux_3d(int dtype, void* flux, const int64_t* flux_strides,
                             const void* field, const int64_t* field_strides, int64_t nz,
                             int64_t ny, int64_t nx, double prefactor, int reset_ghost_zone,
                             void* stream);
+/* The three components of a vector field in one launch. */
+int sopht_diffusion_flux_vector_3d(int dtype, void* const flux[3], const int64_t* flux_strides,
+                                   const void* const field[3], const int64_t* field_strides,
+                                   int64_t nz, int64_t ny, int64_t nx, double prefactor, int reset,
+                                   void* stream);
 
 /* gen_diffusion_timestep_euler_forward_pyst_kernel_3d (scalar) —
  * .../diffusion_timestep_3d.py:12-80. flux (border reset) then field += flux. */
@@ -85,6 +90,11 @@ int sopht_diffusion_timestep_euler_forward_3d(int dtype, void* field,
                                               const int64_t* flux_strides, int64_t nz,
                                               int64_t ny, int64_t nx, double nu_dt_by_dx2,
                                               void* stream);
+/* Component by component through one scalar flux field, which keeps the last component's flux. */
+int sopht_diffusion_timestep_euler_forward_vector_3d(int dtype, void* const field[3],
+                                                     const int64_t* field_strides, void* flux,
+                                                     const int64_t* flux_strides, int64_t nz, int64_t ny,
+                                                     int64_t nx, double nu_dt_by_dx2, void* stream);
 
 /* gen_penalise_field_boundary_pyst_kernel_3d (scalar) —
  * .../penalise_field_boundary_3d.py:13-240. In place. sine_tables holds, for x then y then
@@ -93,6 +103,10 @@ int sopht_diffusion_timestep_euler_forward_3d(int dtype, void* field,
 int sopht_penalise_field_boundary_3d(int dtype, void* field, const int64_t* field_strides,
                                      int64_t nz, int64_t ny, int64_t nx, int width,
                                      const double* sine_tables, void* stream);
+/* The three components of a vector field in one launch. */
+int sopht_penalise_field_boundary_vector_3d(int dtype, void* const field[3], const int64_t* field_strides,
+                                            int64_t nz, int64_t ny, int64_t nx, int width,
+                                            const double* tables, void* stream);
 
 /* gen_divergence_pyst_kernel_3d — .../divergence_3d.py:13-96. */
 int sopht_divergence_3d(int dtype, void* divergence, const int64_t* divergence_strides,
@@ -105,14 +119,23 @@ int sopht_divergence_3d(int dtype, void* divergence, const int64_t* divergence_s
  * set_fixed_val_at_boundaries :200-268, complex_product :146-197 (interleaved complex). */
 int sopht_set_fixed_val_3d(int dtype, void* field, const int64_t* strides, int64_t nz,
                            int64_t ny, int64_t nx, double value, void* stream);
+int sopht_set_fixed_val_vector_3d(int dtype, void* const field[3], const int64_t* strides, int64_t nz,
+                                  int64_t ny, int64_t nx, const double* values, void* stream);
 int sopht_add_fixed_val_3d(int dtype, void* sum_field, const int64_t* sum_strides,
                            const void* field, const int64_t* field_strides, int64_t nz,
                            int64_t ny, int64_t nx, double value, void* stream);
+int sopht_add_fixed_val_vector_3d(int dtype, void* const sum[3], const int64_t* sum_strides,
+                                  const void* const field[3], const int64_t* field_strides, int64_t nz,
+                                  int64_t ny, int64_t nx, const double* values, void* stream);
 int sopht_elementwise_saxpby_3d(int dtype, void* sum_field, const int64_t* sum_strides,
                                 const void* field_1, const int64_t* f1_strides,
                                 const void* field_2, const int64_t* f2_strides, int64_t nz,
                                 int64_t ny, int64_t nx, double field_1_prefac,
                                 double field_2_prefac, void* stream);
+int sopht_elementwise_saxpby_vector_3d(int dtype, void* const sum[3], const int64_t* sum_strides,
+                                       const void* const f1[3], const int64_t* f1_strides,
+                                       const void* const f2[3], const int64_t* f2_strides, int64_t nz,
+                                       int64_t ny, int64_t nx, double a, double b, void* stream);
 int sopht_elementwise_sum_3d(int dtype, void* sum_field, const int64_t* sum_strides,
                              const void* field_1, const int64_t* f1_strides,
                              const void* field_2, const int64_t* f2_strides, int64_t nz,

@@ -86,6 +86,12 @@ SIGNATURES = {
         _i, _vp, _pi64, _vp, _pi64, _p3, _pi64, _i64, _i64, _i64, _d, _vp],
     "sopht_advection_timestep_euler_forward_conservative_eno3_3d": [
         _i, _i, _p3, _pi64, _vp, _pi64, _p3, _pi64, _i64, _i64, _i64, _d, _vp],
+    "sopht_diffusion_flux_vector_3d": [_i, _p3, _pi64, _p3, _pi64, _i64, _i64, _i64, _d, _i, _vp],
+    "sopht_diffusion_timestep_euler_forward_vector_3d": [_i, _p3, _pi64, _vp, _pi64, _i64, _i64, _i64, _d, _vp],
+    "sopht_penalise_field_boundary_vector_3d": [_i, _p3, _pi64, _i64, _i64, _i64, _i, _vp, _vp],
+    "sopht_set_fixed_val_vector_3d": [_i, _p3, _pi64, _i64, _i64, _i64, _vp, _vp],
+    "sopht_add_fixed_val_vector_3d": [_i, _p3, _pi64, _p3, _pi64, _i64, _i64, _i64, _vp, _vp],
+    "sopht_elementwise_saxpby_vector_3d": [_i, _p3, _pi64, _p3, _pi64, _p3, _pi64, _i64, _i64, _i64, _d, _d, _vp],
     "sopht_vorticity_stretching_timestep_3d": [
         _i, _i, _p3, _pi64, _p3, _pi64, _p3, _pi64, _vp, _vp, _i64, _i64, _i64, _d, _d, _vp],
     "sopht_poisson3d_create": [_i, _i64, _i64, _i64, _d, _vp, C.POINTER(_vp)],
@@ -224,6 +230,15 @@ def comps(v):
     stride, without building the component views)."""
     base, step = v.data_ptr(), v.stride(0) * v.element_size()
     return _p3(base, base + step, base + 2 * step)
+
+
+def is_vector(*fields) -> bool:
+    """Whether every field is one tensor of three components (not, say, a list of three)."""
+    return all(hasattr(v, "data_ptr") and v.dim() == 4 and v.shape[0] >= 3 for v in fields)
+
+
+def three_values(v) -> C.Array:
+    return (C.c_double * 3)(float(v[0]), float(v[1]), float(v[2]))
 
 
 def first(t):

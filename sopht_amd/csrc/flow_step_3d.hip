@@ -135,11 +135,9 @@ int step_impl(sopht_ns3d* P, const void* vort_in, void* vort_out, const void* ve
         if (rc) return rc;
       }
     }
-    for (int c = 0; c < 3; ++c) {
-      int rc = sopht_penalise_field_boundary_3d(P->dtype, w + c * n, st, g.nz, g.ny, g.nx, P->width,
-                                                P->sine, s);
-      if (rc) return rc;
-    }
+    void* const wc[3] = {w, w + n, w + 2 * n};
+    int rc = sopht_penalise_field_boundary_vector_3d(P->dtype, wc, st, g.nz, g.ny, g.nx, P->width, P->sine, s);
+    if (rc) return rc;
   } else {
     launch_sc<T>(ml, g, ps, w, F, pD, make_pen(P), wf && zero_forcing, s, fflags, s1m);
     SOPHT_CHECK_LAUNCH();
@@ -174,14 +172,12 @@ int recover_impl(sopht_ns3d* P, void* vort, void* vel, void* psi, const double* 
   const int64_t n = g.nz * g.ny * g.nx;
   T* w = static_cast<T*>(vort);
   T* ps = static_cast<T*>(psi);
-  for (int c = 0; c < 3; ++c) {
-    int rc = sopht_penalise_field_boundary_3d(P->dtype, w + c * n, st, g.nz, g.ny, g.nx, P->width,
-                                              P->sine, s);
-    if (rc) return rc;
-  }
+  void* const wc[3] = {w, w + n, w + 2 * n};
+  int rc = sopht_penalise_field_boundary_vector_3d(P->dtype, wc, st, g.nz, g.ny, g.nx, P->width, P->sine, s);
+  if (rc) return rc;
   void* const sol[3] = {ps, ps + n, ps + 2 * n};
   const void* const rhs[3] = {w, w + n, w + 2 * n};
-  int rc = P->fastdiag ? fastdiag_vector_solve_timed(P->fastdiag, sol, st, rhs, st, s, nullptr, 0)
+  rc = P->fastdiag ? fastdiag_vector_solve_timed(P->fastdiag, sol, st, rhs, st, s, nullptr, 0)
                        : sopht_poisson3d_vector_solve(P->poisson, sol, st, rhs, st, s);
   if (rc) return rc;
   const T U0 = P->with_free_stream ? T(U[0]) : T(0);

@@ -501,5 +501,218 @@ __global__ void __launch_bounds__(kRowThreads)
   }
 }
 
+// ------------------------------------------------------------------ curl, Laplacian, divergence
+
+// What a stencil kernel does with its output field.
+enum RowMode {
+  kRowInside,  // store the inside cells, leave the border
+  kRowReset,   // store the inside cells and zeros on the border
+  kRowAdd      // add to the inside cells
+};
+
+template <typename T, int MODE>
+__device__ __forceinline__ void row_out(const RowCol<T, 1>& c, const RowGeo& g, T* p, rvec<T> v, unsigned inside, int z) {
+  if constexpr (MODE == kRowAdd) {
+    if (inside) rstore(p, rload_own(c, g, static_cast<const T*>(p), z) + v, inside);
+  } else if constexpr (MODE == kRowReset) {
+#pragma unroll
+    for (int k = 0; k < RowVec<T>::V; ++k) v[k] = inside >> k & 1u ? v[k] : T(0);
+    rstore(p, v, c.own);
+  } else {
+    rstore(p, v, inside);
+  }
+}
+
+// p curl_h(f) (curl_3d.py:13-132) and its accumulating form
+// (update_vorticity_from_velocity_forcing_3d.py:12-132). Bound by memory: f0 and f1 are
+// differentiated along z and march in registers, so a plane costs 7 16-byte loads per thread.
+// 96 x 128 x 192 FP32 with the border reset: 16 us (3.5 TB/s) against 25 us with one cell per
+// thread plus six border launches of 2.4 to 5 us.
+template <typename T, int MODE>
+__global__ void __launch_bounds__(kRowThreads) k_curl_rows(RowGeo g, Rows3<T> o, Rows3<const T> f, T p) {
+  constexpr int V = RowVec<T>::V;
+  using vec = rvec<T>;
+  const RowCol<T, 1> c(g);
+  const int fr = c.yl * f.s.y + c.x, orow = c.y * o.s.y + c.x;
+  const int zm = c.z0 > 0 ? c.z0 - 1 : 0;
+  vec xm = rload(f.p[0] + zm * f.s.z + fr), ym = rload(f.p[1] + zm * f.s.z + fr);
+  vec xc = rload(f.p[0] + c.z0 * f.s.z + fr), yc = rload(f.p[1] + c.z0 * f.s.z + fr);
+  for (int z = c.z0; z < c.z1; ++z) {
+    const bool plane = z > 0 && z < g.nz - 1;  // the same for the whole workgroup
+    vec r0 = {}, r1 = {}, r2 = {}, xp = xc, yp = yc;
+    if (z < g.nz - 1) {
+      xp = rload(f.p[0] + (z + 1) * f.s.z + fr);
+      yp = rload(f.p[1] + (z + 1) * f.s.z + fr);
+    }
+    if (plane) {
+      const T* f0 = f.p[0] + z * f.s.z + fr;
+      const T* f2 = f.p[2] + z * f.s.z + fr;
+      const vec zc = rload(f2);
+      const vec z_yp = rload(f2 + f.s.y), z_ym = rload(f2 - f.s.y);
+      const vec x_yp = rload(f0 + f.s.y), x_ym = rload(f0 - f.s.y);
+      const T zl = from_prev_lane(zc[V - 1]), zr = from_next_lane(zc[0]);
+      const T yl = from_prev_lane(yc[V - 1]), yr = from_next_lane(yc[0]);
+#pragma unroll
+      for (int k = 0; k < V; ++k) {
+        const T z_r = k < V - 1 ? zc[k < V - 1 ? k + 1 : k] : zr, z_l = k > 0 ? zc[k > 0 ? k - 1 : k] : zl;
+        const T y_r = k < V - 1 ? yc[k < V - 1 ? k + 1 : k] : yr, y_l = k > 0 ? yc[k > 0 ? k - 1 : k] : yl;
+        r0[k] = p * (z_yp[k] - z_ym[k] - yp[k] + ym[k]);
+        r1[k] = p * (xp[k] - xm[k] - z_r + z_l);
+        r2[k] = p * (y_r - y_l - x_yp[k] + x_ym[k]);
+      }
+    }
+    const unsigned inside = plane && c.yin ? c.own & c.inner : 0u;
+    row_out<T, MODE>(c, g, o.p[0] + z * o.s.z + orow, r0, inside, z);
+    row_out<T, MODE>(c, g, o.p[1] + z * o.s.z + orow, r1, inside, z);
+    row_out<T, MODE>(c, g, o.p[2] + z * o.s.z + orow, r2, inside, z);
+    xm = xc;
+    xc = xp;
+    ym = yc;
+    yc = yp;
+  }
+}
+
+// p lap_h(f) of one scalar field per gridDim.y (diffusion_flux_3d.py:14-115). Bound by memory:
+// 130 x 170 x 250 FP32, 10.4 us (4.2 TB/s) against 21 us with one cell per thread plus six
+// border launches of 2.2 to 4.6 us.
+template <typename T, int MODE>
+__global__ void __launch_bounds__(kRowThreads) k_laplacian_rows(RowGeo g, Rows3<T> o, Rows3<const T> in, T p) {
+  constexpr int V = RowVec<T>::V;
+  using vec = rvec<T>;
+  const RowCol<T, 1> c(g);
+  const T* const f = in.p[blockIdx.y];
+  T* const out = o.p[blockIdx.y];
+  const int fr = c.yl * in.s.y + c.x, orow = c.y * o.s.y + c.x;
+  vec fm = rload(f + (c.z0 > 0 ? c.z0 - 1 : 0) * in.s.z + fr), fc = rload(f + c.z0 * in.s.z + fr);
+  for (int z = c.z0; z < c.z1; ++z) {
+    const bool plane = z > 0 && z < g.nz - 1;
+    const T* fz = f + z * in.s.z + fr;
+    vec r = {}, fp = fc;
+    if (z < g.nz - 1) fp = rload(fz + in.s.z);
+    if (plane) {
+      const vec yp = rload(fz + in.s.y), ym = rload(fz - in.s.y);
+      const T xl = from_prev_lane(fc[V - 1]), xr = from_next_lane(fc[0]);
+#pragma unroll
+      for (int k = 0; k < V; ++k) {
+        const T right = k < V - 1 ? fc[k < V - 1 ? k + 1 : k] : xr, left = k > 0 ? fc[k > 0 ? k - 1 : k] : xl;
+        r[k] = p * (fp[k] + fm[k] + yp[k] + ym[k] + right + left - T(6) * fc[k]);
+      }
+    }
+    const unsigned inside = plane && c.yin ? c.own & c.inner : 0u;
+    row_out<T, MODE>(c, g, out + z * o.s.z + orow, r, inside, z);
+    fm = fc;
+    fc = fp;
+  }
+}
+
+// div_h(f) (divergence_3d.py:13-96). Bound by memory: 130 x 170 x 250 FP32,
+// 15 us (5.8 TB/s) against 23 us with one cell per thread plus six border launches.
+template <typename T, int MODE>
+__global__ void __launch_bounds__(kRowThreads)
+    k_divergence_rows(RowGeo g, T* out, RowStrides os, Rows3<const T> f, T inv_dx) {
+  constexpr int V = RowVec<T>::V;
+  using vec = rvec<T>;
+  const RowCol<T, 1> c(g);
+  const int fr = c.yl * f.s.y + c.x, orow = c.y * os.y + c.x;
+  vec zm = rload(f.p[2] + (c.z0 > 0 ? c.z0 - 1 : 0) * f.s.z + fr), zc = rload(f.p[2] + c.z0 * f.s.z + fr);
+  for (int z = c.z0; z < c.z1; ++z) {
+    const bool plane = z > 0 && z < g.nz - 1;
+    vec r = {}, zp = zc;
+    if (z < g.nz - 1) zp = rload(f.p[2] + (z + 1) * f.s.z + fr);
+    if (plane) {
+      const vec xc = rload(f.p[0] + z * f.s.z + fr);
+      const vec yp = rload(f.p[1] + z * f.s.z + fr + f.s.y), ym = rload(f.p[1] + z * f.s.z + fr - f.s.y);
+      const T xl = from_prev_lane(xc[V - 1]), xr = from_next_lane(xc[0]);
+#pragma unroll
+      for (int k = 0; k < V; ++k) {
+        const T right = k < V - 1 ? xc[k < V - 1 ? k + 1 : k] : xr, left = k > 0 ? xc[k > 0 ? k - 1 : k] : xl;
+        r[k] = T(0.5) * inv_dx * (right - left + yp[k] - ym[k] + zp[k] - zm[k]);
+      }
+    }
+    const unsigned inside = plane && c.yin ? c.own & c.inner : 0u;
+    row_out<T, MODE>(c, g, out + z * os.z + orow, r, inside, z);
+    zm = zc;
+    zc = zp;
+  }
+}
+
+// ------------------------------------------------------------------ pointwise operators
+
+// Whether the fields of a box are dense: their cells follow each other without gaps.
+inline bool dense(const int64_t* s, int64_t ny, int64_t nx) { return s[2] == 1 && s[1] == nx && s[0] == ny * nx; }
+
+template <typename T, int N>
+struct Flat {
+  T* out[3];
+  const T* in[N > 0 ? N : 1][3];
+  int64_t n;  // cells
+};
+
+// out = fn(comp, in...) over the cells of up to three dense components (gridDim.y), 16 bytes a
+// thread. Bound by memory: the sum of two 130 x 170 x 250 FP32 fields takes 10.9 us (6.1 TB/s, most
+// of it from the caches) against 18.4 us with one cell per thread and 64-bit divisions.
+template <typename T, int N, typename Fn>
+__global__ void __launch_bounds__(256) k_flat(Flat<T, N> a, Fn fn) {
+  constexpr int V = RowVec<T>::V;
+  const int c = int(blockIdx.y);
+  const int64_t i = (blockIdx.x * int64_t(256) + threadIdx.x) * V;
+  auto one = [&](const T* v) -> T {
+    if constexpr (N == 0) return fn(c);
+    else if constexpr (N == 1) return fn(c, v[0]);
+    else return fn(c, v[0], v[1]);
+  };
+  if (i + V <= a.n) {
+    rvec<T> in[N > 0 ? N : 1] = {}, o;
+#pragma unroll
+    for (int q = 0; q < N; ++q) in[q] = rload(a.in[q][c] + i);
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+      T v[N > 0 ? N : 1] = {};
+#pragma unroll
+      for (int q = 0; q < N; ++q) v[q] = in[q][k];
+      o[k] = one(v);
+    }
+    *reinterpret_cast<rvec<T>*>(a.out[c] + i) = o;
+  } else {
+    for (int64_t j = i; j < a.n; ++j) {
+      T v[N > 0 ? N : 1] = {};
+      for (int q = 0; q < N; ++q) v[q] = a.in[q][c][j];
+      a.out[c][j] = one(v);
+    }
+  }
+}
+
+// result = a x b on dense fields (elementwise_ops_3d.py:390-449). 96 x 128 x 192 FP32: 13.4 us
+// (6.3 TB/s) against 18 us with one cell per thread.
+template <typename T>
+__global__ void __launch_bounds__(256) k_cross_flat(Flat<T, 2> f) {
+  constexpr int V = RowVec<T>::V;
+  const int64_t i = (blockIdx.x * int64_t(256) + threadIdx.x) * V;
+  if (i + V <= f.n) {
+    rvec<T> a[3], b[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      a[c] = rload(f.in[0][c] + i);
+      b[c] = rload(f.in[1][c] + i);
+    }
+    *reinterpret_cast<rvec<T>*>(f.out[0] + i) = a[1] * b[2] - b[1] * a[2];
+    *reinterpret_cast<rvec<T>*>(f.out[1] + i) = a[2] * b[0] - b[2] * a[0];
+    *reinterpret_cast<rvec<T>*>(f.out[2] + i) = a[0] * b[1] - b[0] * a[1];
+  } else {
+    for (int64_t j = i; j < f.n; ++j) {
+      const T a0 = f.in[0][0][j], a1 = f.in[0][1][j], a2 = f.in[0][2][j];
+      const T b0 = f.in[1][0][j], b1 = f.in[1][1][j], b2 = f.in[1][2][j];
+      f.out[0][j] = a1 * b2 - b1 * a2;
+      f.out[1][j] = a2 * b0 - b2 * a0;
+      f.out[2][j] = a0 * b1 - b0 * a1;
+    }
+  }
+}
+
+template <typename T>
+inline dim3 flat_grid(int64_t n, int comps) {
+  return dim3(unsigned((n + 256 * RowVec<T>::V - 1) / (256 * RowVec<T>::V)), unsigned(comps));
+}
+
 }  // namespace
 }  // namespace sopht

@@ -1,9 +1,11 @@
 // Standalone drop-in grid stencils (the gen_*_pyst_kernel_3d family) for gfx950.
 //
 // These keep the reference's per-op semantics exactly (which cells each op writes, border
-// resets, strided views) and run one thread per written cell with x-fastest lanes, so
-// every neighbour access along x is coalesced and y/z neighbours come from L2. The flow
-// step itself does not use them: it runs the fused sweeps in flow_step_3d.hip.
+// resets, strided views). Fields whose cells are adjacent along x go to the row-vector kernels
+// (row_march.h; pointwise operators need dense fields), which write the border in the same
+// launch; other strides run one thread per written cell with x-fastest lanes and a launch per
+// border slab. The flow step itself does not use them: it runs the fused sweeps in
+// flow_step_3d.hip.
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -94,17 +96,25 @@ __global__ void __launch_bounds__(256) shell_kernel(int64_t z0, int64_t y0, int6
   }
 }
 
+// comps repeats the box over gridDim.y (fn reads the component from blockIdx.y).
 template <typename Fn>
-int launch_shell(int64_t z0, int64_t y0, int64_t x0, int64_t bz, int64_t by, int64_t bx, Fn fn,
+int launch_shell(int64_t z0, int64_t y0, int64_t x0, int64_t bz, int64_t by, int64_t bx, int comps, Fn fn,
                  hipStream_t s) {
-  if (bz < 2 || by < 2 || bx < 2) return launch_box(z0, y0, x0, bz, by, bx, fn, s);
-  const int64_t total = 2 * (by * bx + (bz - 2) * bx + (bz - 2) * (by - 2));
+  const bool shell = bz >= 2 && by >= 2 && bx >= 2;
+  const int64_t total = shell ? 2 * (by * bx + (bz - 2) * bx + (bz - 2) * (by - 2)) : bz * by * bx;
+  if (total <= 0) return SOPHT_OK;
   int blocks = ceil_div(total, 256);
   if (blocks > 65536) blocks = 65536;
-  shell_kernel<<<blocks, 256, 0, s>>>(z0, y0, x0, bz, by, bx, fn);
+  const dim3 grid{unsigned(blocks), unsigned(comps), 1u};
+  if (shell)
+    shell_kernel<<<grid, 256, 0, s>>>(z0, y0, x0, bz, by, bx, fn);
+  else
+    box_kernel<<<grid, 256, 0, s>>>(z0, y0, x0, bz, by, bx, fn);
   SOPHT_CHECK_LAUNCH();
   return SOPHT_OK;
 }
+
+constexpr int kRowChunk = 16;  // planes per workgroup of the curl, Laplacian and divergence
 
 inline hipStream_t as_stream(void* s) { return static_cast<hipStream_t>(s); }
 
@@ -113,6 +123,13 @@ template <typename T>
 int curl_impl(void* const out[3], const int64_t* os, const void* const in[3], const int64_t* is,
               int64_t nz, int64_t ny, int64_t nx, T p, int reset, bool accumulate,
               hipStream_t s) {
+  if (row_box_ok<T, 1>(nz, ny, nx) && row_strides_ok(os, nz, ny, nx) && row_strides_ok(is, nz, ny, nx)) {
+    const RowGeo g = row_geo<T>(nz, ny, nx, kRowChunk);
+    auto* kernel = accumulate ? k_curl_rows<T, kRowAdd> : (reset ? k_curl_rows<T, kRowReset> : k_curl_rows<T, kRowInside>);
+    kernel<<<row_blocks(g), kRowThreads, 0, s>>>(g, rows3<T>(out, os), rows3<T>(in, is), p);
+    SOPHT_CHECK_LAUNCH();
+    return SOPHT_OK;
+  }
   View3<T> o0 = make_view<T>(out[0], os), o1 = make_view<T>(out[1], os),
            o2 = make_view<T>(out[2], os);
   View3<T> fx = make_view<T>(in[0], is), fy = make_view<T>(in[1], is), fz = make_view<T>(in[2], is);
@@ -180,6 +197,18 @@ template <typename T>
 int cross_impl(void* const r[3], const int64_t* rs, const void* const a[3], const int64_t* as,
                const void* const b[3], const int64_t* bs, int64_t nz, int64_t ny, int64_t nx,
                hipStream_t s) {
+  if (dense(rs, ny, nx) && dense(as, ny, nx) && dense(bs, ny, nx)) {
+    Flat<T, 2> f{};
+    f.n = nz * ny * nx;
+    for (int c = 0; c < 3; ++c) {
+      f.out[c] = static_cast<T*>(r[c]);
+      f.in[0][c] = static_cast<const T*>(a[c]);
+      f.in[1][c] = static_cast<const T*>(b[c]);
+    }
+    k_cross_flat<T><<<flat_grid<T>(f.n, 1), 256, 0, s>>>(f);
+    SOPHT_CHECK_LAUNCH();
+    return SOPHT_OK;
+  }
   View3<T> r0 = make_view<T>(r[0], rs), r1 = make_view<T>(r[1], rs), r2 = make_view<T>(r[2], rs);
   View3<T> a0 = make_view<T>(a[0], as), a1 = make_view<T>(a[1], as), a2 = make_view<T>(a[2], as);
   View3<T> b0 = make_view<T>(b[0], bs), b1 = make_view<T>(b[1], bs), b2 = make_view<T>(b[2], bs);
@@ -195,30 +224,144 @@ int cross_impl(void* const r[3], const int64_t* rs, const void* const a[3], cons
       s);
 }
 
-template <typename T>
-int diffusion_flux_impl(void* flux, const int64_t* fs, const void* field, const int64_t* is,
-                        int64_t nz, int64_t ny, int64_t nx, T p, int reset, hipStream_t s) {
-  View3<T> o = make_view<T>(flux, fs), f = make_view<T>(field, is);
-  int rc = SOPHT_OK;
-  if (nz > 2 && ny > 2 && nx > 2) {
-    rc = launch_box(
-        1, 1, 1, nz - 2, ny - 2, nx - 2,
+// out = fn(comp, in...) over ncomp fields of one box; flat over dense fields.
+template <typename T, int N, typename Fn>
+int pointwise(int ncomp, void* const* out, const int64_t* os, const void* const* const* in, const int64_t* const* is,
+              int64_t nz, int64_t ny, int64_t nx, Fn fn, hipStream_t s) {
+  bool flat = dense(os, ny, nx);
+  for (int q = 0; q < N; ++q) flat = flat && dense(is[q], ny, nx);
+  if (flat) {
+    Flat<T, N> f{};
+    f.n = nz * ny * nx;
+    for (int c = 0; c < ncomp; ++c) {
+      f.out[c] = static_cast<T*>(out[c]);
+      for (int q = 0; q < N; ++q) f.in[q][c] = static_cast<const T*>(in[q][c]);
+    }
+    k_flat<T, N><<<flat_grid<T>(f.n, ncomp), 256, 0, s>>>(f, fn);
+    SOPHT_CHECK_LAUNCH();
+    return SOPHT_OK;
+  }
+  for (int c = 0; c < ncomp; ++c) {
+    View3<T> o = make_view<T>(out[c], os), a = o, b = o;
+    if constexpr (N > 0) a = make_view<T>(in[0][c], is[0]);
+    if constexpr (N > 1) b = make_view<T>(in[1][c], is[1]);
+    int rc = launch_box(
+        0, 0, 0, nz, ny, nx,
         [=] __device__(int64_t z, int64_t y, int64_t x) {
-          o(z, y, x) = p * (f(z + 1, y, x) + f(z - 1, y, x) + f(z, y + 1, x) + f(z, y - 1, x) +
-                            f(z, y, x + 1) + f(z, y, x - 1) - T(6) * f(z, y, x));
+          if constexpr (N == 0) o(z, y, x) = fn(c);
+          else if constexpr (N == 1) o(z, y, x) = fn(c, a(z, y, x));
+          else o(z, y, x) = fn(c, a(z, y, x), b(z, y, x));
         },
         s);
     if (rc) return rc;
   }
-  if (reset)
-    rc = launch_boundary_slabs(
-        nz, ny, nx, 1, [=] __device__(int64_t z, int64_t y, int64_t x) { o(z, y, x) = T(0); }, s);
+  return SOPHT_OK;
+}
+
+template <typename T>
+struct Three {
+  T v[3];
+};
+
+template <typename T>
+int set_impl(int ncomp, void* const* out, const int64_t* os, int64_t nz, int64_t ny, int64_t nx, Three<T> value,
+             hipStream_t s) {
+  return pointwise<T, 0>(ncomp, out, os, nullptr, nullptr, nz, ny, nx,
+                         [=] __device__(int c) -> T { return value.v[c]; }, s);
+}
+
+template <typename T>
+int add_fixed_impl(int ncomp, void* const* out, const int64_t* os, const void* const* in, const int64_t* is,
+                   int64_t nz, int64_t ny, int64_t nx, Three<T> value, hipStream_t s) {
+  const void* const* ins[1] = {in};
+  const int64_t* iss[1] = {is};
+  return pointwise<T, 1>(ncomp, out, os, ins, iss, nz, ny, nx,
+                         [=] __device__(int c, T a) -> T { return a + value.v[c]; }, s);
+}
+
+// out = ta a + tb b
+template <typename T>
+int axpby_impl(int ncomp, void* const* out, const int64_t* os, const void* const* a, const int64_t* as,
+               const void* const* b, const int64_t* bs, int64_t nz, int64_t ny, int64_t nx, T ta, T tb, hipStream_t s) {
+  const void* const* ins[2] = {a, b};
+  const int64_t* iss[2] = {as, bs};
+  if (ta == T(1) && tb == T(1))  // a sum: the same value, without the products
+    return pointwise<T, 2>(ncomp, out, os, ins, iss, nz, ny, nx,
+                           [=] __device__(int, T x, T y) -> T { return x + y; }, s);
+  return pointwise<T, 2>(ncomp, out, os, ins, iss, nz, ny, nx,
+                         [=] __device__(int, T x, T y) -> T { return ta * x + tb * y; }, s);
+}
+
+template <typename T>
+int copy_impl(void* out, const int64_t* os, const void* in, const int64_t* is, int64_t nz, int64_t ny, int64_t nx,
+              hipStream_t s) {
+  const void* const* ins[1] = {&in};
+  const int64_t* iss[1] = {is};
+  return pointwise<T, 1>(1, &out, os, ins, iss, nz, ny, nx, [=] __device__(int, T a) -> T { return a; }, s);
+}
+
+template <typename T>
+int diffusion_flux_impl(int ncomp, void* const* flux, const int64_t* fs, const void* const* field, const int64_t* is,
+                        int64_t nz, int64_t ny, int64_t nx, T p, int reset, hipStream_t s) {
+  if (row_box_ok<T, 1>(nz, ny, nx) && row_strides_ok(fs, nz, ny, nx) && row_strides_ok(is, nz, ny, nx)) {
+    const RowGeo g = row_geo<T>(nz, ny, nx, kRowChunk);
+    Rows3<T> o{};
+    Rows3<const T> in{};
+    o.s = row_strides(fs);
+    in.s = row_strides(is);
+    for (int c = 0; c < ncomp; ++c) {
+      o.p[c] = static_cast<T*>(flux[c]);
+      in.p[c] = static_cast<const T*>(field[c]);
+    }
+    auto* kernel = reset ? k_laplacian_rows<T, kRowReset> : k_laplacian_rows<T, kRowInside>;
+    kernel<<<dim3(row_blocks(g), unsigned(ncomp)), kRowThreads, 0, s>>>(g, o, in, p);
+    SOPHT_CHECK_LAUNCH();
+    return SOPHT_OK;
+  }
+  int rc = SOPHT_OK;
+  for (int c = 0; c < ncomp && !rc; ++c) {
+    View3<T> o = make_view<T>(flux[c], fs), f = make_view<T>(field[c], is);
+    if (nz > 2 && ny > 2 && nx > 2) {
+      rc = launch_box(
+          1, 1, 1, nz - 2, ny - 2, nx - 2,
+          [=] __device__(int64_t z, int64_t y, int64_t x) {
+            o(z, y, x) = p * (f(z + 1, y, x) + f(z - 1, y, x) + f(z, y + 1, x) + f(z, y - 1, x) +
+                              f(z, y, x + 1) + f(z, y, x - 1) - T(6) * f(z, y, x));
+          },
+          s);
+    }
+    if (reset && !rc)
+      rc = launch_boundary_slabs(
+          nz, ny, nx, 1, [=] __device__(int64_t z, int64_t y, int64_t x) { o(z, y, x) = T(0); }, s);
+  }
   return rc;
+}
+
+// flux = p lap_h(field), 0 on the border, then field += flux, component by component through
+// one scalar flux field (diffusion_timestep_3d.py:12-80).
+template <typename T>
+int diffusion_step_impl(int ncomp, void* const* field, const int64_t* fs, void* flux, const int64_t* xs, int64_t nz,
+                        int64_t ny, int64_t nx, T p, hipStream_t s) {
+  for (int c = 0; c < ncomp; ++c) {
+    const void* f = field[c];
+    const void* x = flux;
+    int rc = diffusion_flux_impl<T>(1, &flux, xs, &f, fs, nz, ny, nx, p, 1, s);
+    if (!rc) rc = axpby_impl<T>(1, &field[c], fs, &f, fs, &x, xs, nz, ny, nx, T(1), T(1), s);
+    if (rc) return rc;
+  }
+  return SOPHT_OK;
 }
 
 template <typename T>
 int divergence_impl(void* div, const int64_t* ds, const void* const in[3], const int64_t* is,
                     int64_t nz, int64_t ny, int64_t nx, T inv_dx, int reset, hipStream_t s) {
+  if (row_box_ok<T, 1>(nz, ny, nx) && row_strides_ok(ds, nz, ny, nx) && row_strides_ok(is, nz, ny, nx)) {
+    const RowGeo g = row_geo<T>(nz, ny, nx, kRowChunk);
+    auto* kernel = reset ? k_divergence_rows<T, kRowReset> : k_divergence_rows<T, kRowInside>;
+    kernel<<<row_blocks(g), kRowThreads, 0, s>>>(g, static_cast<T*>(div), row_strides(ds), rows3<T>(in, is), inv_dx);
+    SOPHT_CHECK_LAUNCH();
+    return SOPHT_OK;
+  }
   View3<T> o = make_view<T>(div, ds);
   View3<T> fx = make_view<T>(in[0], is), fy = make_view<T>(in[1], is), fz = make_view<T>(in[2], is);
   int rc = SOPHT_OK;
@@ -252,7 +395,7 @@ struct SineTables {
 };
 
 template <typename T>
-int penalise_impl(void* field, const int64_t* fs, int64_t nz, int64_t ny, int64_t nx, int w,
+int penalise_impl(int ncomp, void* const* fields, const int64_t* fs, int64_t nz, int64_t ny, int64_t nx, int w,
                   const double* tables, hipStream_t s) {
   if (w == 0) return SOPHT_OK;
   SOPHT_REQUIRE(w > 0 && w <= 8, "penalty width must be in [0, 8]");
@@ -263,13 +406,17 @@ int penalise_impl(void* field, const int64_t* fs, int64_t nz, int64_t ny, int64_
       st.f[a][i] = T(tables[a * 2 * w + i]);
       st.b[a][i] = T(tables[a * 2 * w + w + i]);
     }
-  View3<T> f = make_view<T>(field, fs);
+  Rows3<T> fields3{};
+  for (int c = 0; c < ncomp; ++c) fields3.p[c] = static_cast<T*>(fields[c]);
+  const View3<T> shape = make_view<T>(static_cast<void*>(nullptr), fs);
   const int64_t cz0 = w - 1, cz1 = nz - w, cy0 = w - 1, cy1 = ny - w, cx0 = w - 1, cx1 = nx - w;
   const int64_t bz = cz1 - cz0 + 1, by = cy1 - cy0 + 1, bx = cx1 - cx0 + 1;
   // only the surface of the core box [w-1, n-w]^3 has work: one thread per surface cell
   return launch_shell(
-      cz0, cy0, cx0, bz, by, bx,
+      cz0, cy0, cx0, bz, by, bx, ncomp,
       [=] __device__(int64_t z, int64_t y, int64_t x) {
+        View3<T> f = shape;
+        f.p = blockIdx.y == 0 ? fields3.p[0] : (blockIdx.y == 1 ? fields3.p[1] : fields3.p[2]);
         const bool onz = (z == cz0) || (z == cz1), ony = (y == cy0) || (y == cy1),
                    onx = (x == cx0) || (x == cx1);
         if (!(onz || ony || onx)) return;
@@ -470,9 +617,7 @@ int eno3_set_impl(void* flux, const int64_t* fs, const void* field, const int64_
   for (int a = 0; a < 3; ++a) apart = apart && !fields_meet<T>(flux, fs, vel[a], vs, nz, ny, nx);
   if (apart && eno3_rows_ok<T>(fs, is, vs, nz, ny, nx) && !fields_meet<T>(flux, fs, field, is, nz, ny, nx))
     return eno3_rows<T, true>(flux, fs, field, is, vel, vs, nz, ny, nx, inv_dx, s);
-  View3<T> o = make_view<T>(flux, fs);
-  int rc = launch_box(
-      0, 0, 0, nz, ny, nx, [=] __device__(int64_t z, int64_t y, int64_t x) { o(z, y, x) = T(0); }, s);
+  int rc = set_impl<T>(1, &flux, fs, nz, ny, nx, Three<T>{}, s);
   return rc ? rc : eno3_impl<T>(flux, fs, field, is, vel, vs, nz, ny, nx, inv_dx, s);
 }
 
@@ -485,10 +630,9 @@ int eno3_step_impl(int ncomp, void* const field[3], const int64_t* is, void* flu
   for (int c = 0; c < ncomp; ++c) {
     int rc = eno3_set_impl<T>(flux, fs, field[c], is, vel, vs, nz, ny, nx, inv_dx, s);
     if (rc) return rc;
-    View3<T> f = make_view<T>(field[c], is), o = make_view<T>(flux, fs);
-    rc = launch_box(
-        0, 0, 0, nz, ny, nx,
-        [=] __device__(int64_t z, int64_t y, int64_t x) { f(z, y, x) = f(z, y, x) + o(z, y, x); }, s);
+    const void* f = field[c];
+    const void* x = flux;
+    rc = axpby_impl<T>(1, &field[c], is, &f, is, &x, fs, nz, ny, nx, T(1), T(1), s);
     if (rc) return rc;
   }
   return SOPHT_OK;
@@ -581,15 +725,8 @@ int eno3_adjoint_impl(void* field_adj, const int64_t* fas, void* const vel_adj[3
                     row_strides_ok(is, nz, ny, nx) && row_strides_ok(vs, nz, ny, nx) &&
                     (!has_f || row_strides_ok(fas, nz, ny, nx)) && (!has_v || row_strides_ok(vas, nz, ny, nx));
   if (set && !rows) {  // clear, then add
-    int rc = SOPHT_OK;
-    auto clear = [&](void* p, const int64_t* st) {
-      View3<T> o = make_view<T>(p, st);
-      if (!rc)
-        rc = launch_box(
-            0, 0, 0, nz, ny, nx, [=] __device__(int64_t z, int64_t y, int64_t x) { o(z, y, x) = T(0); }, s);
-    };
-    if (has_f) clear(field_adj, fas);
-    for (int a = 0; has_v && a < 3; ++a) clear(vel_adj[a], vas);
+    int rc = has_f ? set_impl<T>(1, &field_adj, fas, nz, ny, nx, Three<T>{}, s) : SOPHT_OK;
+    if (has_v && !rc) rc = set_impl<T>(3, vel_adj, vas, nz, ny, nx, Three<T>{}, s);
     if (rc) return rc;
   }
   if (nz <= 4 || ny <= 4 || nx <= 4) return SOPHT_OK;
@@ -684,15 +821,6 @@ int stretching_impl(void* const flux[3], const int64_t* fs, const void* const w[
   return SOPHT_OK;
 }
 
-template <typename T>
-int axpby(void* out, const int64_t* os, const void* a, const int64_t* as, const void* b, const int64_t* bs,
-          int64_t nz, int64_t ny, int64_t nx, T ta, T tb, hipStream_t s) {
-  View3<T> o = make_view<T>(out, os), x1 = make_view<T>(a, as), x2 = make_view<T>(b, bs);
-  return launch_box(
-      0, 0, 0, nz, ny, nx,
-      [=] __device__(int64_t z, int64_t y, int64_t x) { o(z, y, x) = ta * x1(z, y, x) + tb * x2(z, y, x); }, s);
-}
-
 // Euler (scheme 0) and SSPRK3 (scheme 1) stretching steps. One pass where the row-vector
 // kernel takes the fields and none of the fields it writes meets another operand; otherwise
 // the sequence of fluxes, sums and axpbys of the reference, which reads and writes in its order.
@@ -728,7 +856,7 @@ int stretching_step_impl(int scheme, void* const w[3], const int64_t* ws, const 
   int rc = SOPHT_OK;
   auto add = [&](void* const o[3], const int64_t* os, const void* const a[3], const int64_t* as, T ta,
                  const void* const b[3], const int64_t* bs, T tb) {
-    for (int c = 0; c < 3 && !rc; ++c) rc = axpby<T>(o[c], os, a[c], as, b[c], bs, nz, ny, nx, ta, tb, s);
+    if (!rc) rc = axpby_impl<T>(3, o, os, a, as, b, bs, nz, ny, nx, ta, tb, s);
   };
   auto stage = [&](void* const v[3], const int64_t* vs, T q) {
     if (!rc) rc = stretching_impl<T>(flux, fs, v, vs, u, us, nz, ny, nx, q, s);
@@ -878,20 +1006,29 @@ int sopht_diffusion_flux_3d(int dtype, void* flux, const int64_t* fs, const void
                             const int64_t* is, int64_t nz, int64_t ny, int64_t nx,
                             double prefactor, int reset, void* stream) {
   REQUIRE_GRID(nz, ny, nx);
-  DISPATCH(dtype, diffusion_flux_impl<T>(flux, fs, field, is, nz, ny, nx, T(prefactor), reset,
+  DISPATCH(dtype, diffusion_flux_impl<T>(1, &flux, fs, &field, is, nz, ny, nx, T(prefactor), reset,
                                          as_stream(stream)));
 }
 
-int sopht_elementwise_sum_3d(int dtype, void* sum, const int64_t* ss, const void* f1,
-                             const int64_t* s1, const void* f2, const int64_t* s2, int64_t nz,
-                             int64_t ny, int64_t nx, void* stream);
+int sopht_diffusion_flux_vector_3d(int dtype, void* const flux[3], const int64_t* fs, const void* const field[3],
+                                   const int64_t* is, int64_t nz, int64_t ny, int64_t nx, double prefactor,
+                                   int reset, void* stream) {
+  REQUIRE_GRID(nz, ny, nx);
+  DISPATCH(dtype, diffusion_flux_impl<T>(3, flux, fs, field, is, nz, ny, nx, T(prefactor), reset, as_stream(stream)));
+}
 
 int sopht_diffusion_timestep_euler_forward_3d(int dtype, void* field, const int64_t* fs,
                                               void* flux, const int64_t* xs, int64_t nz,
                                               int64_t ny, int64_t nx, double p, void* stream) {
-  int rc = sopht_diffusion_flux_3d(dtype, flux, xs, field, fs, nz, ny, nx, p, 1, stream);
-  if (rc) return rc;
-  return sopht_elementwise_sum_3d(dtype, field, fs, field, fs, flux, xs, nz, ny, nx, stream);
+  REQUIRE_GRID(nz, ny, nx);
+  DISPATCH(dtype, diffusion_step_impl<T>(1, &field, fs, flux, xs, nz, ny, nx, T(p), as_stream(stream)));
+}
+
+int sopht_diffusion_timestep_euler_forward_vector_3d(int dtype, void* const field[3], const int64_t* fs, void* flux,
+                                                     const int64_t* xs, int64_t nz, int64_t ny, int64_t nx, double p,
+                                                     void* stream) {
+  REQUIRE_GRID(nz, ny, nx);
+  DISPATCH(dtype, diffusion_step_impl<T>(3, field, fs, flux, xs, nz, ny, nx, T(p), as_stream(stream)));
 }
 
 int sopht_penalise_field_boundary_3d(int dtype, void* field, const int64_t* fs, int64_t nz,
@@ -899,7 +1036,15 @@ int sopht_penalise_field_boundary_3d(int dtype, void* field, const int64_t* fs, 
                                      void* stream) {
   REQUIRE_GRID(nz, ny, nx);
   SOPHT_REQUIRE(width >= 0, "Invalid width for boundary zone, must be a non-negative integer");
-  DISPATCH(dtype, penalise_impl<T>(field, fs, nz, ny, nx, width, tables, as_stream(stream)));
+  DISPATCH(dtype, penalise_impl<T>(1, &field, fs, nz, ny, nx, width, tables, as_stream(stream)));
+}
+
+int sopht_penalise_field_boundary_vector_3d(int dtype, void* const field[3], const int64_t* fs, int64_t nz,
+                                            int64_t ny, int64_t nx, int width, const double* tables,
+                                            void* stream) {
+  REQUIRE_GRID(nz, ny, nx);
+  SOPHT_REQUIRE(width >= 0, "Invalid width for boundary zone, must be a non-negative integer");
+  DISPATCH(dtype, penalise_impl<T>(3, field, fs, nz, ny, nx, width, tables, as_stream(stream)));
 }
 
 int sopht_divergence_3d(int dtype, void* div, const int64_t* ds, const void* const field[3],
@@ -913,71 +1058,60 @@ int sopht_divergence_3d(int dtype, void* div, const int64_t* ds, const void* con
 int sopht_set_fixed_val_3d(int dtype, void* field, const int64_t* st, int64_t nz, int64_t ny,
                            int64_t nx, double value, void* stream) {
   REQUIRE_GRID(nz, ny, nx);
-  DISPATCH(dtype, ([&] {
-             View3<T> f = make_view<T>(field, st);
-             const T v = T(value);
-             return launch_box(0, 0, 0, nz, ny, nx,
-                               [=] __device__(int64_t z, int64_t y, int64_t x) { f(z, y, x) = v; },
-                               as_stream(stream));
-           }()));
+  DISPATCH(dtype, set_impl<T>(1, &field, st, nz, ny, nx, Three<T>{{T(value), T(0), T(0)}}, as_stream(stream)));
+}
+
+int sopht_set_fixed_val_vector_3d(int dtype, void* const field[3], const int64_t* st, int64_t nz, int64_t ny,
+                                  int64_t nx, const double* values, void* stream) {
+  REQUIRE_GRID(nz, ny, nx);
+  SOPHT_REQUIRE(values != nullptr, "three values required");
+  DISPATCH(dtype, set_impl<T>(3, field, st, nz, ny, nx, Three<T>{{T(values[0]), T(values[1]), T(values[2])}},
+                              as_stream(stream)));
 }
 
 int sopht_add_fixed_val_3d(int dtype, void* sum, const int64_t* ss, const void* field,
                            const int64_t* fs, int64_t nz, int64_t ny, int64_t nx, double value,
                            void* stream) {
   REQUIRE_GRID(nz, ny, nx);
-  DISPATCH(dtype, ([&] {
-             View3<T> o = make_view<T>(sum, ss), f = make_view<T>(field, fs);
-             const T v = T(value);
-             return launch_box(
-                 0, 0, 0, nz, ny, nx,
-                 [=] __device__(int64_t z, int64_t y, int64_t x) { o(z, y, x) = f(z, y, x) + v; },
-                 as_stream(stream));
-           }()));
+  DISPATCH(dtype, add_fixed_impl<T>(1, &sum, ss, &field, fs, nz, ny, nx, Three<T>{{T(value), T(0), T(0)}},
+                                    as_stream(stream)));
+}
+
+int sopht_add_fixed_val_vector_3d(int dtype, void* const sum[3], const int64_t* ss, const void* const field[3],
+                                  const int64_t* fs, int64_t nz, int64_t ny, int64_t nx, const double* values,
+                                  void* stream) {
+  REQUIRE_GRID(nz, ny, nx);
+  SOPHT_REQUIRE(values != nullptr, "three values required");
+  DISPATCH(dtype, add_fixed_impl<T>(3, sum, ss, field, fs, nz, ny, nx,
+                                    Three<T>{{T(values[0]), T(values[1]), T(values[2])}}, as_stream(stream)));
 }
 
 int sopht_elementwise_saxpby_3d(int dtype, void* sum, const int64_t* ss, const void* f1,
                                 const int64_t* s1, const void* f2, const int64_t* s2, int64_t nz,
                                 int64_t ny, int64_t nx, double a, double b, void* stream) {
   REQUIRE_GRID(nz, ny, nx);
-  DISPATCH(dtype, ([&] {
-             View3<T> o = make_view<T>(sum, ss), x1 = make_view<T>(f1, s1), x2 = make_view<T>(f2, s2);
-             const T ta = T(a), tb = T(b);
-             return launch_box(
-                 0, 0, 0, nz, ny, nx,
-                 [=] __device__(int64_t z, int64_t y, int64_t x) {
-                   o(z, y, x) = ta * x1(z, y, x) + tb * x2(z, y, x);
-                 },
-                 as_stream(stream));
-           }()));
+  DISPATCH(dtype, axpby_impl<T>(1, &sum, ss, &f1, s1, &f2, s2, nz, ny, nx, T(a), T(b), as_stream(stream)));
+}
+
+int sopht_elementwise_saxpby_vector_3d(int dtype, void* const sum[3], const int64_t* ss, const void* const f1[3],
+                                       const int64_t* s1, const void* const f2[3], const int64_t* s2, int64_t nz,
+                                       int64_t ny, int64_t nx, double a, double b, void* stream) {
+  REQUIRE_GRID(nz, ny, nx);
+  DISPATCH(dtype, axpby_impl<T>(3, sum, ss, f1, s1, f2, s2, nz, ny, nx, T(a), T(b), as_stream(stream)));
 }
 
 int sopht_elementwise_sum_3d(int dtype, void* sum, const int64_t* ss, const void* f1,
                              const int64_t* s1, const void* f2, const int64_t* s2, int64_t nz,
                              int64_t ny, int64_t nx, void* stream) {
   REQUIRE_GRID(nz, ny, nx);
-  DISPATCH(dtype, ([&] {
-             View3<T> o = make_view<T>(sum, ss), x1 = make_view<T>(f1, s1), x2 = make_view<T>(f2, s2);
-             return launch_box(
-                 0, 0, 0, nz, ny, nx,
-                 [=] __device__(int64_t z, int64_t y, int64_t x) {
-                   o(z, y, x) = x1(z, y, x) + x2(z, y, x);
-                 },
-                 as_stream(stream));
-           }()));
+  DISPATCH(dtype, axpby_impl<T>(1, &sum, ss, &f1, s1, &f2, s2, nz, ny, nx, T(1), T(1), as_stream(stream)));
 }
 
 int sopht_elementwise_copy_3d(int dtype, void* field, const int64_t* st, const void* rhs,
                               const int64_t* rs, int64_t nz, int64_t ny, int64_t nx,
                               void* stream) {
   REQUIRE_GRID(nz, ny, nx);
-  DISPATCH(dtype, ([&] {
-             View3<T> o = make_view<T>(field, st), r = make_view<T>(rhs, rs);
-             return launch_box(
-                 0, 0, 0, nz, ny, nx,
-                 [=] __device__(int64_t z, int64_t y, int64_t x) { o(z, y, x) = r(z, y, x); },
-                 as_stream(stream));
-           }()));
+  DISPATCH(dtype, copy_impl<T>(field, st, rhs, rs, nz, ny, nx, as_stream(stream)));
 }
 
 int sopht_set_fixed_val_at_boundaries_3d(int dtype, void* field, const int64_t* st, int64_t nz,

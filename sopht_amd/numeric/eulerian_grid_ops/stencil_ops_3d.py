@@ -148,6 +148,13 @@ def gen_diffusion_flux_pyst_kernel_3d(
     def vector_field_diffusion_flux_pyst_kernel_3d(
         vector_field_diffusion_flux, vector_field, prefactor: float
     ) -> None:
+        if L.is_vector(vector_field_diffusion_flux, vector_field):
+            nz, ny, nx = _shape3(vector_field)
+            L.call("sopht_diffusion_flux_vector_3d", tag, L.comps(vector_field_diffusion_flux),
+                   L.strides3(vector_field_diffusion_flux), L.comps(vector_field), L.strides3(vector_field),
+                   nz, ny, nx, float(prefactor), reset, L.stream_ptr())
+            L.written(vector_field_diffusion_flux)
+            return
         for i in range(3):
             diffusion_flux_pyst_kernel_3d(vector_field_diffusion_flux[i], vector_field[i], prefactor)
 
@@ -180,6 +187,13 @@ def gen_diffusion_timestep_euler_forward_pyst_kernel_3d(
     def vector_field_diffusion_timestep_euler_forward_pyst_kernel_3d(
         vector_field, diffusion_flux, nu_dt_by_dx2: float
     ) -> None:
+        if L.is_vector(vector_field):
+            nz, ny, nx = _shape3(vector_field)
+            L.call("sopht_diffusion_timestep_euler_forward_vector_3d", tag, L.comps(vector_field),
+                   L.strides3(vector_field), L.ptr(diffusion_flux), L.strides3(diffusion_flux), nz, ny, nx,
+                   float(nu_dt_by_dx2), L.stream_ptr())
+            L.written(vector_field, diffusion_flux)
+            return
         for i in range(3):
             diffusion_timestep_euler_forward_pyst_kernel_3d(vector_field[i], diffusion_flux, nu_dt_by_dx2)
 
@@ -245,7 +259,7 @@ def gen_penalise_field_boundary_pyst_kernel_3d(
 
     ctab = (C.c_double * len(tables))(*tables)
 
-    def penalise_field_boundary_pyst_kernel_3d(field) -> None:
+    def penalise(entry, fields, field) -> None:
         nz, ny, nx = _shape3(field)
         if width == 1:
             # the reference's back-slab source ``field[..., -1:0]`` is empty for width 1, and
@@ -253,16 +267,19 @@ def gen_penalise_field_boundary_pyst_kernel_3d(
             msg = (f"could not broadcast input array from shape ({nz},{ny},0) "
                    f"into shape ({nz},{ny},1)")
             raise ValueError(msg)
-        L.call(
-            "sopht_penalise_field_boundary_3d", tag, L.ptr(field), L.strides3(field), nz, ny, nx,
-            width, ctab, L.stream_ptr(),
-        )
+        L.call(entry, tag, fields, L.strides3(field), nz, ny, nx, width, ctab, L.stream_ptr())
         L.written(field)
+
+    def penalise_field_boundary_pyst_kernel_3d(field) -> None:
+        penalise("sopht_penalise_field_boundary_3d", L.ptr(field), field)
 
     if field_type == "scalar":
         return penalise_field_boundary_pyst_kernel_3d
 
     def penalise_vector_field_boundary_pyst_kernel_3d(vector_field) -> None:
+        if L.is_vector(vector_field):
+            penalise("sopht_penalise_field_boundary_vector_3d", L.comps(vector_field), vector_field)
+            return
         for i in range(3):
             penalise_field_boundary_pyst_kernel_3d(vector_field[i])
 
@@ -270,6 +287,13 @@ def gen_penalise_field_boundary_pyst_kernel_3d(
 
 
 # ------------------------------------------------------------------------------ elementwise
+
+
+def _saxpby_vector(tag, s, f1, f2, a, b):
+    nz, ny, nx = _shape3(s)
+    L.call("sopht_elementwise_saxpby_vector_3d", tag, L.comps(s), L.strides3(s), L.comps(f1), L.strides3(f1),
+           L.comps(f2), L.strides3(f2), nz, ny, nx, float(a), float(b), L.stream_ptr())
+    L.written(s)
 
 
 def gen_elementwise_sum_pyst_kernel_3d(
@@ -291,7 +315,9 @@ def gen_elementwise_sum_pyst_kernel_3d(
         L.written(sum_field)
 
     def elementwise_sum_pyst_kernel_3d(sum_field, field_1, field_2) -> None:
-        if field_type == "vector":
+        if field_type == "vector" and L.is_vector(sum_field, field_1, field_2):
+            _saxpby_vector(tag, sum_field, field_1, field_2, 1.0, 1.0)
+        elif field_type == "vector":
             for i in range(3):
                 _sum(sum_field[i], field_1[i], field_2[i])
         else:
@@ -320,6 +346,12 @@ def gen_set_fixed_val_pyst_kernel_3d(
         return set_fixed_val_pyst_kernel_3d
 
     def vector_field_set_fixed_val_pyst_kernel_3d(vector_field, fixed_vals) -> None:
+        if L.is_vector(vector_field):
+            nz, ny, nx = _shape3(vector_field)
+            L.call("sopht_set_fixed_val_vector_3d", tag, L.comps(vector_field), L.strides3(vector_field), nz, ny, nx,
+                   L.three_values(fixed_vals), L.stream_ptr())
+            L.written(vector_field)
+            return
         for i in range(3):
             set_fixed_val_pyst_kernel_3d(vector_field[i], fixed_vals[i])
 
@@ -410,6 +442,13 @@ def gen_add_fixed_val_pyst_kernel_3d(
         return add_fixed_val_pyst_kernel_3d
 
     def vector_field_add_fixed_val_pyst_kernel_3d(sum_field, vector_field, fixed_vals) -> None:
+        if L.is_vector(sum_field, vector_field):
+            nz, ny, nx = _shape3(vector_field)
+            L.call("sopht_add_fixed_val_vector_3d", tag, L.comps(sum_field), L.strides3(sum_field),
+                   L.comps(vector_field), L.strides3(vector_field), nz, ny, nx, L.three_values(fixed_vals),
+                   L.stream_ptr())
+            L.written(sum_field)
+            return
         for i in range(3):
             add_fixed_val_pyst_kernel_3d(sum_field[i], vector_field[i], float(fixed_vals[i]))
 
@@ -433,7 +472,9 @@ def gen_elementwise_saxpby_pyst_kernel_3d(
         L.written(s)
 
     def elementwise_saxpby_pyst_kernel_3d(sum_field, field_1, field_2, field_1_prefac, field_2_prefac) -> None:
-        if field_type == "vector":
+        if field_type == "vector" and L.is_vector(sum_field, field_1, field_2):
+            _saxpby_vector(tag, sum_field, field_1, field_2, field_1_prefac, field_2_prefac)
+        elif field_type == "vector":
             for i in range(3):
                 _saxpby(sum_field[i], field_1[i], field_2[i], field_1_prefac, field_2_prefac)
         else:
@@ -580,7 +621,13 @@ def gen_advection_timestep_euler_forward_conservative_eno3_pyst_kernel_3d(
     def vector_field_advection_timestep_euler_forward_conservative_eno3_pyst_kernel_3d(
         vector_field, advection_flux, velocity, dt_by_dx: float
     ) -> None:
-        step(3, L.comps(vector_field), vector_field, advection_flux, velocity, dt_by_dx)
+        if L.is_vector(vector_field):
+            step(3, L.comps(vector_field), vector_field, advection_flux, velocity, dt_by_dx)
+            return
+        for i in range(3):
+            advection_timestep_euler_forward_conservative_eno3_pyst_kernel_3d(
+                vector_field[i], advection_flux, velocity, dt_by_dx
+            )
 
     return vector_field_advection_timestep_euler_forward_conservative_eno3_pyst_kernel_3d
 

@@ -149,3 +149,78 @@ def test_eno3_adjoint(dev, real_t, shape):
     flux.backward(to_dev(a, dev))
     np.testing.assert_allclose(to_host(fd.grad), fr, atol=bound, rtol=0)
     np.testing.assert_allclose(to_host(ud.grad), ur, atol=bound, rtol=0)
+
+
+@pytest.mark.parametrize("reset", [True, False])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_curl_laplacian_divergence(dev, real_t, shape, reset):
+    rng = np.random.default_rng(15)
+    f = rng.uniform(-1, 1, (3, *shape)).astype(real_t)
+    f64 = f.astype(np.float64)
+    p = real_t(0.25)
+    eps = float(np.finfo(real_t).eps)
+    start = np.full_like(f, 0.5)
+    ref = start.astype(np.float64)
+    S.curl(ref, f64, 0.25, reset_ghost_zone=reset)
+    curl = spne().gen_curl_pyst_kernel_3d(real_t, reset_ghost_zone=reset)
+    both(lambda o, i: curl(o[0], i[0], p), [start], [f], dev, [ref], 2 * 4 * eps * 4)
+    ref = start.astype(np.float64)
+    S.update_vorticity_from_velocity_forcing(ref, f64, 0.25)
+    update = spne().gen_update_vorticity_from_velocity_forcing_pyst_kernel_3d(real_t)
+    both(lambda o, i: update(o[0], i[0], p), [start], [f], dev, [ref], 2 * 5 * eps * 4)
+    ref = start.astype(np.float64)
+    for c in range(3):
+        S.diffusion_flux(ref[c], f64[c], 0.25, reset_ghost_zone=reset)
+    flux = spne().gen_diffusion_flux_pyst_kernel_3d(real_t, field_type="vector", reset_ghost_zone=reset)
+    both(lambda o, i: flux(o[0], i[0], p), [start], [f], dev, [ref], 2 * 8 * eps * 12)
+    scalar = spne().gen_diffusion_flux_pyst_kernel_3d(real_t, reset_ghost_zone=reset)
+    both(lambda o, i: scalar(o[0], i[0], p), [start[0]], [f[0]], dev, [ref[0]], 2 * 8 * eps * 12)
+    ref = start[0].astype(np.float64)
+    S.divergence(ref, f64, 0.25, reset_ghost_zone=reset)
+    div = spne().gen_divergence_pyst_kernel_3d(real_t, reset_ghost_zone=reset)
+    both(lambda o, i: div(o[0], i[0], p), [start[0]], [f], dev, [ref], 2 * 6 * eps * 6)
+
+
+@pytest.mark.parametrize("shape", SHAPES + [(1, 1, 3), (2, 5, 9)])
+def test_vector_forms_of_scalar_operators(dev, real_t, shape):
+    rng = np.random.default_rng(16)
+    a, b = (rng.uniform(-1, 1, (3, *shape)).astype(real_t) for _ in range(2))
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    eps = float(np.finfo(real_t).eps)
+    one = np.ones_like(a)
+    add = spne().gen_add_fixed_val_pyst_kernel_3d(real_t, field_type="vector")
+    vals = (0.5, -0.25, 2.0)
+    col = np.array(vals).reshape(3, 1, 1, 1)
+    both(lambda o, i: add(o[0], i[0], vals), [one], [a], dev, [a64 + col], 2 * eps * 3)
+    fix = spne().gen_set_fixed_val_pyst_kernel_3d(real_t, field_type="vector")
+    both(lambda o, i: fix(o[0], vals), [one], [], dev, [one * col], 0.0)
+    total = spne().gen_elementwise_sum_pyst_kernel_3d(real_t, field_type="vector")
+    both(lambda o, i: total(o[0], o[0], i[0]), [a], [b], dev, [a64 + b64], 2 * eps * 2)
+    saxpby = spne().gen_elementwise_saxpby_pyst_kernel_3d(real_t, field_type="vector")
+    both(lambda o, i: saxpby(o[0], i[0], i[1], 0.75, 0.25), [one], [a, b], dev, [0.75 * a64 + 0.25 * b64], 2 * 3 * eps)
+    cross = spne().gen_elementwise_cross_product_pyst_kernel_3d(real_t)
+    both(lambda o, i: cross(o[0], i[0], i[1]), [one], [a, b], dev, [np.cross(a64, b64, axis=0)], 2 * 3 * eps * 2)
+    step = spne().gen_diffusion_timestep_euler_forward_pyst_kernel_3d(real_t, field_type="vector")
+    refs, flux = a64.copy(), np.zeros(shape)
+    for c in range(3):
+        S.diffusion_timestep_euler_forward(refs[c], flux, 0.125)
+    both(lambda o, i: step(o[0], o[1], real_t(0.125)), [a, one[0]], [], dev, [refs, flux], 2 * 9 * eps * 12)
+    # three tensors instead of one
+    parts = [to_dev(a[c], dev) for c in range(3)]
+    step(parts, to_dev(one[0], dev), real_t(0.125))
+    for c in range(3):
+        np.testing.assert_allclose(to_host(parts[c]), refs[c], atol=2 * 9 * eps * 12, rtol=0)
+
+
+@pytest.mark.parametrize("width,shape", [(2, (4, 4, 4)), (2, (5, 9, 37)), (4, (8, 12, 9))])
+def test_penalised_vector_equals_its_components(dev, real_t, width, shape):
+    rng = np.random.default_rng(17)
+    a = rng.uniform(-1, 1, (3, *shape)).astype(real_t)
+    grid = np.meshgrid(*[(np.arange(n) + 0.5) * 0.1 for n in shape], indexing="ij")
+    args = (width, 0.1, grid[2], grid[1], grid[0], real_t)
+    whole, parts = to_dev(a, dev), to_dev(a, dev)
+    spne().gen_penalise_field_boundary_pyst_kernel_3d(*args, field_type="vector")(whole)
+    one = spne().gen_penalise_field_boundary_pyst_kernel_3d(*args)
+    for c in range(3):
+        one(parts[c])
+    np.testing.assert_array_equal(to_host(whole), to_host(parts))

@@ -85,7 +85,7 @@ int step_impl(sopht_ns3d* P, const void* vort_in, void* vort_out, const void* ve
   const bool s1v = P->s1_vec != 0;
   const int s1_rows = s1v ? P->s1_rows : S1Tile<T>::TY;
   const int s1_cols = s1v ? P->s1_cols : S1Tile<T>::TX;
-  const int s1_chunk = s1v ? P->s1_chunk : kS1Chunk;
+  const int s1_chunk = P->s1_chunk;
   const S1Map s1m{int(ceil_div(g.nx, s1_cols)), int(ceil_div(g.ny, s1_rows)), s1_rows, s1_chunk, s1_cols};
   const int64_t s1_items = int64_t(s1m.tiles_x) * s1m.tiles_y * ceil_div(g.nz, s1_chunk);
   const bool flags_ok = s1_items <= P->s1flags_cap;
@@ -105,7 +105,7 @@ int step_impl(sopht_ns3d* P, const void* vort_in, void* vort_out, const void* ve
                                                             s1m.tiles_x, s1m.tiles_y, remap,
                                                             static_cast<T*>(vort1_out), fflags);
     else if (!s1v)
-      k_s1<T><<<unsigned(s1_items), S1Tile<T>::NT, 0, s>>>(g, w_in, u_in, F, ps, pF, pB, wf, kS1Chunk,
+      k_s1<T><<<unsigned(s1_items), S1Tile<T>::NT, 0, s>>>(g, w_in, u_in, F, ps, pF, pB, wf, s1_chunk,
                                                           s1m.tiles_x, s1m.tiles_y, remap,
                                                           static_cast<T*>(vort1_out), fflags);
     SOPHT_CHECK_LAUNCH();
@@ -256,15 +256,25 @@ int sopht_ns3d_create_with_poisson_solver(int dtype, int64_t nz, int64_t ny, int
   P->filter_type = 0;
   {
     // The vector sweep needs whole 16-byte row vectors and component byte offsets below 2^32.
-    // Its work items hold the most planes (64, 32 or 16) that still make 384 items, one round
-    // of workgroups at one and a half to three per CU. Measured S1 times: 256^3 FP32 (128 x 8
-    // tiles) 0.21 ms at 32 planes against 0.24 at 16 (two chunks per XCD resident at once
-    // doubled the L2 misses) and 0.29 at 64; 256^3 FP64 0.38 ms at 64 against 0.43 at 32;
-    // 192^3 FP64 0.19 ms at 32 against 0.22 at 16; 192^3 FP32 0.11 ms at 16 against 0.16 at
-    // 32. Grids with fewer than 256 items of 16 planes keep the scalar sweep (twice the
-    // workgroups). The environment can force either: SOPHT_S1_SCALAR=1 (the two sweeps give
-    // the same bits) and SOPHT_S1_CHUNK=16/32/64. FP32 rows that are a multiple of 128 cells take tiles of 128
-    // cells by 8 rows, others 64 by 16 (FP64: 64 by 8); SOPHT_S1_COLS=64/128 forces the width.
+    // Its work items hold the most planes (64 down to 2) that still make 400 items, one round
+    // of workgroups at one and a half to three per CU; an item recomputes two planes of B, so
+    // fewer planes cost work, but fewer items leave CUs idle. Measured S1 times (items):
+    //   256^3 FP32 (128 x 8 tiles)  32 planes 0.21 ms (512), 16 planes 0.24 (1024: two chunks
+    //                               per XCD resident at once double the L2 misses)
+    //   192^3 FP64                  32 planes 0.190 ms (432), 16 planes 0.216
+    //   192^3 FP32                  16 planes 0.112 ms (432), 8 planes 0.123
+    //   192 x 128 x 256 FP32        16 planes 0.102 ms (384), 8 planes 0.084 (768)
+    //   96 x 128 x 256 FP32         16 planes 0.079 ms (192), 8 planes 0.057 (384), 4 0.050 (768)
+    //   128^3 FP32                  16 planes 0.068 ms (128), 8 planes 0.041, 4 planes 0.031 (512)
+    //   96^3 FP64                   16 planes 0.064 ms (144), 8 planes 0.043, 4 planes 0.035 (576)
+    // Grids with fewer than 400 items of 2 planes, and rows that are no multiple of 16 bytes,
+    // take the scalar sweep (twice the workgroups per plane), with the most planes (16 down to
+    // 2) that make 512 items: 64^3 FP32 16 planes 0.044 ms, 2 planes 0.013 (vector 0.018);
+    // 64^3 FP64 0.051 and 0.018; 128^3 FP32 (forced) 16 planes 0.048, 8 planes 0.034, 4 0.042.
+    // The environment can force either: SOPHT_S1_SCALAR=1 (16 planes; all choices give the
+    // same bits) and SOPHT_S1_CHUNK=2..64 (a power of two). FP32 rows that are a multiple of
+    // 128 cells take tiles of 128 cells by 8 rows, others 64 by 16 (FP64: 64 by 8);
+    // SOPHT_S1_COLS=64/128 forces the width.
     const int64_t vec = 16 / (dtype == SOPHT_F32 ? 4 : 8);
     const int64_t bytes = nz * ny * nx * (dtype == SOPHT_F32 ? 4 : 8);
     P->s1_cols = dtype == SOPHT_F32 && nx % 128 == 0 ? 128 : 64;
@@ -277,26 +287,26 @@ int sopht_ns3d_create_with_poisson_solver(int dtype, int64_t nz, int64_t ny, int
     const int64_t tiles = ceil_div(nx, P->s1_cols) * ceil_div(ny, P->s1_rows);
     const char* scalar = std::getenv("SOPHT_S1_SCALAR");
     const char* chunk = std::getenv("SOPHT_S1_CHUNK");
-    P->s1_chunk = 16;
-    for (const int c : {64, 32})
-      if (tiles * ceil_div(nz, int64_t(c)) >= 384) {
-        P->s1_chunk = c;
-        break;
-      }
-    bool fill = tiles * ceil_div(nz, 16) >= 256;
+    P->s1_chunk = 64;
+    while (P->s1_chunk > 2 && tiles * ceil_div(nz, int64_t(P->s1_chunk)) < 400) P->s1_chunk /= 2;
+    bool fill = tiles * ceil_div(nz, int64_t(P->s1_chunk)) >= 400;
     if (chunk) {
       const int v = std::atoi(chunk);
-      if (v == 16 || v == 32 || v == 64) {
+      if (v >= 2 && v <= 64 && (v & (v - 1)) == 0) {
         P->s1_chunk = v;
         fill = true;
       }
     }
-    P->s1_vec = nx % vec == 0 && bytes < (int64_t(1) << 32) && fill && !(scalar && std::atoi(scalar) == 1);
-  }
-  {
-    const int64_t i32 = ceil_div(nx, S1Tile<float>::TX) * ceil_div(ny, S1Tile<float>::TY) * ceil_div(nz, kS1Chunk);
-    const int64_t i64 = ceil_div(nx, S1Tile<double>::TX) * ceil_div(ny, S1Tile<double>::TY) * ceil_div(nz, kS1Chunk);
-    P->s1flags_cap = dtype == SOPHT_F32 ? i32 : i64;
+    const bool forced = scalar && std::atoi(scalar) == 1;
+    P->s1_vec = nx % vec == 0 && bytes < (int64_t(1) << 32) && fill && !forced;
+    int64_t used = tiles;  // S1 tiles of a chunk of planes
+    if (!P->s1_vec) {
+      const int64_t ty = dtype == SOPHT_F32 ? S1Tile<float>::TY : S1Tile<double>::TY;
+      used = ceil_div(nx, S1Tile<float>::TX) * ceil_div(ny, ty);
+      P->s1_chunk = kS1Chunk;
+      while (!forced && P->s1_chunk > 2 && used * ceil_div(nz, int64_t(P->s1_chunk)) < 512) P->s1_chunk /= 2;
+    }
+    P->s1flags_cap = used * ceil_div(nz, int64_t(P->s1_chunk));
   }
   if (hipMalloc(&P->partial, P->partial_cap * 8) != hipSuccess ||
       hipMalloc(&P->s2max, P->s2max_cap * 8) != hipSuccess ||
@@ -346,7 +356,7 @@ int sopht_ns3d_poisson_schedule(const sopht_ns3d* P, int* passes, int* zpass_job
 int sopht_ns3d_s1_schedule(const sopht_ns3d* P, int* vector, int* zchunk, int* cols) {
   SOPHT_REQUIRE(P != nullptr, "plan is null");
   if (vector) *vector = P->s1_vec;
-  if (zchunk) *zchunk = P->s1_vec ? P->s1_chunk : sopht::kS1Chunk;
+  if (zchunk) *zchunk = P->s1_chunk;
   if (cols) *cols = P->s1_vec ? P->s1_cols : sopht::S1Tile<float>::TX;
   return SOPHT_OK;
 }

@@ -19,12 +19,13 @@ struct Grid {
   }
 };
 
-// z planes per S1 work item (two extra planes of B are recomputed per item)
+// z planes per S1 work item of the batched step and the scalar sweep's most (two extra planes
+// of B are recomputed per item)
 constexpr int kS1Chunk = 16;
 
 // S1: omega2 = omega1 + pB curl_h(u x omega1), omega1 = omega + pF curl_h(F), with neither
 // omega1 nor B stored in HBM. A workgroup owns a TX x TY tile of (x, y) columns over a chunk
-// of kS1Chunk planes and marches up z. Iteration i
+// of planes and marches up z. Iteration i
 //   (1) produces omega1 and B on plane i over the tile plus its 1-cell edge ring (without
 //       corners); curl_h(F) reads F's neighbours through the caches; B goes to a 3-plane LDS
 //       ring, the tile's own omega1(i), B(i), B(i-1) stay in registers;
@@ -655,9 +656,11 @@ __device__ __forceinline__ void sc_body(Grid g, const T* __restrict__ w2, T* __r
   using V = VecT<T, VEC>;
   const MarchTile m = march_tile<VEC>(g, tiles_x, tiles_y, item, chunk);
   if (zero_forcing && fflags && m.x0 < int(g.nx) && m.y < int(g.ny)) {
-    // the S1 tile holding these cells saw no bit of F set: F is zero there already
-    const int t = ((m.z0 / s1.chunk) * s1.tiles_y + m.y / s1.rows) * s1.tiles_x + m.x0 / s1.cols;
-    if (fflags[t] == 0) zero_forcing = 0;
+    // the S1 tiles holding these cells saw no bit of F set: F is zero there already
+    int any = 0;
+    for (int q = m.z0 / s1.chunk; q <= (m.z1 - 1) / s1.chunk; ++q)
+      any |= fflags[(q * s1.tiles_y + m.y / s1.rows) * s1.tiles_x + m.x0 / s1.cols];
+    if (any == 0) zero_forcing = 0;
   }
   const int nz = int(g.nz), ny = int(g.ny), nx = int(g.nx);
   const int n = nz * ny * nx, sz = ny * nx, sy = nx;

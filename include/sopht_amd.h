@@ -155,7 +155,7 @@ int sopht_elementwise_complex_product_3d(int dtype, void* product, const int64_t
  * sopht/simulator/flow/passive_transport_flow_simulators.py:100-113 (3D): the conservative
  * ENO3 advection step (advection_timestep_3d.py:12-99, inv_dx = -dt_by_dx) followed by the
  * Euler diffusion step (diffusion_timestep_3d.py:12-80, prefactor nu_dt_by_dx2) of ncomp
- * (1 or 3) contiguous (nz, ny, nx) component fields, in place, in one fused sweep; scratch
+ * (1 or 3) contiguous (nz, ny, nx) component fields, in place, in two sweeps; scratch
  * holds ncomp fields of the same shape (contents undefined on return). velocity: three
  * contiguous components. */
 int sopht_passive_transport_step_3d(int dtype, int ncomp, void* const field[3], void* const scratch[3],

@@ -20,6 +20,33 @@
 namespace sopht {
 namespace {
 
+// Visit every cell of the box [z0, z0+bz) x [y0, y0+by) x [x0, x0+bx).
+template <typename Fn>
+__global__ void __launch_bounds__(256) box_kernel(int64_t z0, int64_t y0, int64_t x0, int64_t bz,
+                                                  int64_t by, int64_t bx, Fn fn) {
+  const int64_t total = bz * by * bx;
+  for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < total;
+       i += int64_t(gridDim.x) * blockDim.x) {
+    const int64_t x = i % bx;
+    const int64_t t = i / bx;
+    const int64_t y = t % by;
+    const int64_t z = t / by;
+    fn(z0 + z, y0 + y, x0 + x);
+  }
+}
+
+template <typename Fn>
+int launch_box(int64_t z0, int64_t y0, int64_t x0, int64_t bz, int64_t by, int64_t bx, Fn fn,
+               hipStream_t s) {
+  const int64_t total = bz * by * bx;
+  if (total <= 0) return SOPHT_OK;
+  int blocks = ceil_div(total, 256);
+  if (blocks > 65536) blocks = 65536;
+  box_kernel<<<blocks, 256, 0, s>>>(z0, y0, x0, bz, by, bx, fn);
+  SOPHT_CHECK_LAUNCH();
+  return SOPHT_OK;
+}
+
 constexpr int kRowThreads = 256;
 constexpr int kRowLanes = 62;  // lanes of a wavefront that own a column
 
@@ -274,109 +301,128 @@ __global__ void __launch_bounds__(kRowThreads)
 
 // ------------------------------------------------------------------ ENO3 advection flux
 
-// The flux through the face between cells 0 and 1 of one axis (advection_flux_3d.py:12-233):
-// g = field * velocity at cells -1 .. 2, u the velocity at cells 0 and 1. A cell's front face
-// is its upper neighbour's back face, with the same upwind choice and the same terms, so each
-// face is formed once.
+// The flux through the face between cells 0 and 1 of one axis (advection_flux_3d.py:12-233),
+// from the field f and the velocity u at cells -1 .. 2. A cell's front face is its upper
+// neighbour's back face, with the same upwind choice and the same terms, so each face is formed
+// once. Every product and sum rounds by itself, as the reference's.
 template <typename T>
-__device__ __forceinline__ T eno3_face(T gm, T g0, T g1, T gp, T u0, T u1) {
+__device__ __forceinline__ T eno3_face(T fm, T f0, T f1, T fp, T um, T u0, T u1, T up) {
+#pragma clang fp contract(off)
   const T c13 = T(1.0 / 3.0), c56 = T(5.0 / 6.0), c16 = T(1.0 / 6.0);
-  const bool up = u0 > -u1;
-  return c13 * (up ? g1 : g0) + c56 * (up ? g0 : g1) - c16 * (up ? gm : gp);
+  const bool left = u0 > -u1;
+  const T near = c13 * (left ? f1 : f0) * (left ? u1 : u0), here = c56 * (left ? f0 : f1) * (left ? u0 : u1);
+  return near + here - c16 * (left ? fm : fp) * (left ? um : up);
 }
 
-// ENO3 conservative advection flux on [2:-2]^3: added to the flux field, or (SET) stored with
-// zeros on the border cells, which spares the clearing and the read of the flux field.
+// What k_eno3_rows does with the flux E of [2:-2]^3.
+enum EnoMode {
+  kEnoAdd,  // out += E on [2:-2]^3
+  kEnoSet,  // out = E, 0 on the border cells: spares the clearing and the read of the flux field
+  kEnoStep  // out = field + E, the field on the border cells
+};
+
+// ENO3 conservative advection flux of one scalar field per gridDim.y.
 // A thread forms V + 1 x faces, two rows of y faces and one plane of z faces per plane of V
 // cells; its 13 16-byte loads per plane (field rows y-2..y+2, u_y rows y-2..y+2, u_x, u_z and
 // the field two planes up) come mostly from L1 and L2, and their rate bounds it.
-// 150 x 201 x 230 FP32, storing: 36 us (3.8 TB/s of 5 words per cell) against 94 us with one
+// 150 x 201 x 230 FP32, storing: 30 us (4.7 TB/s of 5 words per cell) against 94 us with one
 // cell per thread plus 7 us for the clearing.
-template <typename T, bool SET>
+template <typename T, int MODE>
 __global__ void __launch_bounds__(kRowThreads)
-    k_eno3_rows(RowGeo g, T* flux, RowStrides os, const T* f, RowStrides fs, Rows3<const T> u, T inv_dx) {
+    k_eno3_rows(RowGeo g, Rows3<T> out, Rows3<const T> field, Rows3<const T> u, T inv_dx) {
   constexpr int V = RowVec<T>::V;
   using vec = rvec<T>;
   const RowCol<T, 2> c(g);
-  const int fr = c.yl * fs.y + c.x, ur = c.yl * u.s.y + c.x, orow = c.y * os.y + c.x;
+  T* const flux = out.p[blockIdx.y];
+  const T* const f = field.p[blockIdx.y];
+  const RowStrides os = out.s, fs = field.s;
+  const int fr = c.yl * fs.y + c.x, ur = c.yl * u.s.y + c.x, orow = c.y * os.y + c.x, frow = c.y * fs.y + c.x;
   // planes with a flux: those of the chunk inside [2, nz - 2)
   const int za = c.z0 < 2 ? 2 : c.z0, zb = c.z1 < g.nz - 2 ? c.z1 : g.nz - 2;
-  if (SET) {
+  if constexpr (MODE != kEnoAdd) {
     for (int z = c.z0; z < c.z1; ++z)
-      if (z < za || z >= zb) rstore(flux + z * os.z + orow, vec{}, c.own);
+      if (z < za || z >= zb)
+        rstore(flux + z * os.z + orow, MODE == kEnoStep ? rload_own(c, g, f + z * fs.z + frow, z) : vec{}, c.own);
   }
   if (za >= zb) return;  // the same for the whole workgroup
-  // along z: the field at z, z+1; u_z at z, z+1; their products at z-1, z, z+1; the back face
+  // along z: the field and u_z at z-1, z, z+1, and the back face
+  vec fm = rload(f + (za - 1) * fs.z + fr), wm = rload(u.p[2] + (za - 1) * u.s.z + ur);
   vec f0 = rload(f + za * fs.z + fr), f1 = rload(f + (za + 1) * fs.z + fr);
   vec w0 = rload(u.p[2] + za * u.s.z + ur), w1 = rload(u.p[2] + (za + 1) * u.s.z + ur);
-  vec gm, g0 = f0 * w0, g1 = f1 * w1, back;
+  vec back;
   {
-    const vec wm = rload(u.p[2] + (za - 1) * u.s.z + ur);
-    gm = rload(f + (za - 1) * fs.z + fr) * wm;
-    const vec gmm = rload(f + (za - 2) * fs.z + fr) * rload(u.p[2] + (za - 2) * u.s.z + ur);
+    const vec fmm = rload(f + (za - 2) * fs.z + fr), wmm = rload(u.p[2] + (za - 2) * u.s.z + ur);
 #pragma unroll
-    for (int k = 0; k < V; ++k) back[k] = eno3_face<T>(gmm[k], gm[k], g0[k], g1[k], wm[k], w0[k]);
+    for (int k = 0; k < V; ++k) back[k] = eno3_face<T>(fmm[k], fm[k], f0[k], f1[k], wmm[k], wm[k], w0[k], w1[k]);
   }
   const unsigned mask = c.yin ? c.own & c.inner : 0u;
   for (int z = za; z < zb; ++z) {
+#pragma clang fp contract(off)
     const T* fz = f + z * fs.z + fr;
     const T* uxz = u.p[0] + z * u.s.z + ur;
     const T* uyz = u.p[1] + z * u.s.z + ur;
     T* oz = flux + z * os.z + orow;
     const vec f2 = rload(fz + 2 * fs.z), w2 = rload(u.p[2] + (z + 2) * u.s.z + ur);
     const vec ux = rload(uxz);
-    vec uy[5], gy[5];
+    vec uy[5], fy[5];
 #pragma unroll
-    for (int r = 0; r < 5; ++r) uy[r] = rload(uyz + (r - 2) * u.s.y);
-#pragma unroll
-    for (int r = 0; r < 5; ++r) gy[r] = (r == 2 ? f0 : rload(fz + (r - 2) * fs.y)) * uy[r];
+    for (int r = 0; r < 5; ++r) {
+      uy[r] = rload(uyz + (r - 2) * u.s.y);
+      fy[r] = r == 2 ? f0 : rload(fz + (r - 2) * fs.y);
+    }
     vec acc = {};
-    if (!SET) acc = rload_own(c, g, static_cast<const T*>(oz), z);
+    if constexpr (MODE == kEnoAdd) acc = rload_own(c, g, static_cast<const T*>(oz), z);
     {  // x faces -1/2 .. V - 1/2 of the vector
-      const vec gx = f0 * ux;
-      T e[V + 4], v[V + 2];  // products at cells -2 .. V + 1, velocities at -1 .. V
-      e[0] = from_prev_lane(gx[V - 2]);
-      e[1] = from_prev_lane(gx[V - 1]);
-      e[V + 2] = from_next_lane(gx[0]);
-      e[V + 3] = from_next_lane(gx[1]);
-      v[0] = from_prev_lane(ux[V - 1]);
-      v[V + 1] = from_next_lane(ux[0]);
+      T e[V + 4], v[V + 4];  // field and velocity at cells -2 .. V + 1
+      e[0] = from_prev_lane(f0[V - 2]);
+      e[1] = from_prev_lane(f0[V - 1]);
+      e[V + 2] = from_next_lane(f0[0]);
+      e[V + 3] = from_next_lane(f0[1]);
+      v[0] = from_prev_lane(ux[V - 2]);
+      v[1] = from_prev_lane(ux[V - 1]);
+      v[V + 2] = from_next_lane(ux[0]);
+      v[V + 3] = from_next_lane(ux[1]);
 #pragma unroll
       for (int k = 0; k < V; ++k) {
-        e[k + 2] = gx[k];
-        v[k + 1] = ux[k];
+        e[k + 2] = f0[k];
+        v[k + 2] = ux[k];
       }
       T face[V + 1];
 #pragma unroll
-      for (int k = 0; k <= V; ++k) face[k] = eno3_face<T>(e[k], e[k + 1], e[k + 2], e[k + 3], v[k], v[k + 1]);
+      for (int k = 0; k <= V; ++k)
+        face[k] = eno3_face<T>(e[k], e[k + 1], e[k + 2], e[k + 3], v[k], v[k + 1], v[k + 2], v[k + 3]);
 #pragma unroll
       for (int k = 0; k < V; ++k) {
         acc[k] = acc[k] + inv_dx * face[k + 1];
         acc[k] = acc[k] - inv_dx * face[k];
       }
     }
-    const vec g2 = f2 * w2;
 #pragma unroll
     for (int k = 0; k < V; ++k) {
-      acc[k] = acc[k] + inv_dx * eno3_face<T>(gy[1][k], gy[2][k], gy[3][k], gy[4][k], uy[2][k], uy[3][k]);
-      acc[k] = acc[k] - inv_dx * eno3_face<T>(gy[0][k], gy[1][k], gy[2][k], gy[3][k], uy[1][k], uy[2][k]);
-      const T front = eno3_face<T>(gm[k], g0[k], g1[k], g2[k], w0[k], w1[k]);
+      acc[k] = acc[k] + inv_dx * eno3_face<T>(fy[1][k], fy[2][k], fy[3][k], fy[4][k], uy[1][k], uy[2][k], uy[3][k], uy[4][k]);
+      acc[k] = acc[k] - inv_dx * eno3_face<T>(fy[0][k], fy[1][k], fy[2][k], fy[3][k], uy[0][k], uy[1][k], uy[2][k], uy[3][k]);
+      const T front = eno3_face<T>(fm[k], f0[k], f1[k], f2[k], wm[k], w0[k], w1[k], w2[k]);
       acc[k] = acc[k] + inv_dx * front;
       acc[k] = acc[k] - inv_dx * back[k];
       back[k] = front;
     }
-    if (SET) {
-#pragma unroll
-      for (int k = 0; k < V; ++k) acc[k] = mask >> k & 1u ? acc[k] : T(0);
-      rstore(oz, acc, c.own);
-    } else {
+    if constexpr (MODE == kEnoAdd) {
       rstore(oz, acc, mask);
+    } else {
+      vec rest = {};
+      if constexpr (MODE == kEnoStep) {
+        rest = f0;
+        if (!c.yin) rest = rload_own(c, g, f + z * fs.z + frow, z);
+        acc = rest + acc;
+      }
+#pragma unroll
+      for (int k = 0; k < V; ++k) acc[k] = mask >> k & 1u ? acc[k] : rest[k];
+      rstore(oz, acc, c.own);
     }
-    gm = g0;
-    g0 = g1;
-    g1 = g2;
+    fm = f0;
     f0 = f1;
     f1 = f2;
+    wm = w0;
     w0 = w1;
     w1 = w2;
   }
@@ -507,7 +553,8 @@ __global__ void __launch_bounds__(kRowThreads)
 enum RowMode {
   kRowInside,  // store the inside cells, leave the border
   kRowReset,   // store the inside cells and zeros on the border
-  kRowAdd      // add to the inside cells
+  kRowAdd,     // add to the inside cells
+  kRowStep     // (Laplacian) store the operand plus the result, the operand on the border
 };
 
 template <typename T, int MODE>
@@ -599,7 +646,16 @@ __global__ void __launch_bounds__(kRowThreads) k_laplacian_rows(RowGeo g, Rows3<
       }
     }
     const unsigned inside = plane && c.yin ? c.own & c.inner : 0u;
-    row_out<T, MODE>(c, g, out + z * o.s.z + orow, r, inside, z);
+    if constexpr (MODE == kRowStep) {
+#pragma clang fp contract(off)
+      vec v = fc;
+      if (!c.yin) v = rload_own(c, g, f + z * in.s.z + c.y * in.s.y + c.x, z);
+#pragma unroll
+      for (int k = 0; k < V; ++k) v[k] = inside >> k & 1u ? v[k] + r[k] : v[k];
+      rstore(out + z * o.s.z + orow, v, c.own);
+    } else {
+      row_out<T, MODE>(c, g, out + z * o.s.z + orow, r, inside, z);
+    }
     fm = fc;
     fc = fp;
   }

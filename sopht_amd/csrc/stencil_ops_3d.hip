@@ -23,33 +23,6 @@ void set_last_error(const char* msg, const char* file, int line) {
 
 namespace {
 
-// Visit every cell of the box [z0, z0+bz) x [y0, y0+by) x [x0, x0+bx).
-template <typename Fn>
-__global__ void __launch_bounds__(256) box_kernel(int64_t z0, int64_t y0, int64_t x0, int64_t bz,
-                                                  int64_t by, int64_t bx, Fn fn) {
-  const int64_t total = bz * by * bx;
-  for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < total;
-       i += int64_t(gridDim.x) * blockDim.x) {
-    const int64_t x = i % bx;
-    const int64_t t = i / bx;
-    const int64_t y = t % by;
-    const int64_t z = t / by;
-    fn(z0 + z, y0 + y, x0 + x);
-  }
-}
-
-template <typename Fn>
-int launch_box(int64_t z0, int64_t y0, int64_t x0, int64_t bz, int64_t by, int64_t bx, Fn fn,
-               hipStream_t s) {
-  const int64_t total = bz * by * bx;
-  if (total <= 0) return SOPHT_OK;
-  int blocks = ceil_div(total, 256);
-  if (blocks > 65536) blocks = 65536;
-  box_kernel<<<blocks, 256, 0, s>>>(z0, y0, x0, bz, by, bx, fn);
-  SOPHT_CHECK_LAUNCH();
-  return SOPHT_OK;
-}
-
 // The six width-w boundary slabs of an (nz, ny, nx) box, written in the reference's order
 // (z front/back, y front/back, x front/back; elementwise_ops_3d.py:228-233). Overlaps are
 // written more than once with the same value.
@@ -566,13 +539,17 @@ bool eno3_rows_ok(const int64_t* fs, const int64_t* is, const int64_t* vs, int64
          row_strides_ok(vs, nz, ny, nx);
 }
 
-template <typename T, bool SET>
+template <typename T, int MODE>
 int eno3_rows(void* flux, const int64_t* fs, const void* field, const int64_t* is, const void* const vel[3],
               const int64_t* vs, int64_t nz, int64_t ny, int64_t nx, T inv_dx, hipStream_t s) {
   const RowGeo g = row_geo<T>(nz, ny, nx, kEnoChunk);
-  k_eno3_rows<T, SET><<<row_blocks(g), kRowThreads, 0, s>>>(g, static_cast<T*>(flux), row_strides(fs),
-                                                          static_cast<const T*>(field), row_strides(is),
-                                                          rows3<T>(vel, vs), inv_dx);
+  Rows3<T> o{};
+  Rows3<const T> f{};
+  o.p[0] = static_cast<T*>(flux);
+  o.s = row_strides(fs);
+  f.p[0] = static_cast<const T*>(field);
+  f.s = row_strides(is);
+  k_eno3_rows<T, MODE><<<row_blocks(g), kRowThreads, 0, s>>>(g, o, f, rows3<T>(vel, vs), inv_dx);
   SOPHT_CHECK_LAUNCH();
   return SOPHT_OK;
 }
@@ -583,7 +560,7 @@ int eno3_impl(void* flux, const int64_t* fs, const void* field, const int64_t* i
               T inv_dx, hipStream_t s) {
   if (nz <= 4 || ny <= 4 || nx <= 4) return SOPHT_OK;
   if (eno3_rows_ok<T>(fs, is, vs, nz, ny, nx))
-    return eno3_rows<T, false>(flux, fs, field, is, vel, vs, nz, ny, nx, inv_dx, s);
+    return eno3_rows<T, kEnoAdd>(flux, fs, field, is, vel, vs, nz, ny, nx, inv_dx, s);
   const Strides3 os3 = strides_of(fs), is3 = strides_of(is), vs3 = strides_of(vs);
   T* o = static_cast<T*>(flux);
   const T* f = static_cast<const T*>(field);
@@ -616,7 +593,7 @@ int eno3_set_impl(void* flux, const int64_t* fs, const void* field, const int64_
   bool apart = true;
   for (int a = 0; a < 3; ++a) apart = apart && !fields_meet<T>(flux, fs, vel[a], vs, nz, ny, nx);
   if (apart && eno3_rows_ok<T>(fs, is, vs, nz, ny, nx) && !fields_meet<T>(flux, fs, field, is, nz, ny, nx))
-    return eno3_rows<T, true>(flux, fs, field, is, vel, vs, nz, ny, nx, inv_dx, s);
+    return eno3_rows<T, kEnoSet>(flux, fs, field, is, vel, vs, nz, ny, nx, inv_dx, s);
   int rc = set_impl<T>(1, &flux, fs, nz, ny, nx, Three<T>{}, s);
   return rc ? rc : eno3_impl<T>(flux, fs, field, is, vel, vs, nz, ny, nx, inv_dx, s);
 }

@@ -4,8 +4,8 @@ Advection-diffusion of a passive scalar or vector ``primary_field`` by a given
 ``velocity_field``. The reference runs two factory kernels per component (the conservative
 ENO3 advection step, then the Euler diffusion step, sharing ``buffer_scalar_field`` as
 flux buffer); here one ``time_step`` is one call of ``sopht_passive_transport_step_3d``:
-a fused sweep that advects and diffuses all components together, reading the velocity
-once, with the advected field kept on chip. ``compute_stable_timestep`` reduces
+an advection sweep over all components into a scratch field and a diffusion sweep from it
+back into the field. ``compute_stable_timestep`` reduces
 ``sum_i |u_i|`` on the device (``sopht_velocity_abs_sum_max_3d``, which also leaves the
 per-cell sums in ``buffer_scalar_field`` as the reference does) and reads back one scalar.
 
@@ -60,8 +60,7 @@ class PassiveTransportFlowSimulator(FlowSimulator):
         self.primary_field = make(*comp_shape) if self._ncomp == 1 else make(self._ncomp, *comp_shape)
         self.velocity_field = make(self.grid_dim, *comp_shape)
         self.buffer_scalar_field = make(*comp_shape)
-        # the sweep writes the new field out of place (neighbouring tiles still read the old
-        # one), then copies it back: one scratch field per component
+        # the advected field, one scratch field per component
         self._next = make(self._ncomp, *comp_shape)
         self._partials = make(_PARTIALS)
         self._vmax = make(1)

@@ -1,4 +1,5 @@
-"""Drop-in ``FastDiagPoissonSolver3D`` on rocBLAS GEMMs (gfx950 MFMA).
+"""Drop-in ``FastDiagPoissonSolver3D`` on cosine transforms, or rocBLAS GEMMs (gfx950 MFMA) for
+sizes without a transform.
 
 Same constructor and methods as
 ``sopht/numeric/eulerian_grid_ops/poisson_solver_3d/FastDiagPoissonSolver3D.py:12-202``:

@@ -51,6 +51,7 @@ struct Member {
   int* pcount;
   int* poff;
   uint32_t* plist;
+  uint32_t* owners;
   int padded;
 };
 
@@ -133,7 +134,7 @@ __global__ void __launch_bounds__(256) k_vbf_time_step_batch(const Member<T>* M)
 template <typename T>
 __global__ void __launch_bounds__(256) k_vbf_lag_force_batch(const Member<T>* M, const int64_t* off,
                                                              int count, int64_t total) {
-  const int64_t node = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  const int64_t node = int64_t(xcd_run(int(gridDim.x), int(blockIdx.x))) * 4 + (threadIdx.x >> 6);
   if (node >= total) return;  // whole wavefronts leave together; no barriers follow
   const int m = find_member(off, count, node);
   vbf_lag_force_node<T>(M[m].vb, node - off[m], threadIdx.x & 63);
@@ -165,7 +166,7 @@ __global__ void __launch_bounds__(512) k_spread_plan_batch(const Member<T>* M, c
   __syncthreads();
   const int64_t gid = (int64_t(blockIdx.x) - off[m]) * 512 + threadIdx.x;
   if ((gid >> 6) < n)
-    spread_plan_slot(S.g.nz, S.g.ny, S.g.nx, sk, n, S.flag, S.pcount, S.poff, S.plist, gid);
+    spread_plan_slot(S.g.nz, S.g.ny, S.g.nx, sk, n, S.flag, S.pcount, S.poff, S.plist, S.owners, gid);
 }
 
 template <typename T>
@@ -173,11 +174,18 @@ __global__ void __launch_bounds__(512) k_spread_replay_batch(const Member<T>* M,
                                                              int count) {
   const int m = find_member(off, count, blockIdx.x);
   const Member<T>& S = M[m];
-  const int64_t gid = (int64_t(blockIdx.x) - off[m]) * 512 + threadIdx.x;
-  if (gid == 0) atomicExch(S.flag + 1, 0);
-  if (gid < 64 * S.vb.n)
-    spread_replay_slot<T, false>(3, S.Fw, S.g.nz, S.g.ny, S.g.nx, S.vb.F, S.vb.weights, S.keys, S.vb.n,
-                          S.pcount, S.poff, S.plist, gid);
+  constexpr int G = 512 / kReplayLanes;
+  __shared__ __align__(16) T stage[G][3][kReplayLanes];
+  const int64_t b = int64_t(blockIdx.x) - off[m];
+  if (b == 0 && threadIdx.x == 0) atomicExch(S.flag + 1, 0);
+  const int owned = flag_load(S.flag + 3);
+  const int g = int(threadIdx.x) / kReplayLanes;
+  for (int64_t o0 = b * G; o0 < owned; o0 += (off[m + 1] - off[m]) * G) {
+    const bool live = o0 + g < owned;
+    const int64_t o = live ? o0 + g : 0;
+    spread_replay_cell<T>(3, S.Fw, uint32_t(S.g.ny), uint32_t(S.g.nx), S.vb.F, S.vb.weights, S.keys, S.vb.n,
+                          live ? S.pcount[o] : 0, S.poff[o], S.plist, S.owners[o], stage[g]);
+  }
 }
 
 // F = 0 on every member (once, before the first step; afterwards SC leaves F zeroed)
@@ -396,6 +404,7 @@ int batch_build(sopht_ns3d_batch* B, const sopht_batch_member* mem, hipStream_t 
       S.pcount = w->pcount;
       S.poff = w->poff;
       S.plist = w->plist;
+      S.owners = w->owners;
       S.padded = int(w->padded);
       B->max_padded = std::max(B->max_padded, S.padded);
     }

@@ -88,6 +88,13 @@ __device__ __forceinline__ Cplx<T> mul_mi(Cplx<T> a) {
   return INV ? Cplx<T>{-a.im, a.re} : Cplx<T>{a.im, -a.re};
 }
 
+// The work item of this workgroup when each XCD is to take a contiguous run of items (workgroup
+// b runs on XCD b mod 8, and each XCD has its own L2), for any number of workgroups.
+__device__ __forceinline__ int xcd_run(int blocks, int b) {
+  const int per = blocks / 8, more = blocks % 8, xcd = b % 8;
+  return xcd * per + (xcd < more ? xcd : more) + b / 8;
+}
+
 inline int ceil_div(int64_t a, int64_t b) { return static_cast<int>((a + b - 1) / b); }
 
 // Per-stage timing with HIP events recorded on the launch stream between consecutive

@@ -192,10 +192,9 @@ int spread_impl(int dtype, int ncomp, sopht_spread3d* ws, void* const eul[3], co
                 F.sz = es[0]; F.sy = es[1]; F.sx = es[2];
                 const T* L = static_cast<const T*>(lag);
                 const T* W = static_cast<const T*>(weights);
-                // about four wavefronts per node for the wavefront form (a node owns ~4 cells)
-                k_spread_replay<T><<<std::min(8192, blocks_for(n * 4, 4)), 256, 0, s>>>(
-                    ncomp, F, nz, ny, nx, L, W, ws->keys, n, ws->pcount, ws->poff, ws->plist,
-                    ws->owners, ws->flag);
+                // a node owns up to about eight cells; a workgroup takes 16 at a time
+                k_spread_replay<T><<<std::min(8192, blocks_for(n, 2)), 256, 0, s>>>(
+                    ncomp, F, ny, nx, L, W, ws->keys, n, ws->pcount, ws->poff, ws->plist, ws->owners, ws->flag);
               }()));
   SOPHT_CHECK_LAUNCH();
   return SOPHT_OK;

@@ -17,14 +17,14 @@ struct sopht_spread3d {
   uint64_t* prev;     // unsorted keys of the previous call, padded
   int* flag;          // [0] out-of-domain, [1] keys changed since the plan was built,
                       // [2] fill counter of the plan's contributor list, [3] owner count,
-                      // [4] largest contributor count of an owned cell (8 ints)
-  // Gather plan, rebuilt only when the keys change: for support slot t = 64 p + s of sorted
-  // node p that owns its cell, pcount[t] contributors starting at plist[poff[t]], each
-  // (node << 6 | slot) in increasing node order; pcount[t] = 0 for the other slots.
+                      // [5] a declared plan turned out stale (8 ints)
+  // Gather plan, rebuilt only when the keys change: owners[o] (o < flag[3]) is a support slot
+  // t = 64 p + s of sorted node p that owns its cell, with pcount[o] contributors starting at
+  // plist[poff[o]], each (node << 6 | slot) in increasing node order.
   int* pcount;
   int* poff;
   uint32_t* plist;
-  uint32_t* owners;   // owning slots t of the plan (flag[3] of them), for the list merge
+  uint32_t* owners;
   // Lower-bound table of the sorted keys over the bounding box of the node base cells (built
   // with the sort when the box fits, else bbox[0] = 0 and the plan build searches the keys):
   // bbox = {valid, z0, y0, x0, Z, Y, X}; table[l] = number of sorted keys whose cell comes
@@ -51,17 +51,6 @@ __device__ __forceinline__ void ib_wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Value of v in lane j (j uniform over the wavefront).
-__device__ __forceinline__ float lane_value(float v, int j) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), j));
-}
-__device__ __forceinline__ double lane_value(double v, int j) {
-  const uint64_t b = __builtin_bit_cast(uint64_t, v);
-  const uint32_t lo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(b)), j));
-  const uint32_t hi = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(b >> 32)), j));
-  return __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
 }
 
 // numpy floor_divide for doubles (npy_divmod): exact floor of a / b including the
@@ -298,7 +287,9 @@ __device__ __forceinline__ void vbf_lag_force_node(const VbfArgs<T>& A, int64_t 
 
 template <typename T>
 __global__ void __launch_bounds__(256) k_vbf_lag_force(VbfArgs<T> A) {
-  const int64_t i = int64_t(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  // a node's weights and support go to 256 lines that its neighbours in number share: runs of
+  // nodes per XCD complete those lines in one L2 (3000 nodes FP32 13.1 -> 10.4 us)
+  const int64_t i = int64_t(xcd_run(int(gridDim.x), int(blockIdx.x))) * (blockDim.x >> 6) + (threadIdx.x >> 6);
   if (i >= A.n) return;  // whole wavefronts leave together; no barriers follow
   vbf_lag_force_node<T>(A, i, threadIdx.x & 63);
 }
@@ -566,7 +557,6 @@ __global__ void __launch_bounds__(1024) k_bitonic_lds(const uint64_t* prev, uint
                                                       int64_t nx, int* table, int* bb, int cap) {
   extern __shared__ uint64_t sk[];
   if (flag_load(flag + 1) == 0) return;  // keys unchanged: sort and table stay valid
-  if (threadIdx.x == 0) atomicExch(flag + 4, 0);
   bitonic_block(prev, keys, padded, flag, sk);
   int* cnt = reinterpret_cast<int*>(sk + padded);
   cell_table_block(sk, padded, ny, nx, cap, cnt, cnt + cap, cnt + cap + 1024, table, bb);
@@ -597,7 +587,6 @@ __global__ void k_copy_keys(const uint64_t* src, uint64_t* dst, int64_t m, int* 
   if (i == 0) {
     atomicExch(flag + 2, 0);
     atomicExch(flag + 3, 0);
-    atomicExch(flag + 4, 0);
     bb[0] = 0;  // no box table on this path: the plan build searches the keys
   }
 }
@@ -643,15 +632,12 @@ struct EulW3 {
 __device__ __forceinline__ void spread_plan_slot(int64_t nz, int64_t ny, int64_t nx,
                                                  const uint64_t* keys, int64_t n, int* flag,
                                                  int* pcount, int* poff, uint32_t* plist,
-                                                 int64_t gid) {
+                                                 uint32_t* owners, int64_t gid) {
   const int64_t p = gid >> 6;
   const int slot = int(gid & 63);
   if (p >= n) return;
   const uint64_t kp = keys[p];
-  if (kp == ~uint64_t(0)) {  // out-of-domain node (sorted to the end)
-    pcount[gid] = 0;
-    return;
-  }
+  if (kp == ~uint64_t(0)) return;  // out-of-domain node (sorted to the end)
   const int64_t cell0 = int64_t(kp >> 32);
   const int64_t bx = cell0 % nx, by = (cell0 / nx) % ny, bz = cell0 / (nx * ny);
   const int kz = slot >> 4, ky = (slot >> 2) & 3, kx = slot & 3;
@@ -685,14 +671,12 @@ __device__ __forceinline__ void spread_plan_slot(int64_t nz, int64_t ny, int64_t
       }
     }
   }
-  if (!owner) {
-    pcount[gid] = 0;
-    return;
-  }
-  // the list's place in plist depends on scheduling; its contents do not
-  const int base = atomicAdd(flag + 2, m);
-  pcount[gid] = m;
-  poff[gid] = base;
+  if (!owner) return;
+  // the places in the lists depend on scheduling; their contents do not
+  const int base = atomicAdd(flag + 2, m), o = atomicAdd(flag + 3, 1);
+  owners[o] = uint32_t(gid);
+  pcount[o] = m;
+  poff[o] = base;
   int64_t last = -1;
   for (int k = 0; k < m; ++k) {
     int64_t best = INT64_MAX;
@@ -719,9 +703,9 @@ __device__ __forceinline__ void spread_plan_slot(int64_t nz, int64_t ny, int64_t
 // is the first of c's contributors in key order, i.e. when the first non-empty range among
 // c's candidate base-cell ranges (searched in increasing key order) starts at p. An owner
 // also counts its contributors m (the lengths of all 16 ranges); a workgroup then reserves
-// its owners' places in the owner list and their m-entry windows of the contributor list
-// with one atomic each (same-address atomics from every owner serialise). pcount[t] = m for
-// owners, 0 otherwise. Ranges: a box-table lookup (two per range) when the table is valid,
+// its owners' places o in the owner list and their m-entry windows of the contributor list
+// with one atomic each (same-address atomics from every owner serialise): owners[o] = t,
+// pcount[o] = m, poff[o] = the window. Ranges: a box-table lookup (two per range) when the table is valid,
 // else binary searches of the sorted keys.
 __device__ __forceinline__ int spread_owner_count(int64_t nz, int64_t ny, int64_t nx,
                                                   const uint64_t* keys, int64_t n, int64_t gid,
@@ -784,7 +768,7 @@ __global__ void __launch_bounds__(512) k_spread_owner(int64_t nz, int64_t ny, in
                                                       const int* table, const int* bb) {
   if (flag_load(flag + 1) == 0) return;  // plan still valid (uniform for the launch)
   extern __shared__ uint64_t skeys[];
-  __shared__ int wo[8], wm[8], wx[8], base_o, base_m;
+  __shared__ int wo[8], wm[8], base_o, base_m;
   const bool use_table = bb[0] != 0;     // uniform
   const uint64_t* keys = gkeys;
   if constexpr (LDS_KEYS) {
@@ -798,43 +782,37 @@ __global__ void __launch_bounds__(512) k_spread_owner(int64_t nz, int64_t ny, in
   const int64_t gid = blockIdx.x * int64_t(blockDim.x) + tid;
   const bool live = (gid >> 6) < n;
   const int m = live ? spread_owner_count(nz, ny, nx, keys, n, gid, table, bb, use_table) : 0;
-  int so = m > 0 ? 1 : 0, sm = m, mx = m;  // inclusive scans (and the maximum) over the wavefront
+  int so = m > 0 ? 1 : 0, sm = m;  // inclusive scans over the wavefront
   for (int sft = 1; sft < 64; sft <<= 1) {
     const int a = __shfl_up(so, sft, 64), b = __shfl_up(sm, sft, 64);
-    const int c = __shfl_xor(mx, sft, 64);
     if (lane >= sft) {
       so += a;
       sm += b;
     }
-    mx = c > mx ? c : mx;
   }
   if (lane == 63) {
     wo[w] = so;
     wm[w] = sm;
-    wx[w] = mx;
   }
   __syncthreads();
   if (tid == 0) {
-    int to = 0, tm = 0, tx = 0;
+    int to = 0, tm = 0;
     for (int i = 0; i < int(blockDim.x >> 6); ++i) {
       const int a = wo[i], b = wm[i];
       wo[i] = to;
       wm[i] = tm;
       to += a;
       tm += b;
-      tx = wx[i] > tx ? wx[i] : tx;
     }
     base_o = to > 0 ? atomicAdd(flag + 3, to) : 0;
     base_m = tm > 0 ? atomicAdd(flag + 2, tm) : 0;
-    if (tx > 0) atomicMax(flag + 4, tx);
   }
   __syncthreads();
-  if (live) {
-    pcount[gid] = m;
-    if (m > 0) {
-      owners[base_o + wo[w] + so - 1] = uint32_t(gid);
-      poff[gid] = base_m + wm[w] + sm - m;
-    }
+  if (live && m > 0) {  // the owner's place in the list holds its count and window too
+    const int o = base_o + wo[w] + so - 1;
+    owners[o] = uint32_t(gid);
+    pcount[o] = m;
+    poff[o] = base_m + wm[w] + sm - m;
   }
 }
 
@@ -849,7 +827,7 @@ constexpr int kMergeWaves = 4, kMergeCap = 1024;  // LDS entries per wavefront
 
 __device__ __forceinline__ void spread_merge_owner(int64_t nz, int64_t ny, int64_t nx,
                                                    const uint64_t* keys, int64_t n, int* flag,
-                                                   int* pcount, int* poff, uint32_t* plist,
+                                                   int reserved, int base, uint32_t* plist,
                                                    int64_t gid, int lane, uint32_t* stage,
                                                    const int* table, const int* bb, bool use_table) {
   const int64_t p = gid >> 6;
@@ -875,12 +853,10 @@ __device__ __forceinline__ void spread_merge_owner(int64_t nz, int64_t ny, int64
     const int v = __shfl_up(incl, sft, 64);
     if (lane >= sft) incl += v;
   }
-  // the lanes' runs telescope to the owner pass's ranges, so the total equals pcount[gid];
+  // the lanes' runs telescope to the owner pass's ranges, so the total equals the count reserved;
   // the window reserved there is never exceeded
   const int mc = __shfl(incl, 63, 64);
-  const int reserved = pcount[gid];
   const int m = mc < reserved ? mc : reserved;
-  const int base = poff[gid];
   const int mine = incl - len;  // this lane's window in the stage
   if (mc <= kMergeCap) {        // uniform: rank the staged entries
     // entries (node << 6 | slot) with unique nodes: their order is the node order, and an
@@ -930,137 +906,90 @@ __global__ void __launch_bounds__(64 * kMergeWaves) k_spread_merge(
   const int64_t waves = int64_t(gridDim.x) * kMergeWaves;
   const int64_t count = flag_load(flag + 3);
   for (int64_t o = int64_t(blockIdx.x) * kMergeWaves + w; o < count; o += waves)
-    spread_merge_owner(nz, ny, nx, keys, n, flag, pcount, poff, plist, int64_t(owners[o]), lane,
+    spread_merge_owner(nz, ny, nx, keys, n, flag, pcount[o], poff[o], plist, int64_t(owners[o]), lane,
                        stage[w], table, bb, use_table);
 }
 
-// contributors per cell whose list entries a replay thread loads all at once
-constexpr int kReplayGather = 32;
-
-// Plan replay for the batched step (every call; one thread per support slot): each owned cell
-// adds its contributors F_lag[node] w[slot][node] in increasing node order, every product and
-// sum rounded separately, exactly as the reference's serial `F[block] += F_n * w_n`. GATHER
-// (the single-simulator replay, whose cells have at most kReplayGather contributors): a cell's
-// list entries are loaded at once and its products formed eight at a time (19.8 -> 16.6 us at
-// the 3000-node sphere). The batched replay keeps the plain loop: its dense small-grid members
-// have cells with hundreds of contributors, and the gathered form made that launch slower
-// (4.13 -> 4.18 ms per batched step).
-template <typename T, bool GATHER>
-__device__ __forceinline__ void spread_replay_slot(int ncomp, const EulW3<T>& F, int64_t nz,
-                                                   int64_t ny, int64_t nx, const T* lag,
-                                                   const T* weights, const uint64_t* keys,
-                                                   int64_t n, const int* pcount, const int* poff,
-                                                   const uint32_t* plist, int64_t gid) {
-#pragma clang fp contract(off)
-  const int m = pcount[gid];
-  if (m == 0) return;
-  const int64_t cell0 = int64_t(keys[gid >> 6] >> 32);
-  const int slot = int(gid & 63);
-  const int64_t cx = cell0 % nx + (slot & 3), cy = (cell0 / nx) % ny + ((slot >> 2) & 3),
-                cz = cell0 / (nx * ny) + (slot >> 4);
-  const int64_t cidx = cz * F.sz + cy * F.sy + cx * F.sx;
-  T acc[3];
-  for (int c = 0; c < ncomp; ++c) acc[c] = F.p[c][cidx];
-  const int o = poff[gid];
-  if (GATHER && m <= kReplayGather) {
-    // every list entry of the cell is loaded first and then the products in groups of eight,
-    // so the loads of many contributions are in flight together; the sums still run one after
-    // another in list order
-    uint32_t es[kReplayGather];
-    static_for_sort<0, kReplayGather>([&](auto k_) {
-      constexpr int k = decltype(k_)::value;
-      es[k] = k < m ? plist[o + k] : 0u;
-    });
-    static_for_sort<0, kReplayGather / 8>([&](auto g_) {
-      constexpr int g0 = 8 * decltype(g_)::value;
-      if (g0 < m) {
-        T pr[8][3];
-        static_for_sort<0, 8>([&](auto k_) {
-          constexpr int k = decltype(k_)::value;
-          const int64_t node = int64_t(es[g0 + k] >> 6);
-          const bool live = g0 + k < m;
-          const T w = live ? weights[int64_t(es[g0 + k] & 63u) * n + node] : T(0);
-          static_for_sort<0, 3>([&](auto c_) {
-            constexpr int c = decltype(c_)::value;
-            pr[k][c] = (live && c < ncomp) ? lag[c * n + node] * w : T(0);
-          });
-        });
-        static_for_sort<0, 8>([&](auto k_) {
-          constexpr int k = decltype(k_)::value;
-          if (g0 + k < m)
-            static_for_sort<0, 3>([&](auto c_) {
-              constexpr int c = decltype(c_)::value;
-              if (c < ncomp) acc[c] = acc[c] + pr[k][c];
-            });
-        });
-      }
-    });
-  } else {
-#pragma unroll 4
-    for (int k = 0; k < m; ++k) {
-      const uint32_t e = plist[o + k];
-      const int64_t node = int64_t(e >> 6);
-      const T w = weights[int64_t(e & 63u) * n + node];
-      for (int c = 0; c < ncomp; ++c) acc[c] = acc[c] + lag[c * n + node] * w;
-    }
-  }
-  for (int c = 0; c < ncomp; ++c) F.p[c][cidx] = acc[c];
-}
-
-// Plan replay over the owner list of the plan build, in one of two forms chosen on the device
-// from the plan's largest contributor count (uniform for the launch):
-// - at most kThreadReplayMax contributors per cell: one thread per owned cell, the per-slot sum
-//   of spread_replay_slot without the idle slots;
-// - more: one wavefront per owned cell. The lanes load up to 64 contributions at once and form
-//   their products F_lag[node] w[slot][node]; the products are then added to the cell's value
-//   one after another in increasing node order (every lane keeps the same running sum).
-// Either way every product and sum is rounded separately, exactly as the reference's serial
-// `F[block] += F_n * w_n`. Clears the keys-changed flag for the next call.
-constexpr int kThreadReplayMax = 32;
+// Plan replay (every call): each owned cell adds its contributors F_lag[node] w[slot][node] in
+// increasing node order, every product and sum rounded separately, exactly as the reference's
+// serial `F[block] += F_n * w_n`.
+// A cell takes 16 lanes, four cells a wavefront. The lanes load 16 contributions at once (the
+// next 16 while the current ones are summed) and leave their products in LDS; lane c then adds
+// component c's products one after another, so the three serial sums of the four cells run in
+// one instruction stream. Bound by the latency of the chain owner -> window -> list entry ->
+// weight and force -> sum (and, in large batches, by the gathers' requests to L2). Measured
+// against one thread per cell for cells of at most 32 contributors, else one wavefront per cell
+// with the 64 lanes repeating every sum: 3000-node sphere, 256^3 FP32, 11.1 us (17.8); 2000-node
+// ellipsoid, 128^3 FP32, 9.8 (26.6); 1200-node sphere, 64^3 FP64, 9.2 (26.6). The batch of 16
+// members of 1000 nodes takes 32.6 us (31.2 with one thread per support slot).
+constexpr int kReplayLanes = 16;
 
 template <typename T>
-__global__ void __launch_bounds__(256) k_spread_replay(
-    int ncomp, EulW3<T> F, int64_t nz, int64_t ny, int64_t nx, const T* lag, const T* weights,
-    const uint64_t* keys, int64_t n, const int* pcount, const int* poff, const uint32_t* plist,
-    const uint32_t* owners, int* flag) {
+__device__ __forceinline__ void spread_replay_cell(int ncomp, const EulW3<T>& F, uint32_t ny, uint32_t nx,
+                                                   const T* lag, const T* weights, const uint64_t* keys,
+                                                   int64_t n, int m, int base, const uint32_t* plist,
+                                                   uint32_t gid, T (*stage)[kReplayLanes]) {
 #pragma clang fp contract(off)
+  const int l = int(threadIdx.x) & (kReplayLanes - 1);
+  T* cell = nullptr;  // lanes 0 .. ncomp - 1: the cell's value of their component
+  T acc = T(0);
+  if (m > 0 && l < ncomp) {
+    const uint32_t cell0 = uint32_t(keys[gid >> 6] >> 32), slot = gid & 63u;
+    const uint32_t row = cell0 / nx, cx = cell0 - row * nx + (slot & 3u), cy = row % ny + ((slot >> 2) & 3u),
+                   cz = row / ny + (slot >> 4);
+    T* const p = l == 0 ? F.p[0] : (l == 1 ? F.p[1] : F.p[2]);
+    cell = p + (int64_t(cz) * F.sz + int64_t(cy) * F.sy + int64_t(cx) * F.sx);
+    acc = *cell;
+  }
+  int most = m;  // of the wavefront's cells
+  for (int sft = kReplayLanes; sft < 64; sft <<= 1) {
+    const int o = __shfl_xor(most, sft, 64);
+    most = o > most ? o : most;
+  }
+  T pr[3];
+  auto fetch = [&](int k) {
+    const bool in = k + l < m;
+    const uint32_t e = in ? plist[base + k + l] : 0u;
+    const int64_t node = int64_t(e >> 6);
+    const T w = in ? weights[int64_t(e & 63u) * n + node] : T(0);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) pr[c] = in && c < ncomp ? lag[c * n + node] * w : T(0);
+  };
+  fetch(0);
+  for (int k0 = 0; k0 < most; k0 += kReplayLanes) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) stage[c][l] = pr[c];
+    ib_wave_sync();
+    if (k0 + kReplayLanes < most) fetch(k0 + kReplayLanes);
+    if (l < 3) {
+      T v[kReplayLanes];
+#pragma unroll
+      for (int j = 0; j < kReplayLanes; ++j) v[j] = stage[l][j];
+#pragma unroll
+      for (int j = 0; j < kReplayLanes; ++j) acc = k0 + j < m ? acc + v[j] : acc;
+    }
+    ib_wave_sync();
+  }
+  if (cell) *cell = acc;
+}
+
+// The replay over the owner list of the plan build. Clears the keys-changed flag for the next
+// call.
+template <typename T>
+__global__ void __launch_bounds__(256) k_spread_replay(
+    int ncomp, EulW3<T> F, int64_t ny, int64_t nx, const T* lag, const T* weights, const uint64_t* keys,
+    int64_t n, const int* pcount, const int* poff, const uint32_t* plist, const uint32_t* owners, int* flag) {
+  constexpr int G = 256 / kReplayLanes;
+  __shared__ __align__(16) T stage[G][3][kReplayLanes];
   if (flag_load(flag + 5) != 0) return;  // a plan declared valid whose keys changed (uniform)
   if (blockIdx.x == 0 && threadIdx.x == 0) atomicExch(flag + 1, 0);
-  const int64_t count = flag_load(flag + 3);
-  if (flag_load(flag + 4) <= kThreadReplayMax) {
-    for (int64_t o = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; o < count;
-         o += int64_t(gridDim.x) * blockDim.x)
-      spread_replay_slot<T, true>(ncomp, F, nz, ny, nx, lag, weights, keys, n, pcount, poff,
-                                  plist, int64_t(owners[o]));
-    return;
-  }
-  const int lane = int(threadIdx.x & 63);
-  const int64_t waves = int64_t(gridDim.x) * (blockDim.x >> 6);
-  for (int64_t o = int64_t(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6); o < count; o += waves) {
-    const int64_t gid = int64_t(owners[o]);
-    const int m = pcount[gid];
-    const int base = poff[gid];
-    const int64_t cell0 = int64_t(keys[gid >> 6] >> 32);
-    const int slot = int(gid & 63);
-    const int64_t cx = cell0 % nx + (slot & 3), cy = (cell0 / nx) % ny + ((slot >> 2) & 3),
-                  cz = cell0 / (nx * ny) + (slot >> 4);
-    const int64_t cidx = cz * F.sz + cy * F.sy + cx * F.sx;
-    T acc[3] = {T(0), T(0), T(0)};
-    for (int c = 0; c < ncomp; ++c) acc[c] = F.p[c][cidx];
-    for (int k0 = 0; k0 < m; k0 += 64) {
-      T p[3] = {T(0), T(0), T(0)};
-      if (k0 + lane < m) {
-        const uint32_t e = plist[base + k0 + lane];
-        const int64_t node = int64_t(e >> 6);
-        const T w = weights[int64_t(e & 63u) * n + node];
-        for (int c = 0; c < ncomp; ++c) p[c] = lag[c * n + node] * w;
-      }
-      const int cnt = m - k0 < 64 ? m - k0 : 64;
-      for (int j = 0; j < cnt; ++j)
-        for (int c = 0; c < ncomp; ++c) acc[c] = acc[c] + lane_value(p[c], j);
-    }
-    if (lane == 0)
-      for (int c = 0; c < ncomp; ++c) F.p[c][cidx] = acc[c];
+  const int count = flag_load(flag + 3);
+  const int g = int(threadIdx.x) / kReplayLanes;
+  for (int64_t o0 = int64_t(blockIdx.x) * G; o0 < count; o0 += int64_t(gridDim.x) * G) {
+    const bool live = o0 + g < count;
+    const int64_t o = live ? o0 + g : 0;
+    spread_replay_cell<T>(ncomp, F, uint32_t(ny), uint32_t(nx), lag, weights, keys, n, live ? pcount[o] : 0, poff[o],
+                          plist, owners[o], stage[g]);
   }
 }
 

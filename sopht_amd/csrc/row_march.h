@@ -117,11 +117,8 @@ struct RowCol {
   unsigned own, inner;  // cells to store; those inside in x
 
   __device__ __forceinline__ RowCol(const RowGeo& g) {
-    // contiguous runs of workgroups per XCD, so that rows shared by neighbouring workgroups
-    // meet in one L2 (workgroup b runs on XCD b mod 8)
-    const int total = int(gridDim.x), per = total / 8, more = total % 8;
-    const int xcd = int(blockIdx.x) % 8;
-    const int item = xcd * per + (xcd < more ? xcd : more) + int(blockIdx.x) / 8;
+    // rows shared by neighbouring workgroups meet in one L2
+    const int item = xcd_run(int(gridDim.x), int(blockIdx.x));
     const int tile = item % g.tiles;
     z0 = (item / g.tiles) * g.chunk;
     z1 = z0 + g.chunk < g.nz ? z0 + g.chunk : g.nz;

@@ -250,7 +250,7 @@ int sopht_poisson3d_destroy(sopht_poisson3d* plan);
 /* Bytes of device scratch the plan holds (for capacity planning). */
 int64_t sopht_poisson3d_scratch_bytes(const sopht_poisson3d* plan);
 /* The plan's FFT schedule (no counterpart in the reference, which leaves it to FFTW's
- * planner): *passes is 3 (x transform fused with the inner y sums; FP32, nx = ny) or 5, and
+ * planner): *passes is 3 (x transform fused with the inner y sums; FP32, 2 nx and 2 ny from 96 to 512) or 5, and
  * *zpass_jobs the jobs per workgroup of the three-pass z pass, timed over {1, 2, 3, 6} when
  * the plan was created (SOPHT_POISSON_ZJOBS in the environment fixes it; 0 with five passes).
  * Results do not depend on it. Either pointer may be null. */

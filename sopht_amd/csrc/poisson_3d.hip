@@ -22,6 +22,7 @@
 
 #include "common.h"
 #include "fft_reg.h"
+#include "poisson_xy.h"
 
 struct sopht_poisson3d {
   int dtype;
@@ -39,139 +40,6 @@ struct sopht_poisson3d {
 
 namespace sopht {
 namespace {
-
-// A streaming store of one complex value: the next pass reads it back from HBM, so it need
-// not stay in the cache hierarchy.
-template <typename T>
-__device__ __forceinline__ void store_stream(Cplx<T>* p, Cplx<T> v) {
-  typedef T pair __attribute__((ext_vector_type(2)));
-  pair w;
-  w.x = v.re;
-  w.y = v.im;
-  __builtin_nontemporal_store(w, reinterpret_cast<pair*>(p));
-}
-
-using rfft::LinePlan;
-using rfft::region_stride;
-using rfft::static_for;
-using rfft::team_fft;
-
-// Slab rows (kx = 0..nx) are padded to a whole number of 128-byte lines, so every column
-// tile of the y and z passes reads and writes whole cache lines.
-template <typename T>
-constexpr int kLineCplx = 128 / int(sizeof(Cplx<T>));
-#ifndef SOPHT_COL_HALF
-#define SOPHT_COL_HALF 1
-#endif
-#ifndef SOPHT_ROW_PAD
-#define SOPHT_ROW_PAD 1
-#endif
-// Column tiles are half a 128-byte line when SOPHT_COL_HALF is set; the two halves of a line
-// then go to workgroups b and b + 8, which the dispatcher sends to the same XCD one after the
-// other, so the second half is read from that XCD's L2.
-constexpr int kColHalf = SOPHT_COL_HALF;
-constexpr int64_t kRowPad = SOPHT_ROW_PAD;
-// Columns per slab tile of the three-pass schedule. Measured at 256^3 FP32 (pass A + z pass +
-// pass C): 16 columns 1.21 ms, 8 columns 1.20 ms (the z pass faster, passes A and C slower),
-// 4 columns 2.2 ms (pass A's writes become 32-byte pieces of lines from four planes, which
-// other workgroups write).
-#ifndef SOPHT_SLAB_TILE
-#define SOPHT_SLAB_TILE 16
-#endif
-constexpr int kSlabTile = SOPHT_SLAB_TILE;
-static_assert(16 % kSlabTile == 0, "slab tiles divide a 128-byte line");
-
-// (row, first kx) of the column tile of workgroup b; false for the padding workgroups.
-__device__ __forceinline__ bool col_tile(int64_t b, int64_t ncols, int64_t nrows, int wc,
-                                         int64_t& row, int64_t& kx0) {
-  if (kColHalf) {
-    const int64_t lines = (ncols + 2 * wc - 1) / (2 * wc);
-    const int64_t line = (b / 16) * 8 + b % 8;
-    const int64_t half = (b / 8) % 2;
-    row = line / lines;
-    kx0 = ((line % lines) * 2 + half) * wc;
-    return row < nrows;
-  }
-  const int64_t tiles = (ncols + wc - 1) / wc;
-  row = b / tiles;
-  kx0 = (b % tiles) * wc;
-  return row < nrows;
-}
-
-// The same with a line split in PARTS tiles: the parts of a line go to workgroups
-// b + 8 p (p < PARTS), which the dispatcher sends to one XCD.
-template <int PARTS>
-__device__ __forceinline__ bool col_tile_parts(int64_t b, int64_t ncols, int64_t nrows, int wc,
-                                               int64_t& row, int64_t& kx0) {
-  const int64_t lines = (ncols + PARTS * wc - 1) / (PARTS * wc);
-  const int64_t line = (b / (8 * PARTS)) * 8 + b % 8;
-  const int64_t part = (b / 8) % PARTS;
-  row = line / lines;
-  kx0 = ((line % lines) * PARTS + part) * wc;
-  return row < nrows;
-}
-
-inline int64_t col_tile_parts_blocks(int parts, int64_t ncols, int64_t nrows, int wc) {
-  const int64_t lines = (ncols + parts * wc - 1) / (parts * wc);
-  return 8 * parts * ((lines * nrows + 7) / 8);
-}
-
-inline int64_t col_tile_blocks(int64_t ncols, int64_t nrows, int wc) {
-  if (kColHalf) {
-    const int64_t lines = (ncols + 2 * wc - 1) / (2 * wc);
-    return 16 * ((lines * nrows + 7) / 8);
-  }
-  return (ncols + wc - 1) / wc * nrows;
-}
-
-inline int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
-
-struct SlabGeom {
-  int64_t nz, ny, nx;  // physical grid
-  int64_t rs;          // row stride (complex elements), >= nx + 1
-  int64_t gz;          // G^ line stride (elements), >= nz + 1
-  int ncomp;
-  // H index of (c, z, ky, kx)
-  __device__ __forceinline__ int64_t h(int c, int64_t z, int64_t ky, int64_t kx) const {
-    return ((int64_t(c) * nz + z) * (2 * ny) + ky) * rs + kx;
-  }
-  // the same as a 32-bit offset (plan creation checks that the slab has < 2^31 elements):
-  // loads then take a uniform base plus one VGPR of offset
-  __device__ __forceinline__ int hi(int c, int z, int ky, int kx) const {
-    return ((c * int(nz) + z) * (2 * int(ny)) + ky) * int(rs) + kx;
-  }
-  // The three-pass schedule keeps the slab in column tiles of kSlabTile columns with z inside
-  // a tile: (c, ky, kx / kSlabTile, z, kx % kSlabTile). The z pass then reads and writes each
-  // tile's z line as one contiguous run; with 16 columns (one 128-byte line per plane) the x/y
-  // passes still move whole lines (rs is a multiple of 16 there).
-  // (Unsigned arithmetic: the divisions by the power-of-two tile width are shifts.) Moving by
-  // dr rows adds dr rs nz; moving by a whole number of tiles, dk columns, adds dk nz.
-  __device__ __forceinline__ int ti(int c, int z, int ky, int kx) const {
-    const unsigned k = unsigned(kx);
-    return int((((unsigned(c) * 2u * unsigned(ny) + unsigned(ky)) * (unsigned(rs) / kSlabTile) + k / kSlabTile) *
-                    unsigned(nz) + unsigned(z)) * kSlabTile + k % kSlabTile);
-  }
-  __device__ __forceinline__ int64_t row_h(int64_t r) const {  // H row of input row r
-    const int c = int(r / (nz * ny));
-    const int64_t rem = r % (nz * ny);
-    return h(c, rem / ny, rem % ny, 0);
-  }
-};
-
-// Component fields of a solve: up to three pointers by value, or (batched solves over many
-// instances of one grid size) a device table of one pointer per component.
-struct CompPtrs {
-  const void* p[3];
-  const void* const* tab;
-  int64_t sz, sy, sx;
-  __device__ __forceinline__ const void* get(int c) const { return tab ? tab[c] : p[c]; }
-};
-struct CompPtrsW {
-  void* p[3];
-  void* const* tab;
-  int64_t sz, sy, sx;
-  __device__ __forceinline__ void* get(int c) const { return tab ? tab[c] : p[c]; }
-};
 
 // Row passes (x): one team of T threads per row pair, RowTile::NTEAM teams per workgroup.
 template <typename T, int L>
@@ -517,324 +385,6 @@ __global__ void __launch_bounds__((RowTile<T, L>::NT)) k5_xc2r(SlabGeom g, const
       if (pa) __builtin_nontemporal_store(v[e].re, pa + x * out.sx);
       if (pb) __builtin_nontemporal_store(v[e].im, pb + x * out.sx);
     }
-  });
-}
-
-// ------------------------------------------------------------------ three-pass schedule
-// The y transform (length LY = 2 ny = 4 L2) is split by decimation in time, y = 4 y2 + y1 and
-// ky = k2 + L2 k1:
-//   Y[k2 + L2 k1] = sum_{y1<4} w4^{y1 k1} * [ w_LY^{y1 k2} * sum_{y2} x[4 y2 + y1] w_L2^{y2 k2} ]
-// and its inverse the same way with conjugate roots. Pass A (ka_xy_fwd) runs per (c, z, y1):
-// the x transforms of the rows y = 4 y2 + y1, then the inner L2-point sums over y2 and the
-// twiddle, stored in slab row y1 L2 + k2. The z pass (k3_zconv4) applies the 4-point sums
-// over y1 before its convolution and their inverse after it. Pass C (kc_yx_inv) undoes the
-// twiddle and the inner sums and runs the inverse x transforms. So the x-pass outputs
-// (K1 -> K2) and the inverse y-pass outputs (K4 -> K5) of the five-pass schedule never reach
-// HBM: 24 words per cell fewer.
-
-// Elements of a thread's half spectrum per chunk of the y sums: the most, up to 64 / TX, that
-// divide EX / 2 and keep the chunk's column teams and staging rows within the workgroup.
-constexpr int xy_chunk_elems(int EX, int TX, int T2, int NT, int L2) {
-  int best = 1;
-  for (int k = 1; k == 1 || k * TX <= 64; ++k) {
-    const int cw = k * TX;
-    if ((EX / 2) % k == 0 && cw * T2 <= NT && NT % cw == 0 && L2 % (NT / cw) == 0) best = k;
-  }
-  return best;
-}
-
-// A workgroup of pass A or C holds the ny / 4 rows of its (c, z, y1) as row pairs (two real
-// rows per complex x transform), PPT pairs per team of TX threads. The y sums run on chunks of
-// CW = KC TX columns (kx = CW ch + TX kk + t, element KC ch + kk of every x thread; the last
-// chunk is kx = nx alone), one team of T2 threads per column, staged through LDS. Lines of
-// fewer than 64 x threads take KC > 1, so a chunk still spans a wavefront's width of columns
-// and the workgroup passes fewer chunk barriers.
-template <typename T, int LX, int LY>
-struct XYPass {
-  static constexpr int EX = LinePlan<LX>::E, TX = LinePlan<LX>::T;
-  static constexpr int L2 = LY / 4;
-  static constexpr int E2 = LinePlan<L2>::E, T2 = LinePlan<L2>::T;
-  static constexpr int NY2 = L2 / 2;      // rows of a workgroup (y2 < ny / 4)
-  static constexpr int NPAIR = NY2 / 2;
-  static constexpr int NTEAM = NPAIR * TX <= 1024 ? NPAIR : 1024 / TX;
-  static constexpr int PPT = NPAIR / NTEAM;  // row pairs per x team
-  static constexpr int NT = NTEAM * TX;
-  static constexpr int KC = xy_chunk_elems(EX, TX, T2, NT, L2);
-  static constexpr int CW = KC * TX;         // columns per chunk: kx = CW ch + kk TX + t, kk < KC
-  static constexpr int NCH = EX / 2 / KC + 1;  // the last chunk is kx = nx alone
-  static constexpr int SX = region_stride<LX, false>();
-  static constexpr int S2 = region_stride<L2, true>();
-  // staging tile [row][P]: the column teams' accesses (T2 rows of 32 / T2 columns per half
-  // wavefront) fall in distinct banks when P = 32 / T2 (mod 32)
-  static constexpr int P = (CW + 31) / 32 * 32 + 32 / T2;
-  static constexpr int TW2 = rfft::tw_lds_size<L2>();                // padded w_L2 table
-  static constexpr int XPH = NTEAM * SX + rfft::tw_lds_size<LX>();  // x regions, x table
-  static constexpr int CREG = CW * S2;         // column regions
-  static constexpr int STG = L2 * P;           // staging tile
-  static constexpr int UNION = XPH > CREG ? (XPH > STG ? XPH : STG) : (CREG > STG ? CREG : STG);
-  static constexpr size_t lds = size_t(TW2 + L2 + UNION) * sizeof(Cplx<T>);
-  // the staging tile moves to and from HBM as rows of CW columns: thread tid takes column
-  // tid % CW of the rows tid / CW + q NT / CW
-  static constexpr int RSTEP = NT / CW, NQ = L2 / RSTEP;
-  static_assert(LY % 8 == 0 && NPAIR % NTEAM == 0 && NTEAM >= T2 && T2 <= 32, "three-pass geometry");
-  static_assert(NT % CW == 0 && L2 % RSTEP == 0 && CW * T2 <= NT, "whole staging rows per thread");
-};
-
-// Pass A: x real-to-complex of the rows y = 4 y2 + y1 of (c, z) (two rows per complex FFT,
-// separated as in k1_xr2c), then per column kx the zero-padded L2-point FFT over y2 times
-// w_LY^{y1 k2}, stored in slab row y1 L2 + k2.
-template <typename T, int LX, int LY>
-__global__ void __launch_bounds__((XYPass<T, LX, LY>::NT)) ka_xy_fwd(SlabGeom g, CompPtrs in, Cplx<T>* H,
-                                                                    const Cplx<T>* twx, const Cplx<T>* twy) {
-  using F = XYPass<T, LX, LY>;
-  constexpr int EX = F::EX, TX = F::TX, L2 = F::L2, E2 = F::E2, T2 = F::T2, PPT = F::PPT, P = F::P;
-  constexpr int CW = F::CW, NT = F::NT;
-  extern __shared__ unsigned char smem_raw[];
-  Cplx<T>* const tw2 = reinterpret_cast<Cplx<T>*>(smem_raw);  // w_L2^m = w_LY^{4m}, padded
-  Cplx<T>* const twr = tw2 + F::TW2;                           // w_LY^{y1 k2}
-  Cplx<T>* const U = twr + L2;
-  const int tid = threadIdx.x;
-  const int y1 = int(blockIdx.x & 3);
-  const int cz = int(blockIdx.x >> 2);
-  const int c = cz / int(g.nz), z = cz % int(g.nz);
-  const int team = tid / TX, t = tid % TX;
-  for (int i = tid; i < L2; i += NT) {
-    tw2[rfft::tw_slot(i)] = twy[4 * i];  // padded (w_L2^m = w_LY^{4m})
-    twr[i] = twy[(y1 * i) % LY];
-  }
-  Cplx<T>* const twxl = U + F::NTEAM * F::SX;
-  rfft::load_tw_lds<T, LX>(twxl, twx, tid, NT);
-  const T* base = static_cast<const T*>(in.get(c)) + int64_t(z) * in.sz;
-  Cplx<T> v[PPT][EX];
-  static_for<0, PPT>([&](auto p_) {
-    constexpr int p = decltype(p_)::value;
-    const int y2 = 2 * (team * PPT + p);
-    const T* ra = base + int64_t(4 * y2 + y1) * in.sy + int64_t(t) * in.sx;
-    const T* rb = ra + 4 * in.sy;
-    static_for<0, EX>([&](auto e_) {
-      constexpr int e = decltype(e_)::value;
-      if constexpr (e < EX / 2) {
-        v[p][e] = Cplx<T>{ra[int64_t(TX * e) * in.sx], rb[int64_t(TX * e) * in.sx]};
-      } else {
-        v[p][e] = Cplx<T>{T(0), T(0)};
-      }
-    });
-  });
-  __syncthreads();  // tables complete
-  Cplx<T>* const xline = U + team * F::SX;
-  // half spectra kx = TX e + t (e <= EX / 2; e = EX / 2 is kx = nx, lane 0 only)
-  Cplx<T> A[PPT][EX / 2 + 1], B[PPT][EX / 2 + 1];
-  const int mirror_lane = (TX - t) % TX;
-  static_for<0, PPT>([&](auto p_) {
-    constexpr int p = decltype(p_)::value;
-    rfft::team_fft<T, LX, false, true, true>(v[p], xline, twxl, t);
-    static_for<0, EX / 2 + 1>([&](auto e_) {
-      constexpr int e = decltype(e_)::value;
-      // Z[LX - k], k = TX e + t: lane TX - t, element EX - 1 - e (t > 0); lane 0: EX - e
-      const Cplx<T> zk = v[p][e];
-      Cplx<T> zm;
-      zm.re = __shfl(v[p][EX - 1 - e].re, mirror_lane, TX);
-      zm.im = __shfl(v[p][EX - 1 - e].im, mirror_lane, TX);
-      if (t == 0) zm = v[p][(EX - e) % EX];
-      A[p][e] = Cplx<T>{T(0.5) * (zk.re + zm.re), T(0.5) * (zk.im - zm.im)};
-      B[p][e] = Cplx<T>{T(0.5) * (zk.im + zm.im), T(0.5) * (zm.re - zk.re)};
-    });
-  });
-  __syncthreads();  // x regions free: the chunk phase reuses the area
-  const int col = tid / T2, t2 = tid % T2;
-  const bool col_role = tid < CW * T2;
-  Cplx<T>* const creg = U + col * F::S2;
-  // staging rows to HBM: column sc of rows sr + q RSTEP
-  const int sc = tid % CW, sr = tid / CW;
-  static_for<0, F::NCH>([&](auto ch_) {
-    constexpr int ch = decltype(ch_)::value;
-    constexpr bool last = ch == F::NCH - 1;  // kx = nx alone
-    if constexpr (last) {
-      if (t == 0) {
-        static_for<0, PPT>([&](auto p_) {
-          constexpr int p = decltype(p_)::value;
-          const int y2 = 2 * (team * PPT + p);
-          U[y2 * P] = A[p][EX / 2];
-          U[(y2 + 1) * P] = B[p][EX / 2];
-        });
-      }
-    } else {
-      static_for<0, F::KC>([&](auto k_) {
-        constexpr int kk = decltype(k_)::value;
-        static_for<0, PPT>([&](auto p_) {
-          constexpr int p = decltype(p_)::value;
-          const int y2 = 2 * (team * PPT + p);
-          U[y2 * P + kk * TX + t] = A[p][ch * F::KC + kk];
-          U[(y2 + 1) * P + kk * TX + t] = B[p][ch * F::KC + kk];
-        });
-      });
-    }
-    __syncthreads();
-    const bool live = col_role && (!last || col == 0);
-    Cplx<T> w[E2];
-    if (live) {
-      static_for<0, E2>([&](auto e_) {
-        constexpr int e = decltype(e_)::value;
-        if constexpr (e < E2 / 2) w[e] = U[(t2 + T2 * e) * P + col];
-        else w[e] = Cplx<T>{T(0), T(0)};
-      });
-    }
-    __syncthreads();
-    if (live) {
-      rfft::team_fft<T, L2, false, true, true>(w, creg, tw2, t2);
-      static_for<0, E2>([&](auto e_) {
-        constexpr int e = decltype(e_)::value;
-        w[e] = cmul(w[e], twr[t2 + T2 * e]);
-      });
-    }
-    __syncthreads();
-    if (live) {
-      static_for<0, E2>([&](auto e_) {
-        constexpr int e = decltype(e_)::value;
-        U[(t2 + T2 * e) * P + col] = w[e];
-      });
-    }
-    __syncthreads();
-    if (!last || sc == 0) {
-      static_for<0, F::NQ>([&](auto q_) {
-        constexpr int q = decltype(q_)::value;
-        store_stream(H + g.ti(c, z, y1 * L2 + sr + q * F::RSTEP, CW * ch + sc), U[(sr + q * F::RSTEP) * P + sc]);
-      });
-    }
-    __syncthreads();
-  });
-}
-
-// Pass C: per column kx, w_LY^{-y1 k2} times the slab rows y1 L2 + k2, the inverse L2-point
-// FFT over k2 (outputs y2 < ny / 4), then the Hermitian x half spectra of each row pair to one
-// complex inverse FFT (as in k5_xc2r), rows y = 4 y2 + y1 stored (ACC: added). The next
-// chunk's rows are loaded while the current one is transformed.
-template <typename T, int LX, int LY, bool ACC>
-__global__ void __launch_bounds__((XYPass<T, LX, LY>::NT)) kc_yx_inv(SlabGeom g, const Cplx<T>* H, CompPtrsW out,
-                                                                    const Cplx<T>* twx, const Cplx<T>* twy) {
-  using F = XYPass<T, LX, LY>;
-  constexpr int EX = F::EX, TX = F::TX, L2 = F::L2, E2 = F::E2, T2 = F::T2, PPT = F::PPT, P = F::P;
-  constexpr int CW = F::CW, NT = F::NT;
-  extern __shared__ unsigned char smem_raw[];
-  Cplx<T>* const tw2 = reinterpret_cast<Cplx<T>*>(smem_raw);
-  Cplx<T>* const twr = tw2 + F::TW2;
-  Cplx<T>* const U = twr + L2;
-  const int tid = threadIdx.x;
-  const int y1 = int(blockIdx.x & 3);
-  const int cz = int(blockIdx.x >> 2);
-  const int c = cz / int(g.nz), z = cz % int(g.nz);
-  const int team = tid / TX, t = tid % TX;
-  for (int i = tid; i < L2; i += NT) {
-    tw2[rfft::tw_slot(i)] = twy[4 * i];  // padded (w_L2^m = w_LY^{4m})
-    twr[i] = twy[(y1 * i) % LY];
-  }
-  const int col = tid / T2, t2 = tid % T2;
-  const bool col_role = tid < CW * T2;
-  Cplx<T>* const creg = U + col * F::S2;
-  const int mirror_lane = (TX - t) % TX;
-  // the rows of a chunk: thread tid holds elements tid + NT q of the chunk's L2 x ncol block
-  // (addresses formed per load: a hoisted row pointer costs the registers of the prefetch)
-  Cplx<T> pre[F::NQ];
-  const int hsrc = g.ti(c, z, y1 * L2 + tid / CW, tid % CW);
-  const int rowel = int(g.rs) * int(g.nz);  // elements per slab row
-  auto load_chunk = [&](auto ch_) {
-    constexpr int ch = decltype(ch_)::value;
-    constexpr int ncol = ch == F::NCH - 1 ? 1 : CW;
-    static_for<0, F::NQ>([&](auto q_) {
-      constexpr int q = decltype(q_)::value;
-      const int i = tid + q * NT;
-      if constexpr (ncol == CW && CW % kSlabTile == 0) {
-        // row i / CW = tid / CW + q NT / CW, column CW ch + tid % CW
-        pre[q] = H[hsrc + q * (NT / CW) * rowel + CW * ch * int(g.nz)];
-      } else {
-        if (i < L2 * ncol) pre[q] = H[g.ti(c, z, y1 * L2 + i / ncol, CW * ch + i % ncol)];
-      }
-    });
-  };
-  load_chunk(std::integral_constant<int, 0>{});
-  Cplx<T> v[PPT][EX];
-  static_for<0, F::NCH>([&](auto ch_) {
-    constexpr int ch = decltype(ch_)::value;
-    constexpr bool last = ch == F::NCH - 1;
-    constexpr int ncol = last ? 1 : CW;
-    static_for<0, F::NQ>([&](auto q_) {
-      constexpr int q = decltype(q_)::value;
-      const int i = tid + q * NT;
-      if (i < L2 * ncol) U[(i / ncol) * P + i % ncol] = pre[q];
-    });
-    if constexpr (ch + 1 < F::NCH) load_chunk(std::integral_constant<int, ch + 1>{});
-    __syncthreads();  // (first chunk: the tables too)
-    const bool live = col_role && (!last || col == 0);
-    Cplx<T> w[E2];
-    if (live) {
-      static_for<0, E2>([&](auto e_) {
-        constexpr int e = decltype(e_)::value;
-        w[e] = cmulc(U[(t2 + T2 * e) * P + col], twr[t2 + T2 * e]);
-      });
-    }
-    __syncthreads();
-    if (live) rfft::team_fft<T, L2, true, false, true>(w, creg, tw2, t2);
-    __syncthreads();
-    if (live) {
-      static_for<0, E2 / 2>([&](auto e_) {
-        constexpr int e = decltype(e_)::value;
-        U[(t2 + T2 * e) * P + col] = w[e];
-      });
-    }
-    __syncthreads();
-    static_for<0, (last ? 1 : F::KC)>([&](auto k_) {
-      constexpr int kk = decltype(k_)::value;
-      constexpr int e = last ? EX / 2 : ch * F::KC + kk;  // the element of kx = TX e + t
-      static_for<0, PPT>([&](auto p_) {
-        constexpr int p = decltype(p_)::value;
-        const int y2 = 2 * (team * PPT + p);
-        Cplx<T> a = U[y2 * P + kk * TX + t], b = U[(y2 + 1) * P + kk * TX + t];
-        if ((e == 0 && t == 0) || last) {  // kx = 0 and kx = nx: imaginary parts dropped
-          a.im = T(0);
-          b.im = T(0);
-        }
-        const Cplx<T> zk = {a.re - b.im, a.im + b.re};  // Z[k] = A + i B
-        const Cplx<T> zm = {a.re + b.im, b.re - a.im};  // Z[LX - k] = conj(A) + i conj(B)
-        if constexpr (last) {
-          if (t == 0) v[p][EX / 2] = zk;
-        } else {
-          Cplx<T> r;
-          r.re = __shfl(zm.re, mirror_lane, TX);
-          r.im = __shfl(zm.im, mirror_lane, TX);
-          v[p][e] = zk;
-          // Z[LX - k'] of lane TX - t (k' = TX e + TX - t) is element EX - 1 - e of lane t;
-          // lane 0 keeps its own mirror, element EX - e
-          if (t != 0) v[p][EX - 1 - e] = r;
-          if constexpr (e > 0) {
-            if (t == 0) v[p][EX - e] = zm;
-          }
-        }
-      });
-    });
-    __syncthreads();
-  });
-  Cplx<T>* const twxl = U + F::NTEAM * F::SX;
-  rfft::load_tw_lds<T, LX>(twxl, twx, tid, NT);
-  __syncthreads();
-  Cplx<T>* const xline = U + team * F::SX;
-  T* const base = static_cast<T*>(out.get(c)) + int64_t(z) * out.sz;
-  static_for<0, PPT>([&](auto p_) {
-    constexpr int p = decltype(p_)::value;
-    rfft::team_fft<T, LX, true, false, true>(v[p], xline, twxl, t);
-    const int y2 = 2 * (team * PPT + p);
-    T* const ra = base + int64_t(4 * y2 + y1) * out.sy + int64_t(t) * out.sx;
-    T* const rb = ra + 4 * out.sy;
-    static_for<0, EX / 2>([&](auto e_) {
-      constexpr int e = decltype(e_)::value;
-      const int64_t x = int64_t(TX * e) * out.sx;
-      if constexpr (ACC) {
-        ra[x] += v[p][e].re;
-        rb[x] += v[p][e].im;
-      } else {
-        __builtin_nontemporal_store(v[p][e].re, ra + x);
-        __builtin_nontemporal_store(v[p][e].im, rb + x);
-      }
-    });
   });
 }
 
@@ -1184,9 +734,8 @@ int launch_k5(int64_t L, SlabGeom g, const Cplx<T>* H, CompPtrsW out, const Cplx
   return SOPHT_ERR_UNSUPPORTED;
 }
 
-// Line lengths 2 nx = 2 ny of the three-pass schedule, and 2 nz (longer z lines leave the
-// z pass without registers for its next rows).
-#define SOPHT_XY_LENGTHS(X) X(96) X(128) X(192) X(256) X(384) X(512)
+// Line lengths 2 nz of the three-pass schedule (longer z lines leave the z pass without
+// registers for its next rows).
 #define SOPHT_ZROW_LENGTHS(X) \
   X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384) X(512)
 
@@ -1195,64 +744,6 @@ bool zrow_length_supported(int64_t L) {
   SOPHT_ZROW_LENGTHS(X)
 #undef X
   return false;
-}
-
-bool xy_length_supported(int64_t L) {
-#define X(n) if (L == n) return true;
-  SOPHT_XY_LENGTHS(X)
-#undef X
-  return false;
-}
-
-// Workgroups above 64 KB of LDS declare it once per kernel.
-template <typename K>
-int allow_lds(K* kernel, size_t bytes) {
-  if (bytes <= 65536) return SOPHT_OK;
-  SOPHT_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)));
-  return SOPHT_OK;
-}
-
-template <typename T>
-int launch_xy_fwd(int64_t L, SlabGeom g, CompPtrs in, Cplx<T>* H, const Cplx<T>* twx,
-                  const Cplx<T>* twy, hipStream_t s) {
-  const unsigned blocks = unsigned(int64_t(g.ncomp) * g.nz * 4);
-#define X(n)                                                                          \
-  if (L == n) {                                                                       \
-    using F = XYPass<T, n, n>;                                                        \
-    static const int lds_ok = allow_lds(ka_xy_fwd<T, n, n>, F::lds);                  \
-    if (lds_ok) return lds_ok;                                                        \
-    ka_xy_fwd<T, n, n><<<blocks, F::NT, F::lds, s>>>(g, in, H, twx, twy);             \
-    SOPHT_CHECK_LAUNCH();                                                             \
-    return SOPHT_OK;                                                                  \
-  }
-  SOPHT_XY_LENGTHS(X)
-#undef X
-  return SOPHT_ERR_UNSUPPORTED;
-}
-
-template <typename T>
-int launch_yx_inv(int64_t L, SlabGeom g, const Cplx<T>* H, CompPtrsW out, const Cplx<T>* twx,
-                  const Cplx<T>* twy, hipStream_t s, bool acc) {
-  const unsigned blocks = unsigned(int64_t(g.ncomp) * g.nz * 4);
-#define X(n)                                                                          \
-  if (L == n) {                                                                       \
-    using F = XYPass<T, n, n>;                                                        \
-    if (acc) {                                                                        \
-      static const int lds_ok = allow_lds(kc_yx_inv<T, n, n, true>, F::lds);          \
-      if (lds_ok) return lds_ok;                                                      \
-      kc_yx_inv<T, n, n, true><<<blocks, F::NT, F::lds, s>>>(g, H, out, twx, twy);    \
-    } else {                                                                          \
-      static const int lds_ok = allow_lds(kc_yx_inv<T, n, n, false>, F::lds);         \
-      if (lds_ok) return lds_ok;                                                      \
-      kc_yx_inv<T, n, n, false><<<blocks, F::NT, F::lds, s>>>(g, H, out, twx, twy);   \
-    }                                                                                 \
-    SOPHT_CHECK_LAUNCH();                                                             \
-    return SOPHT_OK;                                                                  \
-  }
-  SOPHT_XY_LENGTHS(X)
-#undef X
-  return SOPHT_ERR_UNSUPPORTED;
 }
 
 template <typename T>
@@ -1312,12 +803,13 @@ int solve_impl(sopht_poisson3d* P, int ncomp, void* const sol[3], const int64_t*
   };
   if constexpr (sizeof(T) == 4) {  // the three-pass kernels are built for FP32
     if (P->passes == 3) {
-      if ((rc = launch_xy_fwd<T>(2 * P->nx, g, in, H, twx, twy, s))) return rc;
+      if ((rc = poisson_xy_fwd(2 * P->nx, 2 * P->ny, g, in, H, twx, twy, s))) return rc;
       mark(0);
       if ((rc = launch_k3_rows<T>(2 * P->nz, g, H, static_cast<const T*>(P->ghat), twz, s, P->zjobs)))
         return rc;
       mark(1);
-      rc = launch_yx_inv<T>(2 * P->nx, g, H, out, twx, twy, s, accumulate);
+      rc = accumulate ? poisson_yx_inv_add(2 * P->nx, 2 * P->ny, g, H, out, twx, twy, s)
+                      : poisson_yx_inv(2 * P->nx, 2 * P->ny, g, H, out, twx, twy, s);
       mark(2);
       return rc;
     }
@@ -1524,12 +1016,14 @@ int poisson_create(int dtype, int64_t nz, int64_t ny, int64_t nx, double x_range
     return SOPHT_ERR_UNSUPPORTED;
   }
   P->ghat_bytes = (ny + 1) * (nx + 1) * P->gz * int64_t(rsz);
-  // the three-pass schedule where its kernels are built (FP32, nx = ny, 2 nx in
+  // the three-pass schedule where its kernels are built (FP32, 2 nx and 2 ny in
   // SOPHT_XY_LENGTHS, 2 nz in SOPHT_ZROW_LENGTHS); SOPHT_POISSON_PASSES=5 in the environment
-  // keeps the five-pass one
+  // keeps the five-pass one. Per vector solve it was never slower at any pair of lengths
+  // (five / three passes, ms): 48^3 0.053 / 0.038; nz, ny, nx = 128, 96, 192 0.211 / 0.180;
+  // 48, 128, 256 0.171 / 0.153; 256, 128, 256 0.670 / 0.573; 256, 192, 256 1.10 / 0.98
   const char* forced = std::getenv("SOPHT_POISSON_PASSES");
   const bool five = forced != nullptr && std::atoi(forced) == 5;
-  P->passes = (!five && kRowPad && dtype == SOPHT_F32 && nx == ny && xy_length_supported(2 * nx) &&
+  P->passes = (!five && kRowPad && dtype == SOPHT_F32 && xy_length_supported(2 * nx) && xy_length_supported(2 * ny) &&
                zrow_length_supported(2 * nz)) ? 3 : 5;
   int rc = SOPHT_OK;
   auto fail = [&](int code) {

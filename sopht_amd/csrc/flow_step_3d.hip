@@ -425,12 +425,12 @@ int sopht_ns3d_max_abs_velocity_sum(sopht_ns3d* P, const void* vel, void* out, v
     k_max_abs_sum<float><<<nb, 256, 0, s>>>(static_cast<const float*>(vel), n,
                                            static_cast<float*>(P->partial));
     SOPHT_CHECK_LAUNCH();
-    k_max_final<float><<<1, 256, 0, s>>>(static_cast<const float*>(P->partial), nb, static_cast<float*>(out));
+    k_max_final<float><<<1, 1024, 0, s>>>(static_cast<const float*>(P->partial), nb, static_cast<float*>(out));
   } else {
     k_max_abs_sum<double><<<nb, 256, 0, s>>>(static_cast<const double*>(vel), n,
                                             static_cast<double*>(P->partial));
     SOPHT_CHECK_LAUNCH();
-    k_max_final<double><<<1, 256, 0, s>>>(static_cast<const double*>(P->partial), nb, static_cast<double*>(out));
+    k_max_final<double><<<1, 1024, 0, s>>>(static_cast<const double*>(P->partial), nb, static_cast<double*>(out));
   }
   SOPHT_CHECK_LAUNCH();
   return SOPHT_OK;
@@ -451,9 +451,9 @@ int sopht_ns3d_last_velocity_max(sopht_ns3d* P, const void* vel, void* out, void
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int nb = int(P->s2_partials);
   if (P->dtype == SOPHT_F32)
-    k_max_final<float><<<1, 256, 0, s>>>(static_cast<const float*>(P->s2max), nb, static_cast<float*>(out));
+    k_max_final<float><<<1, 1024, 0, s>>>(static_cast<const float*>(P->s2max), nb, static_cast<float*>(out));
   else
-    k_max_final<double><<<1, 256, 0, s>>>(static_cast<const double*>(P->s2max), nb, static_cast<double*>(out));
+    k_max_final<double><<<1, 1024, 0, s>>>(static_cast<const double*>(P->s2max), nb, static_cast<double*>(out));
   SOPHT_CHECK_LAUNCH();
   return SOPHT_OK;
 }

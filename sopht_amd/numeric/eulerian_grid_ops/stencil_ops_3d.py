@@ -9,6 +9,8 @@ and ``fixed_grid_size`` are accepted and ignored, as in the reference (its
 
 from __future__ import annotations
 
+import functools
+
 from collections.abc import Callable
 
 import numpy as np
@@ -554,25 +556,21 @@ def gen_advection_flux_conservative_eno3_adjoint_kernel_3d(real_t: type) -> Call
     return advection_flux_conservative_eno3_adjoint_kernel_3d
 
 
-def eno3_advection_flux(field, velocity, inv_dx: float):
-    """Differentiable ENO3 conservative advection flux (a ``torch.autograd.Function``).
-
-    Returns a new flux field: zero outside ``[2:-2]^3`` and the reference's ENO3 flux inside.
-    The backward runs the transpose kernel with the forward's stencil choices (they depend
-    on ``velocity`` only), so gradients flow to both ``field`` and ``velocity``; the switch
-    itself is piecewise constant and contributes nothing."""
+@functools.cache
+def _eno3_flux_function():
+    """The ``torch.autograd.Function`` of :func:`eno3_advection_flux` (built on first use, so
+    that importing this module does not import torch)."""
     import torch
-
-    real_t = np.float32 if field.dtype == torch.float32 else np.float64
-    tag = L.dtype_tag(real_t)
 
     class _ENO3Flux(torch.autograd.Function):
         @staticmethod
-        def forward(ctx, f, u):
+        def forward(ctx, f, u, inv_dx):
             f, u = f.contiguous(), u.contiguous()
             flux = torch.empty_like(f)
             nz, ny, nx = _shape3(f)
-            L.call("sopht_advection_flux_conservative_eno3_set_3d", tag, L.ptr(flux), L.strides3(flux),
+            ctx.tag = L.SOPHT_F32 if f.dtype == torch.float32 else L.SOPHT_F64
+            ctx.inv_dx = inv_dx
+            L.call("sopht_advection_flux_conservative_eno3_set_3d", ctx.tag, L.ptr(flux), L.strides3(flux),
                    L.ptr(f), L.strides3(f), L.comps(u), L.strides3(u[0]), nz, ny, nx, float(inv_dx),
                    L.stream_ptr())
             ctx.save_for_backward(f, u)
@@ -585,11 +583,21 @@ def eno3_advection_flux(field, velocity, inv_dx: float):
             gf = torch.empty_like(f) if ctx.needs_input_grad[0] else None
             gu = torch.empty_like(u) if ctx.needs_input_grad[1] else None
             if gf is not None or gu is not None:
-                _eno3_adjoint("sopht_advection_flux_conservative_eno3_adjoint_set_3d", tag, gf, gu, grad_flux, f, u,
-                              inv_dx)
-            return gf, gu
+                _eno3_adjoint("sopht_advection_flux_conservative_eno3_adjoint_set_3d", ctx.tag, gf, gu, grad_flux, f, u,
+                              ctx.inv_dx)
+            return gf, gu, None
 
-    return _ENO3Flux.apply(field, velocity)
+    return _ENO3Flux
+
+
+def eno3_advection_flux(field, velocity, inv_dx: float):
+    """Differentiable ENO3 conservative advection flux (a ``torch.autograd.Function``).
+
+    Returns a new flux field: zero outside ``[2:-2]^3`` and the reference's ENO3 flux inside.
+    The backward runs the transpose kernel with the forward's stencil choices (they depend
+    on ``velocity`` only), so gradients flow to both ``field`` and ``velocity``; the switch
+    itself is piecewise constant and contributes nothing."""
+    return _eno3_flux_function().apply(field, velocity, inv_dx)
 
 
 def gen_advection_timestep_euler_forward_conservative_eno3_pyst_kernel_3d(

@@ -132,7 +132,7 @@ class UnboundedNavierStokesFlowSimulator3D(FlowSimulator):
         self.stream_func_field = torch.zeros_like(self.vorticity_field)
         if self.with_forcing:
             self.eul_grid_forcing_field = torch.zeros_like(self.velocity_field)
-        self._max_out = torch.zeros((), dtype=tdt, device=self._device)
+        self._max_out = L.HostScalar(tdt)
 
     # :328-440
     def _compile_kernels(self):
@@ -246,11 +246,11 @@ class UnboundedNavierStokesFlowSimulator3D(FlowSimulator):
         rc = -1
         if getattr(self, "_velocity_version", None) == self.velocity_field._version:
             rc = lib.sopht_ns3d_last_velocity_max(self._plan, L.ptr(self.velocity_field),
-                                                  L.ptr(self._max_out), L.stream_ptr())
+                                                  self._max_out.arm(), L.stream_ptr())
         if rc != 0:
             L.call("sopht_ns3d_max_abs_velocity_sum", self._plan, L.ptr(self.velocity_field),
-                   L.ptr(self._max_out), L.stream_ptr())
-        return self.real_t(self._max_out.item())
+                   self._max_out.arm(), L.stream_ptr())
+        return self.real_t(self._max_out.read())
 
     def _stable_timestep_from_max(self, vmax):
         """``passive_transport_flow_simulators.py:139-155`` given the velocity maximum."""

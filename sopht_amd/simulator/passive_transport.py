@@ -63,7 +63,7 @@ class PassiveTransportFlowSimulator(FlowSimulator):
         # the advected field, one scratch field per component
         self._next = make(self._ncomp, *comp_shape)
         self._partials = make(_PARTIALS)
-        self._vmax = make(1)
+        self._vmax = L.HostScalar(L.torch_dtype(self.real_t))
 
     def _compile_kernels(self):
         # nothing to generate: the step is one library entry point, bound here
@@ -119,13 +119,13 @@ def compute_advection_diffusion_stable_timestep(
         raise ValueError(msg)
     if _scratch is None:
         _scratch = (torch.empty(_PARTIALS, dtype=v.dtype, device=v.device),
-                    torch.empty(1, dtype=v.dtype, device=v.device))
+                    L.HostScalar(v.dtype))
     partials, vmax = _scratch
     n = velocity_magnitude_field.numel()
     L.call("sopht_velocity_abs_sum_max_3d", L.dtype_tag(real_t), L.comps(v), n, L.ptr(velocity_magnitude_field),
-           L.ptr(partials), int(partials.numel()), L.ptr(vmax), L.stream_ptr())
+           L.ptr(partials), int(partials.numel()), vmax.arm(), L.stream_ptr())
     L.written(velocity_magnitude_field)
     tol = 10 * np.finfo(real_t).eps
-    advective = cfl * dx / (real_t(vmax.item()) + tol)
+    advective = cfl * dx / (real_t(vmax.read()) + tol)
     diffusive = 0.9 * dx**2 / (2 * grid_dim) / kinematic_viscosity + tol
     return min(advective, diffusive)

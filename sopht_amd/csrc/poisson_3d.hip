@@ -23,6 +23,7 @@
 #include "common.h"
 #include "fft_reg.h"
 #include "poisson_xy.h"
+#include "poisson_z.h"
 
 struct sopht_poisson3d {
   int dtype;
@@ -31,6 +32,7 @@ struct sopht_poisson3d {
   void* slab;       // complex slab, 3 components
   void* ghat;       // real octant
   void* tw[3];      // twiddles for lengths 2nx, 2ny, 2nz (x, y, z)
+  int64_t rs;       // slab row stride (complex elements)
   int64_t gz;       // G^ line stride (elements): nz + 1 rounded up to a 128-byte line
   int slab_comps;   // components the slab holds (3, or 3 per instance of a batched class)
   int64_t slab_bytes, ghat_bytes;
@@ -172,36 +174,8 @@ __global__ void __launch_bounds__((ColTile<T, L>::NT)) k_ycols(SlabGeom g, Cplx<
     });
 }
 
-// Waves per SIMD the z pass is compiled for (its VGPR budget: 128 in FP32; a budget of 80,
-// for three 512-thread workgroups per CU, spills).
-template <typename T>
-constexpr int kZconvWaves = sizeof(T) == 4 ? 4 : 2;
-// more elements per thread need more registers: twelve (L = 384, 768) one wavefront less per
-// SIMD, sixteen (L = 1024) two less
-template <typename T, int L>
-constexpr int kZconvWavesFor = sizeof(T) != 4 ? kZconvWaves<T>
-                               : (LinePlan<L>::E >= 16 ? 2 : (LinePlan<L>::E > 8 ? 3 : kZconvWaves<T>));
 // pencil tiles per z-pass workgroup at most (all of them for a 3-component solve)
 constexpr int kZconvJobs = 6;
-
-// Three-stage line plans: the twiddles of a thread's butterflies in the second and last stages
-// depend on the thread only, so a z-pass workgroup computes them once for all its pencils.
-template <typename R>
-struct Plan3 {
-  static constexpr bool ok = false;
-  static constexpr int r0 = 0, r1 = 0, r2 = 0;
-};
-template <int A, int B, int C>
-struct Plan3<rfft::Radices<A, B, C>> {
-  static constexpr bool ok = true;
-  static constexpr int r0 = A, r1 = B, r2 = C;
-};
-template <int L>
-constexpr bool last_twiddles_hoisted() {  // the E = 8 plans (L = 128, 256, 512): 24-28 VGPRs
-  using P = Plan3<typename LinePlan<L>::R>;
-  return P::ok && LinePlan<L>::E == 8;
-}
-constexpr int at_least_1(int v) { return v > 0 ? v : 1; }
 
 // K3: z pencils (c, ky, kx): zero-padded forward FFT, times G^ (real, even), inverse FFT,
 // crop to z < nz. A workgroup owns one kx tile of one |ky| = kyo and runs the pencils of
@@ -388,228 +362,6 @@ __global__ void __launch_bounds__((RowTile<T, L>::NT)) k5_xc2r(SlabGeom g, const
   });
 }
 
-// Build-time choices of the three-pass z pass (measured: ordinary stores beat streaming ones
-// there, quarter-line tiles beat half-line ones, six jobs per workgroup beat two or three).
-#ifndef SOPHT_ZROW_STREAM
-#define SOPHT_ZROW_STREAM 0
-#endif
-#ifndef SOPHT_ZROW_PARTS
-#define SOPHT_ZROW_PARTS 4
-#endif
-#ifndef SOPHT_ZROW_JOBS
-#define SOPHT_ZROW_JOBS 6
-#endif
-#ifndef SOPHT_ZROW_SLOTS
-#define SOPHT_ZROW_SLOTS 2
-#endif
-#ifndef SOPHT_ZROW_PREFETCH
-#define SOPHT_ZROW_PREFETCH 1
-#endif
-constexpr bool kZrowStream = SOPHT_ZROW_STREAM;
-constexpr bool kZrowPrefetch = SOPHT_ZROW_PREFETCH;
-constexpr int kZrowJobs = SOPHT_ZROW_JOBS;
-
-// The z pass of the three-pass schedule. A workgroup owns one kx tile (WC columns) of the row
-// class k2 (slab rows y1 L2 + k2, y1 < 4) and of its mirror class L2 - k2. Per job (component,
-// class) the four rows are loaded, the 4-point DFT over y1 gives the pencils ky = k2 + L2 k1,
-// each pencil is convolved along z as in k3_zconv, and the inverse 4-point DFT returns the rows.
-// The workgroup has two teams per column and transforms two pencils at a time (two LDS tiles),
-// so a thread holds E / 4 values of each row: the next job's rows are loaded during the
-// transforms within 128 VGPRs. The G^ lines of the class, |k2 + L2 k1| folded to <= ny for
-// k1 < 4, are staged in LDS once per workgroup. Slot s of a column takes pencil k1 = s + 2r in
-// round r of a job, and so G^ line s + 2r; in a mirror job it takes pencil 3 - s - 2r, whose
-// ky' = L2 - k2 + L2 (3 - s - 2r) has the line of 2 ny - ky' = k2 + L2 (s + 2r): the same.
-template <typename T, int L>
-struct ZRowTile {
-  static constexpr int E = LinePlan<L>::E, TT = LinePlan<L>::T;
-  // a quarter of a 128-byte line per workgroup (two workgroups per CU); the four quarters of a
-  // line go to workgroups b, b + 8, b + 16, b + 24 (the same XCD), so three come from its L2
-  static constexpr int PARTS = SOPHT_ZROW_PARTS;
-  static constexpr int SLOTS = SOPHT_ZROW_SLOTS;  // pencils per column transformed at once
-  static constexpr int WC = kLineCplx<T> / PARTS;
-  static constexpr int NT = SLOTS * WC * TT;
-  // tiles [slot][column]: the load role's lanes (column, z) hit distinct banks when the
-  // column stride is 8 (mod 32) slots
-  static constexpr int S = TT < 32 ? L + 16 : (WC == 4 ? L + 8 : L + 4);
-  static constexpr int KL = E / (2 * SLOTS);  // z values per row per thread (z = lr + SLOTS TT k)
-  static constexpr int GL = L / 2 + 1;
-  static constexpr size_t lds = size_t(SLOTS * WC * S) * sizeof(Cplx<T>) + size_t(4 * WC * GL) * sizeof(T);
-  static_assert(E % (2 * SLOTS) == 0 && 4 % SLOTS == 0, "the z rows split among the slots");
-};
-
-template <typename T, int L>
-__global__ void __launch_bounds__((ZRowTile<T, L>::NT)) __attribute__((amdgpu_waves_per_eu(kZconvWavesFor<T, L>))) k3_zconv4(SlabGeom g, Cplx<T>* H, const T* ghat,
-                                                                  const Cplx<T>* tw, int jobs) {
-  using ZT = ZRowTile<T, L>;
-  constexpr int E = ZT::E, TT = ZT::TT, WC = ZT::WC, S = ZT::S, KL = ZT::KL, GL = ZT::GL;
-  constexpr int SL = ZT::SLOTS, ZSTEP = SL * TT;
-  extern __shared__ unsigned char smem_raw[];
-  Cplx<T>* xb = reinterpret_cast<Cplx<T>*>(smem_raw);  // tiles [slot][column][z]
-  T* const gl = reinterpret_cast<T*>(xb + SL * WC * S);  // G^ lines [k1][column][kz]
-  const int tid = threadIdx.x;
-  const int lw = tid % WC, lr = tid / WC;  // load role: column, first z
-  const int team = tid / TT, t = tid % TT;  // transform role: team = slot * WC + column
-  const int tcol = team % WC, slot = team / WC;
-  const int64_t ncols = g.nx + 1;
-  const int L2 = int(g.ny) / 2;
-  int64_t k2, kx0;
-  if (!col_tile_parts<ZT::PARTS>(blockIdx.x, ncols, L2 / 2 + 1, WC, k2, kx0)) return;
-  const bool self = k2 == 0 || 2 * k2 == L2;
-  const int alljobs = self ? g.ncomp : 2 * g.ncomp;
-  const int jbeg = int(blockIdx.y) * jobs;
-  if (jbeg >= alljobs) return;
-  const int njobs = alljobs - jbeg < jobs ? alljobs - jbeg : jobs;
-  const int64_t kx = kx0 + lw;
-  const bool live = kx < ncols;
-  const int first_col = 64 / TT >= WC ? 0 : ((tid / 64) * (64 / TT)) % WC;
-  const bool wave_live = kx0 + first_col < ncols;
-  {
-    // every load in flight before the first LDS write (a loop would wait on each in turn)
-    constexpr int NG = 4 * WC * GL, NIT = (NG + ZT::NT - 1) / ZT::NT;
-    T gt[NIT];
-    static_for<0, NIT>([&](auto i_) {
-      constexpr int it = decltype(i_)::value;
-      const int i = tid + it * ZT::NT;
-      const int kz = i % GL, rest = i / GL;
-      const int w = rest % WC, k1 = (rest / WC) & 3;
-      const int ky = int(k2) + L2 * k1;
-      const int kyo = ky <= int(g.ny) ? ky : 2 * int(g.ny) - ky;
-      const int kxt = kx0 + w < ncols ? int(kx0) + w : 0;
-      gt[it] = (it + 1 < NIT || i < NG) ? ghat[(kyo * int(ncols) + kxt) * int(g.gz) + kz] : T(0);
-    });
-    static_for<0, NIT>([&](auto i_) {
-      constexpr int it = decltype(i_)::value;
-      const int i = tid + it * ZT::NT;
-      if (it + 1 < NIT || i < NG) gl[i] = gt[it];
-    });
-  }
-  constexpr int zs = kSlabTile;  // consecutive z of a column tile (ti layout)
-  using P3 = Plan3<typename LinePlan<L>::R>;
-  constexpr int R1 = at_least_1(P3::r1), R2 = at_least_1(P3::r2);
-  constexpr int PER2 = at_least_1(E / R1), PER3 = at_least_1(E / R2);
-  Cplx<T> w2[PER2][R1], w3[PER3][R2];
-  if constexpr (last_twiddles_hoisted<L>()) {
-    static_for<0, PER2>([&](auto p_) {
-      constexpr int p = decltype(p_)::value;
-      rfft::stage_twiddles<T, L, R1, P3::r0>(w2[p], tw, (t + p * TT) % P3::r0);
-    });
-    static_for<0, PER3>([&](auto p_) {
-      constexpr int p = decltype(p_)::value;
-      rfft::stage_twiddles<T, L, R2, P3::r0 * R1>(w3[p], tw, (t + p * TT) % (P3::r0 * R1));
-    });
-  }
-  auto row_col = [&](int jl, int y1) -> int {
-    const int j = jbeg + jl;
-    const int cc = j % g.ncomp;
-    const int cls = j < g.ncomp ? int(k2) : L2 - int(k2);
-    return g.ti(cc, 0, y1 * L2 + cls, live ? int(kx) : 0);
-  };
-  Cplx<T> pf[4][KL];
-  auto load = [&](int j) {
-    static_for<0, 4>([&](auto y_) {
-      constexpr int y1 = decltype(y_)::value;
-      const int colp = row_col(j, y1);
-      static_for<0, KL>([&](auto k_) {
-        constexpr int k = decltype(k_)::value;
-        pf[y1][k] = live ? H[colp + (lr + ZSTEP * k) * zs] : Cplx<T>{T(0), T(0)};
-      });
-    });
-  };
-  Cplx<T>* const line = xb + team * S;
-  if constexpr (kZrowPrefetch) load(0);
-  __syncthreads();  // G^ lines staged
-  for (int j = 0; j < njobs; ++j) {
-    const bool mirror = jbeg + j >= g.ncomp;
-    if constexpr (!kZrowPrefetch) load(j);
-    Cplx<T> y[4][KL];
-    static_for<0, KL>([&](auto k_) {
-      constexpr int k = decltype(k_)::value;
-      Cplx<T> u[4] = {pf[0][k], pf[1][k], pf[2][k], pf[3][k]};
-      rfft::dft4<T, false>(u);
-      static_for<0, 4>([&](auto q_) { y[decltype(q_)::value][k] = u[decltype(q_)::value]; });
-    });
-    if constexpr (kZrowPrefetch) {
-      if (j + 1 < njobs) load(j + 1);
-    }
-    static_for<0, 4 / SL>([&](auto r_) {
-      constexpr int r = decltype(r_)::value;
-      // slot sl takes pencil sl + SL r (a mirror job: 3 - sl - SL r)
-      static_for<0, SL>([&](auto s_) {
-        constexpr int sl = decltype(s_)::value;
-        static_for<0, KL>([&](auto k_) {
-          constexpr int k = decltype(k_)::value;
-          // selects on values (a select of two array elements' addresses would leave y in
-          // scratch memory)
-          const Cplx<T> a = y[3 - sl - SL * r][k], b = y[sl + SL * r][k];
-          xb[(sl * WC + lw) * S + lr + ZSTEP * k] = Cplx<T>{mirror ? a.re : b.re, mirror ? a.im : b.im};
-        });
-      });
-      __syncthreads();
-      Cplx<T> v[E];
-      static_for<0, E>([&](auto e_) {
-        constexpr int e = decltype(e_)::value;
-        if constexpr (e < E / 2) v[e] = line[t + TT * e];
-        else v[e] = Cplx<T>{T(0), T(0)};
-      });
-      rfft::wave_sync();
-      if (wave_live) {
-        const T* const gq = gl + ((slot + SL * r) * WC + tcol) * GL;
-        if constexpr (last_twiddles_hoisted<L>()) {
-          constexpr int R0 = P3::r0, NS3 = R0 * R1;
-          rfft::stockham_stage<T, L, R0, 1, false, true>(v, line, tw, t);
-          rfft::stockham_stage_given<T, L, R1, R0, false>(v, line, w2, t);
-          rfft::stockham_stage_given<T, L, R2, NS3, false>(v, line, w3, t);
-        } else {
-          rfft::team_fft<T, L, false, true>(v, line, tw, t);
-        }
-        static_for<0, E>([&](auto e_) {
-          constexpr int e = decltype(e_)::value;
-          const int kz = t + TT * e;
-          const T gv = gq[kz <= L / 2 ? kz : L - kz];
-          v[e] = Cplx<T>{v[e].re * gv, v[e].im * gv};
-        });
-        if constexpr (last_twiddles_hoisted<L>()) {
-          constexpr int R0 = P3::r0, NS3 = R0 * R1;
-          rfft::stockham_stage<T, L, R0, 1, true, false>(v, line, tw, t);
-          rfft::stockham_stage_given<T, L, R1, R0, true>(v, line, w2, t);
-          rfft::stockham_stage_given<T, L, R2, NS3, true>(v, line, w3, t);
-        } else {
-          rfft::team_fft<T, L, true>(v, line, tw, t);
-        }
-      }
-      static_for<0, E / 2>([&](auto e_) {
-        constexpr int e = decltype(e_)::value;
-        line[t + TT * e] = v[e];
-      });
-      __syncthreads();
-      static_for<0, SL>([&](auto s_) {
-        constexpr int sl = decltype(s_)::value;
-        static_for<0, KL>([&](auto k_) {
-          constexpr int k = decltype(k_)::value;
-          const Cplx<T> val = xb[(sl * WC + lw) * S + lr + ZSTEP * k];
-          Cplx<T>& a = y[3 - sl - SL * r][k];
-          Cplx<T>& b = y[sl + SL * r][k];
-          a = Cplx<T>{mirror ? val.re : a.re, mirror ? val.im : a.im};
-          b = Cplx<T>{mirror ? b.re : val.re, mirror ? b.im : val.im};
-        });
-      });
-      __syncthreads();
-    });
-    if (live) {
-      static_for<0, KL>([&](auto k_) {
-        constexpr int k = decltype(k_)::value;
-        Cplx<T> u[4] = {y[0][k], y[1][k], y[2][k], y[3][k]};
-        rfft::dft4<T, true>(u);
-        static_for<0, 4>([&](auto q_) {
-          constexpr int y1 = decltype(q_)::value;
-          if constexpr (kZrowStream) store_stream(H + row_col(j, y1) + (lr + ZSTEP * k) * zs, u[y1]);
-          else H[row_col(j, y1) + (lr + ZSTEP * k) * zs] = u[y1];
-        });
-      });
-    }
-  }
-}
-
 // ------------------------------------------------------------------ Green's function octant
 // g[z][y][x] = 1/(4 pi r dx) on integer offsets, g[0] = 1/(4 pi dx), in FP64.
 __global__ void k_green_octant(double* g, int64_t nz1, int64_t ny1, int64_t nx1, double dx) {
@@ -734,41 +486,8 @@ int launch_k5(int64_t L, SlabGeom g, const Cplx<T>* H, CompPtrsW out, const Cplx
   return SOPHT_ERR_UNSUPPORTED;
 }
 
-// Line lengths 2 nz of the three-pass schedule (longer z lines leave the z pass without
-// registers for its next rows).
-#define SOPHT_ZROW_LENGTHS(X) \
-  X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384) X(512)
-
-bool zrow_length_supported(int64_t L) {
-#define X(n) if (L == n) return true;
-  SOPHT_ZROW_LENGTHS(X)
-#undef X
-  return false;
-}
-
-template <typename T>
-int launch_k3_rows(int64_t L, SlabGeom g, Cplx<T>* H, const T* ghat, const Cplx<T>* tw,
-                   hipStream_t s, int jobs) {
-#define X(n)                                                                          \
-  if (L == n) {                                                                       \
-    using ZT = ZRowTile<T, n>;                                                        \
-    const int64_t nb = col_tile_parts_blocks(ZT::PARTS, g.nx + 1, g.ny / 4 + 1, ZT::WC); \
-    const unsigned nch = unsigned((2 * g.ncomp + jobs - 1) / jobs);                    \
-    static const int lds_ok = allow_lds(k3_zconv4<T, n>, ZT::lds);                    \
-    if (lds_ok) return lds_ok;                                                        \
-    k3_zconv4<T, n><<<dim3(unsigned(nb), nch), ZT::NT, ZT::lds, s>>>(g, H, ghat, tw, jobs); \
-    SOPHT_CHECK_LAUNCH();                                                             \
-    return SOPHT_OK;                                                                  \
-  }
-  SOPHT_ZROW_LENGTHS(X)
-#undef X
-  return SOPHT_ERR_UNSUPPORTED;
-}
-
-template <typename T>
 SlabGeom slab_geom(const sopht_poisson3d* P, int ncomp) {
-  return SlabGeom{P->nz, P->ny, P->nx, kRowPad ? round_up(P->nx + 1, kLineCplx<T>) : P->nx + 1,
-                  P->gz, ncomp};
+  return SlabGeom{P->nz, P->ny, P->nx, P->rs, P->gz, ncomp};
 }
 
 // ncomp <= 3 components by value (sol, rhs), or any number from device pointer tables
@@ -782,7 +501,7 @@ int solve_impl(sopht_poisson3d* P, int ncomp, void* const sol[3], const int64_t*
     set_last_error("more components than the Poisson plan's slab holds", __FILE__, __LINE__);
     return SOPHT_ERR_INVALID;
   }
-  const SlabGeom g = slab_geom<T>(P, ncomp);
+  const SlabGeom g = slab_geom(P, ncomp);
   CompPtrs in;
   CompPtrsW out;
   in.tab = rhs_tab;
@@ -801,18 +520,15 @@ int solve_impl(sopht_poisson3d* P, int ncomp, void* const sol[3], const int64_t*
   auto mark = [&](int i) {
     if (timer) timer->mark(first_stage + i, s);
   };
-  if constexpr (sizeof(T) == 4) {  // the three-pass kernels are built for FP32
-    if (P->passes == 3) {
-      if ((rc = poisson_xy_fwd(2 * P->nx, 2 * P->ny, g, in, H, twx, twy, s))) return rc;
-      mark(0);
-      if ((rc = launch_k3_rows<T>(2 * P->nz, g, H, static_cast<const T*>(P->ghat), twz, s, P->zjobs)))
-        return rc;
-      mark(1);
-      rc = accumulate ? poisson_yx_inv_add(2 * P->nx, 2 * P->ny, g, H, out, twx, twy, s)
-                      : poisson_yx_inv(2 * P->nx, 2 * P->ny, g, H, out, twx, twy, s);
-      mark(2);
-      return rc;
-    }
+  if (P->passes == 3) {
+    if ((rc = poisson_xy_fwd(2 * P->nx, 2 * P->ny, g, in, H, twx, twy, s))) return rc;
+    mark(0);
+    if ((rc = poisson_z_rows(2 * P->nz, g, H, static_cast<const T*>(P->ghat), twz, s, P->zjobs))) return rc;
+    mark(1);
+    rc = accumulate ? poisson_yx_inv_add(2 * P->nx, 2 * P->ny, g, H, out, twx, twy, s)
+                    : poisson_yx_inv(2 * P->nx, 2 * P->ny, g, H, out, twx, twy, s);
+    mark(2);
+    return rc;
   }
   if ((rc = launch_k1<T>(2 * P->nx, g, in, H, twx, s))) return rc;
   mark(0);
@@ -899,18 +615,19 @@ int build_ghat(sopht_poisson3d* P, hipStream_t s) {
 // G^ staging). Each candidate is timed on the plan's own slab (zeroed) and stream, and the
 // fastest kept; SOPHT_POISSON_ZJOBS in the environment fixes the choice instead. Results do
 // not depend on it: a pencil's arithmetic is the same in any workgroup.
+template <typename T>
 int tune_zpass(sopht_poisson3d* P, hipStream_t s) {
   P->zjobs = kZrowJobs;
-  if (P->passes != 3 || P->dtype != SOPHT_F32) return SOPHT_OK;
+  if (P->passes != 3) return SOPHT_OK;
   if (const char* forced = std::getenv("SOPHT_POISSON_ZJOBS")) {
     const int j = std::atoi(forced);
     if (j >= 1) P->zjobs = j;
     return SOPHT_OK;
   }
-  const SlabGeom g = slab_geom<float>(P, P->slab_comps);
-  Cplx<float>* H = static_cast<Cplx<float>*>(P->slab);
-  const float* gh = static_cast<const float*>(P->ghat);
-  const Cplx<float>* twz = static_cast<const Cplx<float>*>(P->tw[2]);
+  const SlabGeom g = slab_geom(P, P->slab_comps);
+  Cplx<T>* H = static_cast<Cplx<T>*>(P->slab);
+  const T* gh = static_cast<const T*>(P->ghat);
+  const Cplx<T>* twz = static_cast<const Cplx<T>*>(P->tw[2]);
   SOPHT_CHECK_HIP(hipMemsetAsync(P->slab, 0, size_t(P->slab_bytes), s));
   hipEvent_t e0 = nullptr, e1 = nullptr;
   SOPHT_CHECK_HIP(hipEventCreate(&e0));
@@ -923,9 +640,9 @@ int tune_zpass(sopht_poisson3d* P, hipStream_t s) {
   float best = -1.f;
   for (const int jobs : {1, 2, 3, 6}) {
     if (jobs > 2 * g.ncomp) continue;
-    if ((rc = launch_k3_rows<float>(2 * P->nz, g, H, gh, twz, s, jobs))) break;  // warm-up
+    if ((rc = poisson_z_rows(2 * P->nz, g, H, gh, twz, s, jobs))) break;  // warm-up
     if (hipEventRecord(e0, s) != hipSuccess) { rc = SOPHT_ERR_HIP; break; }
-    for (int r = 0; r < 3 && rc == SOPHT_OK; ++r) rc = launch_k3_rows<float>(2 * P->nz, g, H, gh, twz, s, jobs);
+    for (int r = 0; r < 3 && rc == SOPHT_OK; ++r) rc = poisson_z_rows(2 * P->nz, g, H, gh, twz, s, jobs);
     if (rc) break;
     float ms = 0.f;
     if (hipEventRecord(e1, s) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
@@ -1006,7 +723,21 @@ int poisson_create(int dtype, int64_t nz, int64_t ny, int64_t nx, double x_range
   if (dtype == SOPHT_F32) P->dx = double(float(P->dx));  // the reference's real_t(dx)
   const size_t cs = dtype == SOPHT_F32 ? sizeof(Cplx<float>) : sizeof(Cplx<double>);
   const size_t rsz = dtype == SOPHT_F32 ? sizeof(float) : sizeof(double);
-  const int64_t rs = kRowPad ? round_up(nx + 1, int64_t(128 / cs)) : nx + 1;
+  // the three-pass schedule where its kernels are built (2 nx and 2 ny in SOPHT_XY_LENGTHS of
+  // the precision, 2 nz in SOPHT_ZROW_LENGTHS); SOPHT_POISSON_PASSES=5 in the environment
+  // keeps the five-pass one. Per vector solve it was never slower at any pair of lengths
+  // (five / three passes, ms): FP32 48^3 0.053 / 0.038; nz, ny, nx = 128, 96, 192 0.211 / 0.180;
+  // 48, 128, 256 0.171 / 0.153; 256, 128, 256 0.670 / 0.573; 256, 192, 256 1.10 / 0.98; FP64
+  // 48^3 0.068 / 0.046; 64^3 0.079 / 0.057; 96^3 0.192 / 0.151; 128^3 0.330 / 0.330; 192, 128,
+  // 192 0.897 / 0.826; 192^3 1.485 / 1.194
+  const char* forced = std::getenv("SOPHT_POISSON_PASSES");
+  const bool five = forced != nullptr && std::atoi(forced) == 5;
+  P->passes = (!five && kRowPad && xy_length_supported(dtype, 2 * nx) && xy_length_supported(dtype, 2 * ny) &&
+               zrow_length_supported(2 * nz)) ? 3 : 5;
+  // whole 128-byte lines, and whole column tiles of the three-pass slab
+  const int64_t line = P->passes == 3 ? std::max<int64_t>(128 / cs, kSlabTile) : int64_t(128 / cs);
+  const int64_t rs = kRowPad ? round_up(nx + 1, line) : nx + 1;
+  P->rs = rs;
   P->gz = kRowPad ? round_up(nz + 1, int64_t(128 / rsz)) : nz + 1;
   P->slab_comps = comps;
   P->slab_bytes = int64_t(comps) * nz * 2 * ny * rs * int64_t(cs);
@@ -1016,15 +747,6 @@ int poisson_create(int dtype, int64_t nz, int64_t ny, int64_t nx, double x_range
     return SOPHT_ERR_UNSUPPORTED;
   }
   P->ghat_bytes = (ny + 1) * (nx + 1) * P->gz * int64_t(rsz);
-  // the three-pass schedule where its kernels are built (FP32, 2 nx and 2 ny in
-  // SOPHT_XY_LENGTHS, 2 nz in SOPHT_ZROW_LENGTHS); SOPHT_POISSON_PASSES=5 in the environment
-  // keeps the five-pass one. Per vector solve it was never slower at any pair of lengths
-  // (five / three passes, ms): 48^3 0.053 / 0.038; nz, ny, nx = 128, 96, 192 0.211 / 0.180;
-  // 48, 128, 256 0.171 / 0.153; 256, 128, 256 0.670 / 0.573; 256, 192, 256 1.10 / 0.98
-  const char* forced = std::getenv("SOPHT_POISSON_PASSES");
-  const bool five = forced != nullptr && std::atoi(forced) == 5;
-  P->passes = (!five && kRowPad && dtype == SOPHT_F32 && xy_length_supported(2 * nx) && xy_length_supported(2 * ny) &&
-               zrow_length_supported(2 * nz)) ? 3 : 5;
   int rc = SOPHT_OK;
   auto fail = [&](int code) {
     sopht_poisson3d_destroy(P);
@@ -1045,7 +767,8 @@ int poisson_create(int dtype, int64_t nz, int64_t ny, int64_t nx, double x_range
     if (rc) return fail(rc);
   }
   if ((rc = build_ghat(P, s))) return fail(rc);
-  if ((rc = tune_zpass(P, s))) return fail(rc);
+  rc = dtype == SOPHT_F32 ? tune_zpass<float>(P, s) : tune_zpass<double>(P, s);
+  if (rc) return fail(rc);
   *out = P;
   return SOPHT_OK;
 }

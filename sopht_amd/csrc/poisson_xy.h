@@ -1,29 +1,36 @@
 // Passes A and C of the three-pass Poisson schedule: the x and y transforms of a plane's row
-// class in one kernel. FP32 only. Built for every pair of lengths 2 nx, 2 ny below, one
-// translation unit per pass.
+// class in one kernel. Built for every pair of lengths 2 nx, 2 ny below, one translation unit
+// per pass and precision.
 #pragma once
 
 #include "poisson_slab.h"
 
-// Line lengths of x and y that have the kernels.
-#define SOPHT_XY_LENGTHS(X) X(96) X(128) X(192) X(256) X(384) X(512)
+// Line lengths of x and y that have the kernels. (FP64 lines of 512 points leave the passes
+// without registers; those plans keep five passes.)
+#define SOPHT_XY_LENGTHS_F64(X) X(96) X(128) X(192) X(256) X(384)
+#define SOPHT_XY_LENGTHS(X) SOPHT_XY_LENGTHS_F64(X) X(512)
 
 namespace sopht {
 
-inline bool xy_length_supported(int64_t L) {
+inline bool xy_length_supported(int dtype, int64_t L) {
+  if (dtype == SOPHT_F64 && L == 512) return false;
 #define X(n) if (L == n) return true;
   SOPHT_XY_LENGTHS(X)
 #undef X
   return false;
 }
 
-// Pass A: fields -> slab rows y1 L2 + k2; pass C: slab rows -> fields (acc: added).
-int poisson_xy_fwd(int64_t LX, int64_t LY, SlabGeom g, CompPtrs in, Cplx<float>* H, const Cplx<float>* twx,
-                   const Cplx<float>* twy, hipStream_t s);
-int poisson_yx_inv(int64_t LX, int64_t LY, SlabGeom g, const Cplx<float>* H, CompPtrsW out, const Cplx<float>* twx,
-                   const Cplx<float>* twy, hipStream_t s);
-int poisson_yx_inv_add(int64_t LX, int64_t LY, SlabGeom g, const Cplx<float>* H, CompPtrsW out,
-                       const Cplx<float>* twx, const Cplx<float>* twy, hipStream_t s);
+// Pass A: fields -> slab rows y1 L2 + k2; pass C: slab rows -> fields, and its adding form.
+#define SOPHT_XY_PASSES(T)                                                                             \
+  int poisson_xy_fwd(int64_t LX, int64_t LY, SlabGeom g, CompPtrs in, Cplx<T>* H, const Cplx<T>* twx,     \
+                     const Cplx<T>* twy, hipStream_t s);                                                 \
+  int poisson_yx_inv(int64_t LX, int64_t LY, SlabGeom g, const Cplx<T>* H, CompPtrsW out,                 \
+                     const Cplx<T>* twx, const Cplx<T>* twy, hipStream_t s);                             \
+  int poisson_yx_inv_add(int64_t LX, int64_t LY, SlabGeom g, const Cplx<T>* H, CompPtrsW out,             \
+                         const Cplx<T>* twx, const Cplx<T>* twy, hipStream_t s);
+SOPHT_XY_PASSES(float)
+SOPHT_XY_PASSES(double)
+#undef SOPHT_XY_PASSES
 
 namespace {
 
@@ -39,11 +46,13 @@ namespace {
 // (K1 -> K2) and the inverse y-pass outputs (K4 -> K5) of the five-pass schedule never reach
 // HBM: 24 words per cell fewer.
 
-// Elements of a thread's half spectrum per chunk of the y sums: the most, up to 128 / TX, that
-// divide EX / 2 and keep the chunk's column teams and staging rows within the workgroup.
+// Elements of a thread's half spectrum per chunk of the y sums: the most that divide EX / 2 and
+// keep the chunk's column teams and staging rows within the workgroup, for chunks of up to 64
+// columns (128 where TX = 64 would leave one element; 96 columns of a 384 x 384 FP64 plane would
+// not fit the LDS).
 constexpr int xy_chunk_elems(int EX, int TX, int T2, int NT, int L2) {
   int best = 1;
-  for (int k = 1; k == 1 || k * TX <= 128; ++k) {
+  for (int k = 1; k == 1 || k * TX <= (TX == 64 ? 128 : 64); ++k) {
     const int cw = k * TX;
     if ((EX / 2) % k == 0 && cw * T2 <= NT && NT % cw == 0 && L2 % (NT / cw) == 0) best = k;
   }
@@ -255,7 +264,12 @@ __global__ void __launch_bounds__((XYPass<T, LX, LY>::NT)) kc_yx_inv(SlabGeom g,
   const int mirror_lane = (TX - t) % TX;
   // the rows of a chunk: thread tid holds elements tid + NT q of the chunk's L2 x ncol block
   // (addresses formed per load: a hoisted row pointer costs the registers of the prefetch)
-  Cplx<T> pre[F::NQ];
+  // (kept as separate reals: FP64 pairs moved whole would stay in scratch memory)
+  T pre_re[F::NQ] = {}, pre_im[F::NQ] = {};
+  auto keep = [&](auto q_, const Cplx<T>& h) {
+    pre_re[decltype(q_)::value] = h.re;
+    pre_im[decltype(q_)::value] = h.im;
+  };
   const int hsrc = g.ti(c, z, y1 * L2 + tid / CW, tid % CW);
   const int rowel = int(g.rs) * int(g.nz);  // elements per slab row
   auto load_chunk = [&](auto ch_) {
@@ -266,9 +280,11 @@ __global__ void __launch_bounds__((XYPass<T, LX, LY>::NT)) kc_yx_inv(SlabGeom g,
       const int i = tid + q * NT;
       if constexpr (ncol == CW && CW % kSlabTile == 0) {
         // row i / CW = tid / CW + q NT / CW, column CW ch + tid % CW
-        pre[q] = H[hsrc + q * (NT / CW) * rowel + CW * ch * int(g.nz)];
-      } else {
-        if (i < L2 * ncol) pre[q] = H[g.ti(c, z, y1 * L2 + i / ncol, CW * ch + i % ncol)];
+        keep(q_, H[hsrc + q * (NT / CW) * rowel + CW * ch * int(g.nz)]);
+      } else if constexpr (q * NT < L2 * ncol) {
+        // past the block's end its last element again
+        const int k = i < L2 * ncol ? i : L2 * ncol - 1;
+        keep(q_, H[g.ti(c, z, y1 * L2 + k / ncol, CW * ch + k % ncol)]);
       }
     });
   };
@@ -281,7 +297,9 @@ __global__ void __launch_bounds__((XYPass<T, LX, LY>::NT)) kc_yx_inv(SlabGeom g,
     static_for<0, F::NQ>([&](auto q_) {
       constexpr int q = decltype(q_)::value;
       const int i = tid + q * NT;
-      if (i < L2 * ncol) U[(i / ncol) * P + i % ncol] = pre[q];
+      if constexpr (q * NT < L2 * ncol) {
+        if ((q + 1) * NT <= L2 * ncol || i < L2 * ncol) U[(i / ncol) * P + i % ncol] = Cplx<T>{pre_re[q], pre_im[q]};
+      }
     });
     if constexpr (ch + 1 < F::NCH) load_chunk(std::integral_constant<int, ch + 1>{});
     __syncthreads();  // (first chunk: the tables too)
@@ -368,19 +386,25 @@ int allow_lds(K* kernel, size_t bytes) {
   return SOPHT_OK;
 }
 
-// fn(integral_constant<LX>, integral_constant<LY>) for supported lengths.
-template <int LX, typename Fn>
+// fn(integral_constant<LX>, integral_constant<LY>) for the lengths of precision T.
+template <typename T, int LX, typename Fn>
 int with_xy_y(int64_t LY, Fn&& fn) {
 #define X(n) \
   if (LY == n) return fn(std::integral_constant<int, LX>{}, std::integral_constant<int, n>{});
-  SOPHT_XY_LENGTHS(X)
+  SOPHT_XY_LENGTHS_F64(X)
+  if constexpr (sizeof(T) == 4) {
+    X(512)
+  }
 #undef X
   return SOPHT_ERR_UNSUPPORTED;
 }
-template <typename Fn>
+template <typename T, typename Fn>
 int with_xy(int64_t LX, int64_t LY, Fn&& fn) {
-#define X(n) if (LX == n) return with_xy_y<n>(LY, fn);
-  SOPHT_XY_LENGTHS(X)
+#define X(n) if (LX == n) return with_xy_y<T, n>(LY, fn);
+  SOPHT_XY_LENGTHS_F64(X)
+  if constexpr (sizeof(T) == 4) {
+    X(512)
+  }
 #undef X
   return SOPHT_ERR_UNSUPPORTED;
 }

@@ -11,8 +11,9 @@
 // division by the eigenvalue sum, inverse transform), y columns, x rows. Along y and z two
 // neighbouring x cells are the pair, so a field is read as complex numbers as it lies.
 // Bound by memory: 10 words per cell and component. 256^3 FP32, three components: 0.385 ms (rows
-// 0.071 / 0.077, y columns 0.085 / 0.090, z 0.142) against 1.44 ms for the six dense products;
-// faster at every size from 16^3 (0.026 against 0.041 ms) to 384^3 (1.61 against 6.95 ms).
+// 0.071 / 0.076, y columns 0.078 / 0.079, z 0.134, the last by its vector instructions: two
+// transforms and the divisions) against 1.44 ms for the six dense products; faster at every size
+// from 16^3 (0.026 against 0.041 ms) to 384^3 (1.56 against 6.95 ms).
 #include <cmath>
 #include <new>
 #include <vector>
@@ -28,6 +29,7 @@ struct DctPlan {
   void* tw[3] = {};   // exp(-2 pi i m / N), m < N
   void* half[3] = {}; // exp(-i pi k / (2 N)), k < N
   void* lam[3] = {};  // eigenvalues, mode k at k
+  int64_t plane;      // reals between the planes of the workspace
 };
 
 namespace {
@@ -65,18 +67,20 @@ struct DctRows {
 
 template <typename T, int L, bool INV>
 __global__ void __launch_bounds__((DctRows<T, L>::NT))
-    k_dct_rows(const T* in, T* out, int64_t pairs, const Cplx<T>* tw, const Cplx<T>* half) {
+    k_dct_rows(const T* in, T* out, int pairs, int plane_pairs, int64_t in_pad, int64_t out_pad, const Cplx<T>* tw,
+               const Cplx<T>* half) {
   using R = DctRows<T, L>;
   constexpr int E = R::E, TT = R::TT;
   extern __shared__ unsigned char smem_raw[];
   Cplx<T>* const xb = reinterpret_cast<Cplx<T>*>(smem_raw);
   const int t = threadIdx.x % TT, team = threadIdx.x / TT;
-  const int64_t q = int64_t(blockIdx.x) * R::NTEAM + team;
+  const int q = int(blockIdx.x) * R::NTEAM + team;
   const bool live = q < pairs;
+  const int plane = (live ? q : 0) / plane_pairs;
   Cplx<T>* const line = xb + team * R::S;
   Cplx<T>* const twl = xb + R::NTEAM * R::S;
   rfft::load_tw_lds<T, L>(twl, tw, threadIdx.x, R::NT);
-  const T* const a = in + (live ? q : 0) * 2 * L;
+  const T* const a = in + (live ? q : 0) * int64_t(2 * L) + plane * in_pad;
   static_for<0, E>([&](auto e_) {
     const int i = t + TT * decltype(e_)::value;
     line[INV ? i : dct_slot<L>(i)] = Cplx<T>{a[i], a[L + i]};
@@ -101,7 +105,7 @@ __global__ void __launch_bounds__((DctRows<T, L>::NT))
   });
   wave_sync();
   if (!live) return;
-  T* const o = out + q * 2 * L;
+  T* const o = out + q * int64_t(2 * L) + plane * out_pad;
   static_for<0, E>([&](auto e_) {
     constexpr int e = decltype(e_)::value;
     const int i = t + TT * e;
@@ -121,7 +125,11 @@ struct DctCols {
   static constexpr int FULL = 128 / int(sizeof(Cplx<T>));
   static constexpr int WC = FULL * TT <= 512 ? FULL : 512 / TT;
   static constexpr int NT = WC * TT;
-  static constexpr int S = region_stride<L, true>();
+  // a column's cells take neighbouring slots of opposite parity, so two rows of WC columns (half a
+  // wavefront) fall in distinct LDS banks at a stride of 2 (mod 32); at 16, which suits the
+  // exchanges of teams of 16, the loads and stores meet 8 lanes deep: 128^3 FP32 80 against 63 us,
+  // 192^3 FP32 218 against 170 us
+  static constexpr int S = L + 2;
   static constexpr size_t lds = (size_t(WC) * S + rfft::tw_lds_size<L>()) * sizeof(Cplx<T>);
 };
 
@@ -286,11 +294,13 @@ int rows_pass(DctPlan* P, const T* in, T* out, int ncomp, hipStream_t s) {
   return with_length(P->n[2], [&](auto l) -> int {
     constexpr int L = decltype(l)::value;
     using R = DctRows<T, L>;
-    const int64_t pairs = ncomp * P->n[0] * P->n[1] / 2;
+    const int plane_pairs = int(P->n[1] / 2), pairs = int(ncomp * P->n[0]) * plane_pairs;
+    const int64_t pad = P->plane - P->n[1] * P->n[2];
     int rc = allow_lds(k_dct_rows<T, L, INV>, R::lds);
     if (rc) return rc;
     k_dct_rows<T, L, INV><<<ceil_div(pairs, R::NTEAM), R::NT, R::lds, s>>>(
-        in, out, pairs, static_cast<const Cplx<T>*>(P->tw[2]), static_cast<const Cplx<T>*>(P->half[2]));
+        in, out, pairs, plane_pairs, INV ? pad : 0, INV ? 0 : pad, static_cast<const Cplx<T>*>(P->tw[2]),
+        static_cast<const Cplx<T>*>(P->half[2]));
     SOPHT_CHECK_LAUNCH();
     return SOPHT_OK;
   });
@@ -302,7 +312,7 @@ int y_pass(DctPlan* P, T* f, int ncomp, hipStream_t s) {
     constexpr int L = decltype(l)::value;
     using C = DctCols<T, L>;
     const int cols = int(P->n[2] / 2);
-    const ColGeo g{cols, P->n[1] * cols, cols, ceil_div(cols, C::WC)};
+    const ColGeo g{cols, P->plane / 2, cols, ceil_div(cols, C::WC)};
     int rc = allow_lds(k_dct_cols<T, L, INV>, C::lds);
     if (rc) return rc;
     k_dct_cols<T, L, INV><<<unsigned(g.tiles * ncomp * P->n[0]), C::NT, C::lds, s>>>(
@@ -319,7 +329,7 @@ int z_pass(DctPlan* P, T* f, int ncomp, hipStream_t s) {
     constexpr int L = decltype(l)::value;
     using C = DctCols<T, L>;
     const int cols = int(P->n[2] / 2), ny = int(P->n[1]);
-    const int64_t plane = int64_t(ny) * cols;
+    const int64_t plane = P->plane / 2;
     const ColGeo g{plane, cols, cols, ceil_div(cols, C::WC)};
     int rc = allow_lds(k_dct_z<T, L>, C::lds);
     if (rc) return rc;
@@ -390,12 +400,17 @@ bool dct_supported(const int64_t n[3]) {
   return true;
 }
 
+int64_t dct_plane(int dtype, const int64_t n[3]) {
+  return n[1] * n[2] + 128 / (dtype == SOPHT_F32 ? 4 : 8);
+}
+
 int dct_create(int dtype, const int64_t n[3], const double* const lam[3], DctPlan** out) {
   *out = nullptr;
   DctPlan* P = new (std::nothrow) DctPlan();
   SOPHT_REQUIRE(P != nullptr, "out of host memory");
   P->dtype = dtype;
   for (int a = 0; a < 3; ++a) P->n[a] = n[a];
+  P->plane = dct_plane(dtype, n);
   const int rc = dtype == SOPHT_F32 ? tables<float>(P, lam) : tables<double>(P, lam);
   if (rc) {
     dct_destroy(P);

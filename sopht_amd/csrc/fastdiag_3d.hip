@@ -205,8 +205,10 @@ int upload(void** dst, const std::vector<double>& src) {
 
 template <typename T>
 int create_device(sopht_fastdiag3d* P) {
-  SOPHT_CHECK_HIP(hipMalloc(&P->work, 3 * P->n[0] * P->n[1] * P->n[2] * sizeof(T)));
-  if (dct_supported(P->n)) {
+  const bool dct = dct_supported(P->n);
+  const int64_t plane = dct ? dct_plane(P->dtype, P->n) : P->n[1] * P->n[2];
+  SOPHT_CHECK_HIP(hipMalloc(&P->work, 3 * P->n[0] * plane * sizeof(T)));
+  if (dct) {
     std::vector<double> up[3];  // the eigenvalues in increasing order, as the transforms leave the modes
     const double* lam[3];
     for (int a = 0; a < 3; ++a) {

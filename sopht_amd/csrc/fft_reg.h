@@ -254,11 +254,15 @@ struct Swizzle {
 };
 
 // LDS elements reserved per line. Teams of 16 threads share a 32-lane half-wave, so their
-// regions start 16 slots apart (mod 32). Column tiles stage WC = 8 columns with lanes
-// (column, row); a stride of 4 (mod 32) between column regions keeps those accesses
-// conflict-free too.
+// regions start 16 slots apart (mod 32). Shorter teams' lines keep the identity map, whose writes
+// step by the radix, so their regions start 9 apart (2 for teams of 2): an exchange of 24, 32, 48,
+// 64 or 96 points then meets 1.5 to 2 lanes per bank on average, against 4, 6, 8, 5 and 3 at 16
+// (counted on the host). Column tiles stage WC = 8 columns with lanes (column, row); a stride of 4
+// (mod 32) between column regions keeps those accesses conflict-free too.
 template <int L, bool COLUMN>
 constexpr int region_stride() {
+  if (LinePlan<L>::T <= 2) return L + 2;
+  if (LinePlan<L>::T < 16) return L + 9;
   if (LinePlan<L>::T < 32) return L + 16;
   return COLUMN ? L + 4 : L;
 }

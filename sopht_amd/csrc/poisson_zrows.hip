@@ -42,9 +42,12 @@ struct ZRowTile {
   static constexpr int SLOTS = SOPHT_ZROW_SLOTS;  // pencils per column transformed at once
   static constexpr int WC = kLineCplx<T> / PARTS;
   static constexpr int NT = SLOTS * WC * TT;
-  // tiles [slot][column]: the load role's lanes (column, z) hit distinct banks when the
-  // column stride is 8 (mod 32) slots
-  static constexpr int S = TT < 32 ? L + 16 : (WC == 4 ? L + 8 : L + 4);
+  // tiles [slot][column]: the load role's lanes (column, z) hit distinct banks when the column
+  // stride is 8 (mod 32) slots, or 4 (mod 16) of the 16-byte FP64 ones, which are served 16 lanes
+  // at a time; FP32 teams of 16 need 16 for their exchanges, shorter ones 9 as elsewhere
+  static constexpr int S = TT < 16 ? region_stride<L, true>()
+                           : sizeof(T) == 8 ? L + 4
+                           : TT < 32 ? L + 16 : (WC == 4 ? L + 8 : L + 4);
   static constexpr int KL = E / (2 * SLOTS);  // z values per row per thread (z = lr + SLOTS TT k)
   static constexpr int GL = L / 2 + 1;
   static constexpr size_t lds = size_t(SLOTS * WC * S) * sizeof(Cplx<T>) + size_t(4 * WC * GL) * sizeof(T);

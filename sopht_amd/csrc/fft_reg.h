@@ -235,14 +235,14 @@ constexpr bool kTwiddleProducts = SOPHT_TWIDDLE_PRODUCTS;
 // (j / NS) NS R + j % NS + r NS (stride R or NS between lanes) and the next stage reads
 // t + T e (unit stride); the XOR moves the lane bits that would collide onto the bank bits the
 // other pattern leaves free, so on gfx950 (64-bit accesses served 32 lanes at a time by 64
-// four-byte banks) both patterns are conflict-free for every plan from 128 points on
-// (checked exhaustively on the host). The map is an involution on [0, L). Shorter lines keep
-// the identity.
+// four-byte banks) both patterns are conflict-free for the plan of 64 points and every plan from
+// 128 points on (checked exhaustively on the host). The map is an involution on [0, L). The other
+// lines keep the identity.
 template <int L, int NS, int R>
 struct Swizzle {
   static constexpr int T = LinePlan<L>::T;
-  static constexpr bool kOn = L >= 128;
-  static constexpr int A = T >= 32 ? 5 : 4;
+  static constexpr bool kOn = L >= 128 || L == 64;
+  static constexpr int A = T >= 32 ? 5 : (T >= 16 ? 4 : 3);
   static constexpr int MB = NS == 1 ? ilog2(R) : (ilog2(R) < 3 ? ilog2(R) : 3);
   static constexpr int B = NS == 1 ? 0 : 2;
   static_assert(!kOn || (1 << ilog2(R)) == R, "swizzled exchanges need a power-of-two radix");
@@ -254,15 +254,15 @@ struct Swizzle {
 };
 
 // LDS elements reserved per line. Teams of 16 threads share a 32-lane half-wave, so their
-// regions start 16 slots apart (mod 32). Shorter teams' lines keep the identity map, whose writes
-// step by the radix, so their regions start 9 apart (2 for teams of 2): an exchange of 24, 32, 48,
-// 64 or 96 points then meets 1.5 to 2 lanes per bank on average, against 4, 6, 8, 5 and 3 at 16
-// (counted on the host). Column tiles stage WC = 8 columns with lanes (column, row); a stride of 4
+// regions start 16 slots apart (mod 32), those of 64-point lines 8. Shorter teams' other lines keep
+// the identity map, whose writes step by the radix, so their regions start 9 apart (2 for teams
+// of 2): an exchange of 24, 32, 48 or 96 points then meets 1.5 to 2 lanes per bank on average,
+// against 4, 6, 8 and 3 at 16 (counted on the host). Column tiles stage WC = 8 columns with lanes (column, row); a stride of 4
 // (mod 32) between column regions keeps those accesses conflict-free too.
 template <int L, bool COLUMN>
 constexpr int region_stride() {
   if (LinePlan<L>::T <= 2) return L + 2;
-  if (LinePlan<L>::T < 16) return L + 9;
+  if (LinePlan<L>::T < 16) return L == 64 ? L + 8 : L + 9;
   if (LinePlan<L>::T < 32) return L + 16;
   return COLUMN ? L + 4 : L;
 }

@@ -94,9 +94,10 @@ struct XYPass {
   static constexpr int NCH = EX / 2 / KC + 1;  // the last chunk is kx = nx alone
   static constexpr int SX = region_stride<LX, false>();
   static constexpr int S2 = region_stride<L2, true>();
-  // staging tile [row][P]: the column teams' accesses (T2 rows of 32 / T2 columns per half
-  // wavefront) fall in distinct banks when P = 32 / T2 (mod 32)
-  static constexpr int P = (CW + 31) / 32 * 32 + 32 / T2;
+  // staging tile [row][P]: the column teams' accesses (T2 rows of LANES / T2 columns) fall in
+  // distinct banks when P = LANES / T2 (mod LANES), LANES the lanes served at a time
+  static constexpr int LANES = sizeof(T) == 4 ? 32 : 16;
+  static constexpr int P = (CW + LANES - 1) / LANES * LANES + (LANES >= T2 ? LANES / T2 : 1);
   static constexpr int TW2 = rfft::tw_lds_size<L2>();                // padded w_L2 table
   static constexpr int XPH = NTEAM * SX + rfft::tw_lds_size<LX>();  // x regions, x table
   static constexpr int CREG = CW * S2;         // column regions

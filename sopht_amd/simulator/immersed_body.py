@@ -89,10 +89,10 @@ class ThreeDimensionalRigidBodyForcingGrid(ImmersedBodyForcingGrid):
         self.global_frame_relative_position_field = np.zeros_like(self.position_field)
 
     def compute_lag_grid_position_field(self):
-        np.dot(self.rigid_body.director_collection[:, :, 0].T, self.local_frame_relative_position_field,
-               out=self.global_frame_relative_position_field)
-        np.add(self.rigid_body.position_collection, self.global_frame_relative_position_field,
-               out=self.position_field)
+        self.global_frame_relative_position_field[...] = np.dot(
+            self.rigid_body.director_collection[:, :, 0].T, self.local_frame_relative_position_field
+        )
+        self.position_field[...] = self.rigid_body.position_collection + self.global_frame_relative_position_field
 
     def compute_lag_grid_velocity_field(self):
         # V + (omega x r) with omega broadcast over the nodes, written per component with the

@@ -77,7 +77,8 @@ int sopht_diffusion_flux_3d(int dtype, void* flux, const int64_t* flux_strides,
                             const void* field, const int64_t* field_strides, int64_t nz,
                             int64_t ny, int64_t nx, double prefactor, int reset_ghost_zone,
                             void* stream);
-/* The three components of a vector field in one launch. */
+/* The three components of a vector field: in one launch where no component's output meets another
+ * component's fields, else one after another in order. */
 int sopht_diffusion_flux_vector_3d(int dtype, void* const flux[3], const int64_t* flux_strides,
                                    const void* const field[3], const int64_t* field_strides,
                                    int64_t nz, int64_t ny, int64_t nx, double prefactor, int reset,
@@ -103,7 +104,8 @@ int sopht_diffusion_timestep_euler_forward_vector_3d(int dtype, void* const fiel
 int sopht_penalise_field_boundary_3d(int dtype, void* field, const int64_t* field_strides,
                                      int64_t nz, int64_t ny, int64_t nx, int width,
                                      const double* sine_tables, void* stream);
-/* The three components of a vector field in one launch. */
+/* The three components of a vector field: in one launch where no component's output meets another
+ * component's fields, else one after another in order. */
 int sopht_penalise_field_boundary_vector_3d(int dtype, void* const field[3], const int64_t* field_strides,
                                             int64_t nz, int64_t ny, int64_t nx, int width,
                                             const double* tables, void* stream);

@@ -200,6 +200,22 @@ inline bool fields_meet(const void* a, const int64_t* as, const void* b, const i
   return pa < pb + span(bs) && pb < pa + span(as);
 }
 
+// Whether no component's output meets another component's output or operand: such components may
+// run in any order. A caller may pass windows of one tensor (out = t[0:3], in = t[1:4]) or a
+// component repeated by a zero stride; the components then run one after another, as the
+// reference's loop over them does.
+template <typename T>
+inline bool components_apart(int ncomp, void* const* out, const int64_t* os, const void* const* in,
+                             const int64_t* is, int64_t nz, int64_t ny, int64_t nx) {
+  for (int a = 0; a < ncomp; ++a)
+    for (int b = 0; b < ncomp; ++b) {
+      if (a == b) continue;
+      if (fields_meet<T>(out[a], os, out[b], os, nz, ny, nx)) return false;
+      if (in && fields_meet<T>(out[a], os, in[b], is, nz, ny, nx)) return false;
+    }
+  return true;
+}
+
 // ------------------------------------------------------------------ vorticity stretching
 
 template <typename T>
@@ -699,15 +715,16 @@ struct Flat {
   T* out[3];
   const T* in[N > 0 ? N : 1][3];
   int64_t n;  // cells
+  int first;  // component of gridDim.y's first slice
 };
 
-// out = fn(comp, in...) over the cells of up to three dense components (gridDim.y), 16 bytes a
-// thread. Bound by memory: the sum of two 130 x 170 x 250 FP32 fields takes 10.9 us (6.1 TB/s, most
+// out = fn(comp, in...) over the cells of up to three dense components (gridDim.y from a.first), 16
+// bytes a thread. Bound by memory: the sum of two 130 x 170 x 250 FP32 fields takes 10.9 us (6.1 TB/s, most
 // of it from the caches) against 18.4 us with one cell per thread and 64-bit divisions.
 template <typename T, int N, typename Fn>
 __global__ void __launch_bounds__(256) k_flat(Flat<T, N> a, Fn fn) {
   constexpr int V = RowVec<T>::V;
-  const int c = int(blockIdx.y);
+  const int c = a.first + int(blockIdx.y);
   const int64_t i = (blockIdx.x * int64_t(256) + threadIdx.x) * V;
   auto one = [&](const T* v) -> T {
     if constexpr (N == 0) return fn(c);

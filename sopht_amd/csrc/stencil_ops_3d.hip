@@ -197,7 +197,8 @@ int cross_impl(void* const r[3], const int64_t* rs, const void* const a[3], cons
       s);
 }
 
-// out = fn(comp, in...) over ncomp fields of one box; flat over dense fields.
+// out = fn(comp, in...) over ncomp fields of one box; flat over dense fields, all components in
+// one launch where they may run in any order.
 template <typename T, int N, typename Fn>
 int pointwise(int ncomp, void* const* out, const int64_t* os, const void* const* const* in, const int64_t* const* is,
               int64_t nz, int64_t ny, int64_t nx, Fn fn, hipStream_t s) {
@@ -210,8 +211,13 @@ int pointwise(int ncomp, void* const* out, const int64_t* os, const void* const*
       f.out[c] = static_cast<T*>(out[c]);
       for (int q = 0; q < N; ++q) f.in[q][c] = static_cast<const T*>(in[q][c]);
     }
-    k_flat<T, N><<<flat_grid<T>(f.n, ncomp), 256, 0, s>>>(f, fn);
-    SOPHT_CHECK_LAUNCH();
+    bool apart = components_apart<T>(ncomp, out, os, nullptr, nullptr, nz, ny, nx);
+    for (int q = 0; q < N; ++q) apart = apart && components_apart<T>(ncomp, out, os, in[q], is[q], nz, ny, nx);
+    const int together = apart ? ncomp : 1;
+    for (; f.first < ncomp; f.first += together) {
+      k_flat<T, N><<<flat_grid<T>(f.n, together), 256, 0, s>>>(f, fn);
+      SOPHT_CHECK_LAUNCH();
+    }
     return SOPHT_OK;
   }
   for (int c = 0; c < ncomp; ++c) {
@@ -277,6 +283,12 @@ template <typename T>
 int diffusion_flux_impl(int ncomp, void* const* flux, const int64_t* fs, const void* const* field, const int64_t* is,
                         int64_t nz, int64_t ny, int64_t nx, T p, int reset, hipStream_t s) {
   if (row_box_ok<T, 1>(nz, ny, nx) && row_strides_ok(fs, nz, ny, nx) && row_strides_ok(is, nz, ny, nx)) {
+    if (!components_apart<T>(ncomp, flux, fs, field, is, nz, ny, nx)) {
+      int rc = SOPHT_OK;
+      for (int c = 0; c < ncomp && !rc; ++c)
+        rc = diffusion_flux_impl<T>(1, flux + c, fs, field + c, is, nz, ny, nx, p, reset, s);
+      return rc;
+    }
     const RowGeo g = row_geo<T>(nz, ny, nx, kRowChunk);
     Rows3<T> o{};
     Rows3<const T> in{};
@@ -373,6 +385,11 @@ int penalise_impl(int ncomp, void* const* fields, const int64_t* fs, int64_t nz,
   if (w == 0) return SOPHT_OK;
   SOPHT_REQUIRE(w > 0 && w <= 8, "penalty width must be in [0, 8]");
   SOPHT_REQUIRE(2 * w <= nz && 2 * w <= ny && 2 * w <= nx, "grid too small for penalty width");
+  if (!components_apart<T>(ncomp, fields, fs, nullptr, nullptr, nz, ny, nx)) {
+    int rc = SOPHT_OK;
+    for (int c = 0; c < ncomp && !rc; ++c) rc = penalise_impl<T>(1, fields + c, fs, nz, ny, nx, w, tables, s);
+    return rc;
+  }
   SineTables<T> st;
   for (int a = 0; a < 3; ++a)
     for (int i = 0; i < w; ++i) {

@@ -317,14 +317,16 @@ __global__ void __launch_bounds__(kRowThreads)
 // The flux through the face between cells 0 and 1 of one axis (advection_flux_3d.py:12-233),
 // from the field f and the velocity u at cells -1 .. 2. A cell's front face is its upper
 // neighbour's back face, with the same upwind choice and the same terms, so each face is formed
-// once. Every product and sum rounds by itself, as the reference's.
+// once. The weighted field values and the smallest of the three products round by themselves,
+// the other products only in the sums (written out, so that every kernel of the flux gives the
+// same bits): 150 x 201 x 230 FP32, relative error 5.4e-7 against 7.7e-7 with every product
+// rounded, in the same time.
 template <typename T>
 __device__ __forceinline__ T eno3_face(T fm, T f0, T f1, T fp, T um, T u0, T u1, T up) {
-#pragma clang fp contract(off)
   const T c13 = T(1.0 / 3.0), c56 = T(5.0 / 6.0), c16 = T(1.0 / 6.0);
   const bool left = u0 > -u1;
-  const T near = c13 * (left ? f1 : f0) * (left ? u1 : u0), here = c56 * (left ? f0 : f1) * (left ? u0 : u1);
-  return near + here - c16 * (left ? fm : fp) * (left ? um : up);
+  const T far = c16 * (left ? fm : fp) * (left ? um : up);
+  return fma(c56 * (left ? f0 : f1), left ? u0 : u1, fma(c13 * (left ? f1 : f0), left ? u1 : u0, -far));
 }
 
 // What k_eno3_rows does with the flux E of [2:-2]^3.
@@ -370,7 +372,6 @@ __global__ void __launch_bounds__(kRowThreads)
   }
   const unsigned mask = c.yin ? c.own & c.inner : 0u;
   for (int z = za; z < zb; ++z) {
-#pragma clang fp contract(off)
     const T* fz = f + z * fs.z + fr;
     const T* uxz = u.p[0] + z * u.s.z + ur;
     const T* uyz = u.p[1] + z * u.s.z + ur;
@@ -406,17 +407,17 @@ __global__ void __launch_bounds__(kRowThreads)
         face[k] = eno3_face<T>(e[k], e[k + 1], e[k + 2], e[k + 3], v[k], v[k + 1], v[k + 2], v[k + 3]);
 #pragma unroll
       for (int k = 0; k < V; ++k) {
-        acc[k] = acc[k] + inv_dx * face[k + 1];
-        acc[k] = acc[k] - inv_dx * face[k];
+        acc[k] = fma(inv_dx, face[k + 1], acc[k]);
+        acc[k] = fma(-inv_dx, face[k], acc[k]);
       }
     }
 #pragma unroll
     for (int k = 0; k < V; ++k) {
-      acc[k] = acc[k] + inv_dx * eno3_face<T>(fy[1][k], fy[2][k], fy[3][k], fy[4][k], uy[1][k], uy[2][k], uy[3][k], uy[4][k]);
-      acc[k] = acc[k] - inv_dx * eno3_face<T>(fy[0][k], fy[1][k], fy[2][k], fy[3][k], uy[0][k], uy[1][k], uy[2][k], uy[3][k]);
+      acc[k] = fma(inv_dx, eno3_face<T>(fy[1][k], fy[2][k], fy[3][k], fy[4][k], uy[1][k], uy[2][k], uy[3][k], uy[4][k]), acc[k]);
+      acc[k] = fma(-inv_dx, eno3_face<T>(fy[0][k], fy[1][k], fy[2][k], fy[3][k], uy[0][k], uy[1][k], uy[2][k], uy[3][k]), acc[k]);
       const T front = eno3_face<T>(fm[k], f0[k], f1[k], f2[k], wm[k], w0[k], w1[k], w2[k]);
-      acc[k] = acc[k] + inv_dx * front;
-      acc[k] = acc[k] - inv_dx * back[k];
+      acc[k] = fma(inv_dx, front, acc[k]);
+      acc[k] = fma(-inv_dx, back[k], acc[k]);
       back[k] = front;
     }
     if constexpr (MODE == kEnoAdd) {

@@ -463,31 +463,36 @@ inline bool eno3_grid_fits(int64_t bz, int64_t by) {
   return bz > 0 && bz <= 65535 && ceil_div(by, kEnoTy) <= 65535;
 }
 
+// acc plus the front face's flux and minus the back face's of one axis, from the field F and the
+// velocity U at cells -2 .. 2.
+template <typename T>
+__device__ __forceinline__ T eno3_axis(const T* F, const T* U, T acc, T inv_dx) {
+  acc = fma(inv_dx, eno3_face<T>(F[1], F[2], F[3], F[4], U[1], U[2], U[3], U[4]), acc);
+  return fma(-inv_dx, eno3_face<T>(F[0], F[1], F[2], F[3], U[0], U[1], U[2], U[3]), acc);
+}
+
 // ENO3 conservative advection flux (advection_flux_3d.py:12-233): the six sub-stencils
 // accumulate in the reference order on [2:-2]^3; one thread computes all six for its cell.
 template <typename T>
 __device__ __forceinline__ T eno3_cell(const T* f, int64_t fo, Strides3 fs, const T* const u[3],
                                        int64_t uo, Strides3 us, T acc, T inv_dx) {
-  const T c13 = T(1.0 / 3.0), c56 = T(5.0 / 6.0), c16 = T(1.0 / 6.0);
   for (int a = 0; a < 3; ++a) {
     const T* ua = u[a];
     const int64_t sf = fs.step(a), su = us.step(a);
-    auto F = [&](int k) -> T { return f[fo + k * sf]; };
-    auto U = [&](int k) -> T { return ua[uo + k * su]; };
-    T front = (U(0) > -U(1)) ? (c13 * F(1) * U(1) + c56 * F(0) * U(0) - c16 * F(-1) * U(-1))
-                             : (c13 * F(0) * U(0) + c56 * F(1) * U(1) - c16 * F(2) * U(2));
-    acc = acc + inv_dx * front;
-    T back = (U(0) > -U(-1)) ? (c13 * F(0) * U(0) + c56 * F(-1) * U(-1) - c16 * F(-2) * U(-2))
-                             : (c13 * F(-1) * U(-1) + c56 * F(0) * U(0) - c16 * F(1) * U(1));
-    acc = acc - inv_dx * back;
+    T F[5], U[5];
+    for (int k = 0; k < 5; ++k) {
+      F[k] = f[fo + (k - 2) * sf];
+      U[k] = ua[uo + (k - 2) * su];
+    }
+    acc = eno3_axis(F, U, acc, inv_dx);
   }
   return acc;
 }
 
 // The same flux for fields whose cells are not adjacent along x (k_eno3_rows takes the others):
 // a thread owns one (y, x) column of kEnoZc planes and keeps f and u_z at z-2..z+2 in
-// registers, so the z terms cost two loads per cell instead of nine. The x and y terms are read
-// as in eno3_cell, and every expression is the same, so the results are the same bits.
+// registers, so the z terms cost two loads per cell instead of nine. The faces and the order of
+// the sums are those of k_eno3_rows and eno3_cell, so all three give the same bits.
 constexpr int kEnoZc = 16;
 
 template <typename T>
@@ -499,7 +504,6 @@ __global__ void __launch_bounds__(kEnoTx* kEnoTy)
   const int64_t z0 = 2 + int64_t(blockIdx.z) * kEnoZc;
   if (x >= nx - 2 || y >= ny - 2 || z0 >= nz - 2) return;
   const int64_t z1 = z0 + kEnoZc < nz - 2 ? z0 + kEnoZc : nz - 2;
-  const T c13 = T(1.0 / 3.0), c56 = T(5.0 / 6.0), c16 = T(1.0 / 6.0);
   T fw[5], uw[5];
   {
     const int64_t fo = fs.at(z0, y, x), uo = us.at(z0, y, x);
@@ -515,25 +519,15 @@ __global__ void __launch_bounds__(kEnoTx* kEnoTy)
     for (int a = 0; a < 2; ++a) {
       const T* ua = a == 0 ? u0 : u1;
       const int64_t sf = a == 0 ? fs.x : fs.y, su = a == 0 ? us.x : us.y;
-      auto F = [&](int k) -> T { return f[fo + k * sf]; };
-      auto U = [&](int k) -> T { return ua[uo + k * su]; };
-      T front = (U(0) > -U(1)) ? (c13 * F(1) * U(1) + c56 * F(0) * U(0) - c16 * F(-1) * U(-1))
-                               : (c13 * F(0) * U(0) + c56 * F(1) * U(1) - c16 * F(2) * U(2));
-      acc = acc + inv_dx * front;
-      T back = (U(0) > -U(-1)) ? (c13 * F(0) * U(0) + c56 * F(-1) * U(-1) - c16 * F(-2) * U(-2))
-                               : (c13 * F(-1) * U(-1) + c56 * F(0) * U(0) - c16 * F(1) * U(1));
-      acc = acc - inv_dx * back;
+      T F[5], U[5];
+#pragma unroll
+      for (int k = 0; k < 5; ++k) {
+        F[k] = f[fo + (k - 2) * sf];
+        U[k] = ua[uo + (k - 2) * su];
+      }
+      acc = eno3_axis(F, U, acc, inv_dx);
     }
-    {
-      auto F = [&](int k) -> T { return fw[k + 2]; };
-      auto U = [&](int k) -> T { return uw[k + 2]; };
-      T front = (U(0) > -U(1)) ? (c13 * F(1) * U(1) + c56 * F(0) * U(0) - c16 * F(-1) * U(-1))
-                               : (c13 * F(0) * U(0) + c56 * F(1) * U(1) - c16 * F(2) * U(2));
-      acc = acc + inv_dx * front;
-      T back = (U(0) > -U(-1)) ? (c13 * F(0) * U(0) + c56 * F(-1) * U(-1) - c16 * F(-2) * U(-2))
-                               : (c13 * F(-1) * U(-1) + c56 * F(0) * U(0) - c16 * F(1) * U(1));
-      acc = acc - inv_dx * back;
-    }
+    acc = eno3_axis(fw, uw, acc, inv_dx);
     flux[oo] = acc;
     if (z + 1 < z1) {
       // plane z + 3 exists: z + 1 < z1 <= nz - 2

@@ -648,7 +648,7 @@ __global__ void __launch_bounds__(kRowThreads) k_laplacian_rows(RowGeo g, Rows3<
   for (int z = c.z0; z < c.z1; ++z) {
     const bool plane = z > 0 && z < g.nz - 1;
     const T* fz = f + z * in.s.z + fr;
-    vec r = {}, fp = fc;
+    vec r = {}, fp = fc;  // r: lap_h(f), times p but for kRowStep
     if (z < g.nz - 1) fp = rload(fz + in.s.z);
     if (plane) {
       const vec yp = rload(fz + in.s.y), ym = rload(fz - in.s.y);
@@ -656,16 +656,16 @@ __global__ void __launch_bounds__(kRowThreads) k_laplacian_rows(RowGeo g, Rows3<
 #pragma unroll
       for (int k = 0; k < V; ++k) {
         const T right = k < V - 1 ? fc[k < V - 1 ? k + 1 : k] : xr, left = k > 0 ? fc[k > 0 ? k - 1 : k] : xl;
-        r[k] = p * (fp[k] + fm[k] + yp[k] + ym[k] + right + left - T(6) * fc[k]);
+        const T lap = fp[k] + fm[k] + yp[k] + ym[k] + right + left - T(6) * fc[k];
+        r[k] = MODE == kRowStep ? lap : p * lap;
       }
     }
     const unsigned inside = plane && c.yin ? c.own & c.inner : 0u;
     if constexpr (MODE == kRowStep) {
-#pragma clang fp contract(off)
       vec v = fc;
       if (!c.yin) v = rload_own(c, g, f + z * in.s.z + c.y * in.s.y + c.x, z);
 #pragma unroll
-      for (int k = 0; k < V; ++k) v[k] = inside >> k & 1u ? v[k] + r[k] : v[k];
+      for (int k = 0; k < V; ++k) v[k] = inside >> k & 1u ? fma(p, r[k], v[k]) : v[k];
       rstore(out + z * o.s.z + orow, v, c.own);
     } else {
       row_out<T, MODE>(c, g, out + z * o.s.z + orow, r, inside, z);

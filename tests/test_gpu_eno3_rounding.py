@@ -68,3 +68,30 @@ def test_products_are_fused(dev, place, seed):
     out = place(np.zeros_like(f), dev)
     spne().gen_advection_flux_conservative_eno3_pyst_kernel_3d(np.float32)(out, place(f, dev), place(u, dev), 0.5)
     assert rel_l2(to_host(out), exact) < rel_l2(single, exact)
+
+
+@pytest.mark.parametrize("ncomp", [1, 3])
+@pytest.mark.parametrize("real_t,wide", [(np.float32, np.float64), (np.float64, np.longdouble)], ids=["f32", "f64"])
+def test_diffusion_of_the_transport_step_rounds_once(dev, real_t, wide, ncomp):
+    """At rest the transport step is phi + p lap(phi), one fused multiply-add a cell: on integers
+    the Laplacian is exact, and so are the product and the sum in the wider type."""
+    from sopht_amd import _lib as L
+
+    shape = (9, 12, 37)
+    p = real_t(0.1)
+    phi = np.random.default_rng(31).integers(-8, 9, (ncomp, *shape)).astype(real_t)
+    a = phi.astype(wide)
+    ref = a.copy()
+    c = a[:, 1:-1, 1:-1, 1:-1]
+    lap = (a[:, 2:, 1:-1, 1:-1] + a[:, :-2, 1:-1, 1:-1] + a[:, 1:-1, 2:, 1:-1] + a[:, 1:-1, :-2, 1:-1]
+           + a[:, 1:-1, 1:-1, 2:] + a[:, 1:-1, 1:-1, :-2] - 6 * c)
+    ref[:, 1:-1, 1:-1, 1:-1] = c + wide(p) * lap
+    t = to_dev(phi, dev)
+    scratch, u = to_dev(np.zeros_like(phi), dev), to_dev(np.zeros((3, *shape), dtype=real_t), dev)
+
+    def ptrs(v):
+        return L._p3(*([x.data_ptr() for x in v] + [0] * (3 - len(v))))
+
+    L.call("sopht_passive_transport_step_3d", L.dtype_tag(real_t), ncomp, ptrs(t), ptrs(scratch), ptrs(u), *shape, 0.5,
+           float(p), L.stream_ptr())
+    np.testing.assert_array_equal(to_host(t), ref.astype(real_t))

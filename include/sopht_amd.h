@@ -166,10 +166,15 @@ int sopht_passive_transport_step_3d(int dtype, int ncomp, void* const field[3], 
 
 /* compute_advection_diffusion_stable_timestep's reduction —
  * sopht/simulator/flow/passive_transport_flow_simulators.py:139-155: magnitude (optional, n
- * elements) = |u0| + |u1| + |u2| per cell, *out = its maximum (real_t, on the device), over n
+ * elements) = |u0| + |u1| + |u2| per cell, *out = its maximum (real_t, device or pinned memory), over n
  * contiguous cells; partial holds partial_cap real_t words of scratch. */
 int sopht_velocity_abs_sum_max_3d(int dtype, const void* const velocity[3], int64_t n, void* magnitude,
                                   void* partial, int64_t partial_cap, void* out, void* stream);
+
+/* Looks at a real_t in pinned host memory until it is not negative (0) or limit_s seconds have
+ * passed (1): the host's side of a value that a queued kernel stores there, marked as not yet
+ * there by a negative one. Yields the processor between looks; makes no HIP call. */
+int sopht_host_value_wait(int dtype, const void* value, double limit_s);
 
 /* gen_advection_flux_conservative_eno3_pyst_kernel_3d — .../advection_flux_3d.py:12-233.
  * Accumulates into flux on [2:-2]^3 (six sub-stencils in the reference order). */

@@ -6,6 +6,9 @@
 // launch; other strides run one thread per written cell with x-fastest lanes and a launch per
 // border slab. The flow step itself does not use them: it runs the fused sweeps in
 // flow_step_3d.hip.
+#include <sched.h>
+
+#include <chrono>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -952,6 +955,27 @@ using namespace sopht;
 extern "C" {
 
 const char* sopht_last_error(void) { return g_last_error; }
+int sopht_host_value_wait(int dtype, const void* value, double limit_s) {
+  SOPHT_REQUIRE(dtype == SOPHT_F32 || dtype == SOPHT_F64, "dtype must be SOPHT_F32 or SOPHT_F64");
+  SOPHT_REQUIRE(value != nullptr, "null pointer");
+  auto there = [&]() -> bool {
+    if (dtype == SOPHT_F32) {
+      float v;
+      __atomic_load(static_cast<const float*>(value), &v, __ATOMIC_ACQUIRE);
+      return !(v < 0.0f);
+    }
+    double v;
+    __atomic_load(static_cast<const double*>(value), &v, __ATOMIC_ACQUIRE);
+    return !(v < 0.0);
+  };
+  const auto end = std::chrono::steady_clock::now() + std::chrono::duration<double>(limit_s);
+  while (!there()) {
+    if (std::chrono::steady_clock::now() >= end) return there() ? SOPHT_OK : 1;
+    sched_yield();
+  }
+  return SOPHT_OK;
+}
+
 int sopht_version(void) { return 1; }
 
 int sopht_curl_3d(int dtype, void* const curl[3], const int64_t* cs, const void* const field[3],

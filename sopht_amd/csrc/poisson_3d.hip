@@ -34,7 +34,8 @@ struct sopht_poisson3d {
   void* tw[3];      // twiddles for lengths 2nx, 2ny, 2nz (x, y, z)
   int64_t rs;       // slab row stride (complex elements)
   int64_t gz;       // G^ line stride (elements): nz + 1 rounded up to a 128-byte line
-  int slab_comps;   // components the slab holds (3, or 3 per instance of a batched class)
+  int comps;        // components a solve may take (3, or 3 per instance of a batched class)
+  int slab_comps;   // components the slab holds: all of them, or a part of a large class
   int64_t slab_bytes, ghat_bytes;
   int passes;       // 3: x and y passes fused (three-pass schedule), or 5
   int zjobs;        // three-pass z pass: jobs per workgroup, chosen at plan creation
@@ -681,9 +682,15 @@ int poisson_vector_solve_accumulate(sopht_poisson3d* P, void* const sol[3], cons
 
 int poisson_table_solve(sopht_poisson3d* P, int ncomp, void* const* sol_tab, const int64_t* ss,
                         const void* const* rhs_tab, const int64_t* rs, hipStream_t s) {
-  return P->dtype == SOPHT_F32
-             ? solve_impl<float>(P, ncomp, nullptr, ss, nullptr, rs, s, nullptr, 0, sol_tab, rhs_tab)
-             : solve_impl<double>(P, ncomp, nullptr, ss, nullptr, rs, s, nullptr, 0, sol_tab, rhs_tab);
+  SOPHT_REQUIRE(ncomp <= P->comps, "more components than the Poisson plan was created for");
+  for (int c = 0; c < ncomp; c += P->slab_comps) {
+    const int n = std::min(ncomp - c, P->slab_comps);
+    const int rc = P->dtype == SOPHT_F32
+                       ? solve_impl<float>(P, n, nullptr, ss, nullptr, rs, s, nullptr, 0, sol_tab + c, rhs_tab + c)
+                       : solve_impl<double>(P, n, nullptr, ss, nullptr, rs, s, nullptr, 0, sol_tab + c, rhs_tab + c);
+    if (rc) return rc;
+  }
+  return SOPHT_OK;
 }
 
 }  // namespace sopht
@@ -734,14 +741,26 @@ int poisson_create(int dtype, int64_t nz, int64_t ny, int64_t nx, double x_range
   const bool five = forced != nullptr && std::atoi(forced) == 5;
   P->passes = (!five && kRowPad && xy_length_supported(dtype, 2 * nx) && xy_length_supported(dtype, 2 * ny) &&
                zrow_length_supported(2 * nz)) ? 3 : 5;
-  // whole 128-byte lines, and whole column tiles of the three-pass slab
-  const int64_t line = P->passes == 3 ? std::max<int64_t>(128 / cs, kSlabTile) : int64_t(128 / cs);
-  const int64_t rs = kRowPad ? round_up(nx + 1, line) : nx + 1;
+  // rows of whole 128-byte lines, and of whole column tiles of the three-pass slab
+  auto row_stride = [&](int passes) -> int64_t {
+    const int64_t line = passes == 3 ? std::max<int64_t>(128 / cs, kSlabTile) : int64_t(128 / cs);
+    return kRowPad ? round_up(nx + 1, line) : nx + 1;
+  };
+  // The passes index the slab with 32 bits. FP64 rows of the three-pass slab are padded further than
+  // the five-pass ones (192^3: 208 against 200), so some classes of many members (47 and 48 of 192^3)
+  // exceed it only for that: they are solved in parts, each member by the schedule it has alone.
+  auto elements = [&](int64_t c, int passes) -> int64_t { return c * nz * 2 * ny * row_stride(passes); };
+  constexpr int64_t most = (int64_t(1) << 31) - 1;
+  P->comps = P->slab_comps = comps;
+  if (elements(comps, P->passes) > most && elements(comps, 5) <= most) {
+    const int64_t at_once = most / elements(1, P->passes);
+    P->slab_comps = ceil_div(comps, ceil_div(comps, at_once));
+  }
+  const int64_t rs = row_stride(P->passes);
   P->rs = rs;
   P->gz = kRowPad ? round_up(nz + 1, int64_t(128 / rsz)) : nz + 1;
-  P->slab_comps = comps;
-  P->slab_bytes = int64_t(comps) * nz * 2 * ny * rs * int64_t(cs);
-  if (int64_t(comps) * nz * 2 * ny * rs >= (int64_t(1) << 31)) {
+  P->slab_bytes = elements(P->slab_comps, P->passes) * int64_t(cs);
+  if (elements(P->slab_comps, P->passes) > most) {
     delete P;
     set_last_error("Poisson grid too large: the spectral slab must have < 2^31 elements", __FILE__, __LINE__);
     return SOPHT_ERR_UNSUPPORTED;

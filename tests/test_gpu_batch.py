@@ -104,3 +104,48 @@ def test_batch_graph_replays_match_eager(dev):
         for (fa, _, _), (fb, _, _) in zip(eager, graph):
             assert np.array_equal(to_host(fa.vorticity_field), to_host(fb.vorticity_field))
             assert fa.time == fb.time
+
+
+def test_large_double_class_is_accepted_and_matches(dev):
+    """47 members of 192^3 in double precision: the padded rows of the three-pass schedule's slab
+    would exceed 2^31 elements where 48 members' plain rows do not. The class is accepted, its
+    members equal the ones stepped alone, and 49 members are refused."""
+    from types import SimpleNamespace
+
+    import torch
+
+    from sopht_amd import simulator as S
+
+    n, members = 192, 47
+    if torch.cuda.mem_get_info()[0] < 90 * 2**30:
+        pytest.skip("needs 90 GiB of device memory")
+    kw = dict(x_range=1.0, kinematic_viscosity=1e-3, real_t=np.float64)
+    alone = S.UnboundedNavierStokesFlowSimulator3D(grid_size=(n, n, n), **kw)
+    fields = torch.zeros((members, 3, 3, n, n, n), dtype=torch.float64, device=dev)
+    flows = [SimpleNamespace(real_t=np.float64, with_forcing=False, with_free_stream_flow=False, grid_size=(n, n, n),
+                             x_range=1.0, kinematic_viscosity=1e-3, flow_density=1.0, cfl=alone.cfl, time=0.0,
+                             penalty_zone_width=alone.penalty_zone_width, vorticity_field=f[0], velocity_field=f[1],
+                             stream_func_field=f[2], eul_grid_forcing_field=None) for f in fields]
+    with pytest.raises(ValueError, match="too large"):
+        S.BatchedFlowSimulation([(f, None, None) for f in flows + flows[:2]])
+    gen = torch.Generator(device=dev).manual_seed(9)
+    checked = (0, 23, 24, members - 1)
+    for k in checked:
+        flows[k].vorticity_field.normal_(generator=gen)
+        flows[k].velocity_field.normal_(generator=gen)
+    starts = {k: fields[k].clone() for k in checked}
+    sim = S.BatchedFlowSimulation([(f, None, None) for f in flows])
+    (schedule,) = sim.poisson_schedules()
+    assert (schedule["passes"], schedule["components"]) == (3, 3 * members)
+    sim.step(1, use_graph=False)
+    sim.synchronize()
+    sim.close()
+    for k in checked:
+        alone.vorticity_field.copy_(starts[k][0])
+        alone.velocity_field.copy_(starts[k][1])
+        alone.time_step(alone.compute_stable_timestep())
+        assert torch.equal(alone.vorticity_field, flows[k].vorticity_field), k
+        assert torch.equal(alone.stream_func_field, flows[k].stream_func_field), k
+        assert torch.equal(alone.velocity_field, flows[k].velocity_field), k
+    del fields, flows, starts, alone
+    torch.cuda.empty_cache()

@@ -613,8 +613,10 @@ int build_ghat(sopht_poisson3d* P, hipStream_t s) {
 }
 
 // Jobs per workgroup of the three-pass z pass: the fewer, the more workgroups (and the more
-// G^ staging). Each candidate is timed on the plan's own slab (zeroed) and stream, and the
-// fastest kept; SOPHT_POISSON_ZJOBS in the environment fixes the choice instead. Results do
+// G^ staging). Each candidate runs once on the plan's own slab (zeroed) and stream, after one run
+// that is not timed, and the fastest is kept: five z passes. Choices that one run does not tell
+// apart are within 2% of a solve; the wrong end of the range costs up to 60% (48^3).
+// SOPHT_POISSON_ZJOBS in the environment fixes the choice instead. Results do
 // not depend on it: a pencil's arithmetic is the same in any workgroup.
 template <typename T>
 int tune_zpass(sopht_poisson3d* P, hipStream_t s) {
@@ -639,12 +641,12 @@ int tune_zpass(sopht_poisson3d* P, hipStream_t s) {
   }
   int rc = SOPHT_OK;
   float best = -1.f;
+  rc = poisson_z_rows(2 * P->nz, g, H, gh, twz, s, 1);  // warm-up
   for (const int jobs : {1, 2, 3, 6}) {
-    if (jobs > 2 * g.ncomp) continue;
-    if ((rc = poisson_z_rows(2 * P->nz, g, H, gh, twz, s, jobs))) break;  // warm-up
-    if (hipEventRecord(e0, s) != hipSuccess) { rc = SOPHT_ERR_HIP; break; }
-    for (int r = 0; r < 3 && rc == SOPHT_OK; ++r) rc = poisson_z_rows(2 * P->nz, g, H, gh, twz, s, jobs);
     if (rc) break;
+    if (jobs > 2 * g.ncomp) continue;
+    if (hipEventRecord(e0, s) != hipSuccess) { rc = SOPHT_ERR_HIP; break; }
+    if ((rc = poisson_z_rows(2 * P->nz, g, H, gh, twz, s, jobs))) break;
     float ms = 0.f;
     if (hipEventRecord(e1, s) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
         hipEventElapsedTime(&ms, e0, e1) != hipSuccess) {

@@ -1,10 +1,13 @@
 """The row-vector operator kernels at the sizes where they can go wrong: rows shorter than a
 wavefront and longer than a workgroup, row lengths that are no multiple of the vector width
-(the last vector overlaps its neighbour), single chunks of planes and several, thin boxes.
+(the last vector reads past the row's end), single chunks of planes and several, thin boxes.
 
-Each operator runs twice on the same values: on dense fields (row-vector kernels) and on
-fields whose cells are two apart along x (one thread per cell), and both are compared with the
-oracle in double precision. The bound on an operator that sums ``m`` rounded products of
+Each operator runs on the same values in several layouts: dense fields, blocks inside larger
+arrays, blocks that end where their array ends, and fields whose planes are the faster axis
+(row-vector kernels; the pointwise operators take them cell by cell where they are not dense), and
+fields whose cells are two apart along x (one thread per cell). What lies around a block is NaN, so
+that a value read there and used would show, and must be as it was afterwards. Every result is
+compared with the oracle in double precision. The bound on an operator that sums ``m`` rounded products of
 magnitude ``s`` is ``2 m eps s``: each product and each addition rounds once."""
 
 import numpy as np
@@ -37,13 +40,40 @@ def spread_out(a, dev):
     return to_dev(big, dev)[..., ::2]
 
 
+def among(a, dev, front, back, planes_faster=False):
+    """The array as a block on the device, `front` and `back` cells from the ends of each axis of a
+    larger array (z, y, x) of NaN; optionally with the rows of a plane nz rows apart. Returns the
+    larger array too."""
+    b = np.swapaxes(a, -3, -2) if planes_faster else a
+    big = np.full((*b.shape[:-3], *(n + f + k for n, f, k in zip(b.shape[-3:], front, back))), np.nan, dtype=a.dtype)
+    cut = (..., *(slice(f, f + n) for n, f in zip(b.shape[-3:], front)))
+    big[cut] = b
+    t = to_dev(big, dev)
+    view = t[cut]
+    return (view.transpose(-3, -2) if planes_faster else view), t
+
+
+LAYOUTS = {
+    "dense": lambda a, dev: (to_dev(a, dev), None),
+    "spread out": lambda a, dev: (spread_out(a, dev), None),
+    "block": lambda a, dev: among(a, dev, (1, 2, 3), (1, 1, 2)),
+    "block at the end": lambda a, dev: among(a, dev, (1, 1, 1), (0, 0, 0)),
+    "planes faster": lambda a, dev: among(a, dev, (0, 0, 0), (0, 0, 0), True),
+    "block, planes faster": lambda a, dev: among(a, dev, (2, 1, 1), (0, 0, 0), True),
+}
+
+
 def both(run, outputs, inputs, dev, refs, bound):
-    """``run(outputs, inputs)`` on dense and on spread-out fields against ``refs``."""
-    for place in (lambda a: to_dev(a, dev), lambda a: spread_out(a, dev)):
-        outs = [place(a) for a in outputs]
-        run(outs, [place(a) for a in inputs])
-        for o, r in zip(outs, refs):
-            np.testing.assert_allclose(to_host(o), r, atol=bound, rtol=0)
+    """``run(outputs, inputs)`` in every layout against ``refs``."""
+    for name, place in LAYOUTS.items():
+        outs, arrays = zip(*(place(a, dev) for a in outputs))
+        ins = [place(a, dev) for a in inputs]
+        run(list(outs), [v for v, _ in ins])
+        for o, t, r in zip(outs, arrays, refs):
+            np.testing.assert_allclose(to_host(o), r, atol=bound, rtol=0, err_msg=name)
+            if t is not None:  # around the block nothing was written
+                o.fill_(float("nan"))
+                assert t.isnan().all(), name
 
 
 @pytest.mark.parametrize("shape", SHAPES)

@@ -173,7 +173,8 @@ int sopht_velocity_abs_sum_max_3d(int dtype, const void* const velocity[3], int6
 
 /* Looks at a real_t in pinned host memory until it is not negative (0) or limit_s seconds have
  * passed (1): the host's side of a value that a queued kernel stores there, marked as not yet
- * there by a negative one. Yields the processor between looks; makes no HIP call. */
+ * there by a negative one. Yields the processor between looks after the first 50 us; makes no HIP
+ * call. */
 int sopht_host_value_wait(int dtype, const void* value, double limit_s);
 
 /* gen_advection_flux_conservative_eno3_pyst_kernel_3d — .../advection_flux_3d.py:12-233.
@@ -243,7 +244,7 @@ typedef struct sopht_poisson3d sopht_poisson3d;
 
 /* UnboundedPoissonSolverPYFFTW3D.__init__ — .../poisson_solver_3d/UnboundedPoissonSolverPYFFTW3D.py:12-54.
  * Builds the Green's function octant (FP64 on the device) and the pass scratch. Lengths
- * 2*n per axis must factor into 2, 3 and 5 with 8 <= 2n <= 1024. */
+ * 2*n per axis must be one of 8, 12, 16, 24, 32, 48, 64, 96, 128, 192, 256, 384, 512, 768, 1024. */
 int sopht_poisson3d_create(int dtype, int64_t nz, int64_t ny, int64_t nx, double x_range,
                            void* stream, sopht_poisson3d** plan);
 /* solve — :111-149 (scalar). rhs is read only. */
@@ -257,7 +258,8 @@ int sopht_poisson3d_destroy(sopht_poisson3d* plan);
 /* Bytes of device scratch the plan holds (for capacity planning). */
 int64_t sopht_poisson3d_scratch_bytes(const sopht_poisson3d* plan);
 /* The plan's FFT schedule (no counterpart in the reference, which leaves it to FFTW's
- * planner): *passes is 3 (x transform fused with the inner y sums; FP32, 2 nx and 2 ny from 96 to 512) or 5, and
+ * planner): *passes is 3 (x transform fused with the inner y sums; 2 nx and 2 ny among 96, 128, 192, 256,
+ * 384 and, in FP32, 512, and 2 nz up to 512) or 5, and
  * *zpass_jobs the jobs per workgroup of the three-pass z pass, timed over {1, 2, 3, 6} when
  * the plan was created (SOPHT_POISSON_ZJOBS in the environment fixes it; 0 with five passes).
  * Results do not depend on it. Either pointer may be null. */

@@ -256,13 +256,15 @@ class HostScalar:
 
     _LOOK_S = 2e-3
 
-    def __init__(self, tdt):
+    def __init__(self, tdt, pinned=True):
         import torch
 
         self._tdt = tdt
         self._tag = SOPHT_F32 if tdt == torch.float32 else SOPHT_F64
-        self._t = torch.zeros((), dtype=tdt, pin_memory=True)
+        self._t = torch.zeros((), dtype=tdt, pin_memory=pinned)
         self._view = self._t.numpy()
+        self._ptr = _vp(self._t.data_ptr())
+        self._wait = lib().sopht_host_value_wait
 
     def __reduce__(self):  # a copy has pinned memory of its own
         return HostScalar, (self._tdt,)
@@ -270,11 +272,11 @@ class HostScalar:
     def arm(self):
         """The pointer for the launch that writes the value; marks the value as not yet there."""
         self._view[()] = -1.0
-        return _vp(self._t.data_ptr())
+        return self._ptr
 
     def read(self):
         """The value of the launch queued on the current stream since :meth:`arm`."""
-        if lib().sopht_host_value_wait(self._tag, self._t.data_ptr(), self._LOOK_S) != 0:
+        if self._wait(self._tag, self._ptr, self._LOOK_S) != 0:
             import torch
 
             torch.cuda.current_stream().synchronize()

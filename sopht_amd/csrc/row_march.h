@@ -338,9 +338,9 @@ enum EnoMode {
 
 // ENO3 conservative advection flux of one scalar field per gridDim.y.
 // A thread forms V + 1 x faces, two rows of y faces and one plane of z faces per plane of V
-// cells; its 13 16-byte loads per plane (field rows y-2..y+2, u_y rows y-2..y+2, u_x, u_z and
-// the field two planes up) come mostly from L1 and L2, and their rate bounds it.
-// 150 x 201 x 230 FP32, storing: 30 us (4.7 TB/s of 5 words per cell) against 94 us with one
+// cells; its 12 16-byte loads per plane (field rows y-2, y-1, y+1, y+2, u_y rows y-2..y+2, u_x, u_z
+// and the field two planes up) come mostly from L1 and L2, and their rate bounds it.
+// 150 x 201 x 230 FP32, storing: 29 us (4.7 TB/s of 5 words per cell) against 94 us with one
 // cell per thread plus 7 us for the clearing.
 template <typename T, int MODE>
 __global__ void __launch_bounds__(kRowThreads)
@@ -458,7 +458,7 @@ __device__ __forceinline__ T eno3_gather(const T* a, const T* u) {
 // that axis, then field_adj (+)= sum_axis gbar_axis u_axis, vel_adj[axis] (+)= gbar_axis field.
 // SET stores instead of adding, which spares the outputs' clearing and their read (4 of 13
 // words per cell). A gather: no atomics, the same bits on every run.
-// Bound by memory: 150 x 201 x 230 FP32, storing, 52 us (4.8 TB/s of 9 words per cell) against
+// Bound by memory: 150 x 201 x 230 FP32, storing, 53 us (4.7 TB/s of 9 words per cell) against
 // 148 us with one cell per thread, each weighing the 15 fluxes that read it, plus 19 us of clearing.
 template <typename T, bool SET>
 __global__ void __launch_bounds__(kRowThreads)

@@ -797,7 +797,8 @@ int stretching_general(void* const flux[3], const int64_t* fs, const void* const
 }
 
 // The row-vector kernel where the rows allow it (cells adjacent along x, at least one vector
-// per row, outputs apart from the velocity), else one thread per cell.
+// per row), else one thread per cell. Either reads the vorticity at the cells it writes only, so the
+// flux may replace the vorticity; a flux that meets the velocity is not defined in either.
 template <typename T>
 int stretching_impl(void* const flux[3], const int64_t* fs, const void* const w[3],
                     const int64_t* ws, const void* const u[3], const int64_t* us, int64_t nz,
@@ -968,10 +969,16 @@ int sopht_host_value_wait(int dtype, const void* value, double limit_s) {
     __atomic_load(static_cast<const double*>(value), &v, __ATOMIC_ACQUIRE);
     return !(v < 0.0);
   };
-  const auto end = std::chrono::steady_clock::now() + std::chrono::duration<double>(limit_s);
+  // the first looks come closer together than a yield takes (about 0.5 us): short waits are the ones
+  // whose end is in a small step's critical path
+  using Clock = std::chrono::steady_clock;
+  const auto start = Clock::now();
+  const auto end = start + std::chrono::duration<double>(limit_s);
+  const auto close = start + std::chrono::microseconds(50);
   while (!there()) {
-    if (std::chrono::steady_clock::now() >= end) return there() ? SOPHT_OK : 1;
-    sched_yield();
+    const auto now = Clock::now();
+    if (now >= end) return there() ? SOPHT_OK : 1;
+    if (now >= close) sched_yield();
   }
   return SOPHT_OK;
 }

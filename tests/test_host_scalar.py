@@ -27,10 +27,7 @@ def on_the_host(monkeypatch, value):
     """A scalar in ordinary memory, and the queue that its value arrives through."""
     import torch
 
-    s = L.HostScalar.__new__(L.HostScalar)
-    s._tag = L.SOPHT_F64
-    s._t = torch.zeros((), dtype=torch.float64)
-    s._view = s._t.numpy()
+    s = L.HostScalar(torch.float64, pinned=False)
     q = Queue(s, value)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda: q)
     return s, q

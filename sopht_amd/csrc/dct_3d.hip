@@ -10,7 +10,7 @@
 // Five passes per solve: x rows (two rows per transform), y columns, z columns (transform,
 // division by the eigenvalue sum, inverse transform), y columns, x rows. Along y and z two
 // neighbouring x cells are the pair, so a field is read as complex numbers as it lies.
-// Bound by memory: 10 words per cell and component. 256^3 FP32, three components: 0.385 ms (rows
+// Bound by memory: 10 words per cell and component. 256^3 FP32, three components: 0.39 ms (rows
 // 0.071 / 0.076, y columns 0.078 / 0.079, z 0.134, the last by its vector instructions: two
 // transforms and the divisions) against 1.44 ms for the six dense products; faster at every size
 // from 16^3 (0.026 against 0.041 ms) to 384^3 (1.56 against 6.95 ms).

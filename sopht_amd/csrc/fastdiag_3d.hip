@@ -16,9 +16,9 @@
 // V diag(1/l) V^-1 does not depend on the signs or scaling of the eigenvectors, so the
 // result equals the reference's to rounding.
 //
-// Grids whose axes all have a cosine-transform length (16 to 512 cells, 2^a 3^b) solve by
-// cosine transforms (dct_3d.hip), bound by memory: 256^3 FP32 with three components 0.385 ms
-// against 1.44 ms for the products below. The other grids apply the dense basis:
+// Grids whose axes all have a cosine-transform length (16, 24, 32, 48, 64, 96, 128, 192, 256, 384 or
+// 512 cells) solve by cosine transforms (dct_3d.hip), bound by memory: 256^3 FP32 with three
+// components 0.39 ms against 1.44 ms for the products below. The other grids apply the dense basis:
 //
 // Device work per such solve: six GEMMs on the MFMA units through rocBLAS (the three components
 // of a vector field batched into each) and one elementwise spectral scaling. For an N^3

@@ -237,7 +237,9 @@ constexpr bool kTwiddleProducts = SOPHT_TWIDDLE_PRODUCTS;
 // other pattern leaves free, so on gfx950 (64-bit accesses served 32 lanes at a time by 64
 // four-byte banks) both patterns are conflict-free for the plan of 64 points and every plan from
 // 128 points on (checked exhaustively on the host). The map is an involution on [0, L). The other
-// lines keep the identity.
+// lines keep the identity. The counters see more than this model: 9 to 31% of the FP32 passes' LDS
+// cycles are conflicts, and 37 to 46% of the FP64 ones', whose 16-byte elements are served 16 lanes
+// at a time.
 template <int L, int NS, int R>
 struct Swizzle {
   static constexpr int T = LinePlan<L>::T;
@@ -257,8 +259,9 @@ struct Swizzle {
 // regions start 16 slots apart (mod 32), those of 64-point lines 8. Shorter teams' other lines keep
 // the identity map, whose writes step by the radix, so their regions start 9 apart (2 for teams
 // of 2): an exchange of 24, 32, 48 or 96 points then meets 1.5 to 2 lanes per bank on average,
-// against 4, 6, 8 and 3 at 16 (counted on the host). Column tiles stage WC = 8 columns with lanes (column, row); a stride of 4
-// (mod 32) between column regions keeps those accesses conflict-free too.
+// against 4, 6, 8 and 3 at 16 (counted on the host). Column tiles stage WC = 8 columns with lanes
+// (column, row); by the same count a stride of 4 (mod 32) between column regions keeps those
+// accesses conflict-free too.
 template <int L, bool COLUMN>
 constexpr int region_stride() {
   if (LinePlan<L>::T <= 2) return L + 2;

@@ -88,8 +88,7 @@ int step_impl(sopht_ns3d* P, const void* vort_in, void* vort_out, const void* ve
   const int s1_chunk = P->s1_chunk;
   const S1Map s1m{int(ceil_div(g.nx, s1_cols)), int(ceil_div(g.ny, s1_rows)), s1_rows, s1_chunk, s1_cols};
   const int64_t s1_items = int64_t(s1m.tiles_x) * s1m.tiles_y * ceil_div(g.nz, s1_chunk);
-  const bool flags_ok = s1_items <= P->s1flags_cap;
-  int* const fflags = flags_ok ? P->s1flags : nullptr;
+  int* const fflags = P->s1flags;  // one per item
   {
     const int remap = s1_items % 8 == 0 ? 1 : 0;
     if constexpr (sizeof(T) == 4) {

@@ -44,7 +44,9 @@ struct ZRowTile {
   static constexpr int NT = SLOTS * WC * TT;
   // tiles [slot][column]: the load role's lanes (column, z) hit distinct banks when the column
   // stride is 8 (mod 32) slots, or 4 (mod 16) of the 16-byte FP64 ones, which are served 16 lanes
-  // at a time; FP32 teams of 16 need 16 for their exchanges, shorter ones 9 as elsewhere
+  // at a time; FP32 teams of 16 need 16 for their exchanges, shorter ones 9 as elsewhere. (Conflict
+  // cycles of the whole pass, by the counters: 26% of its LDS cycles in FP32, 37% at L = 128 and 43% at
+  // L = 384 in FP64.)
   static constexpr int S = TT < 16 ? region_stride<L, true>()
                            : sizeof(T) == 8 ? L + 4
                            : TT < 32 ? L + 16 : (WC == 4 ? L + 8 : L + 4);

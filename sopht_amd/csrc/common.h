@@ -97,6 +97,38 @@ __device__ __forceinline__ int xcd_run(int blocks, int b) {
 
 inline int ceil_div(int64_t a, int64_t b) { return static_cast<int>((a + b - 1) / b); }
 
+// A kernel that needs more than the default 64 KB of LDS says so before its launch.
+template <typename K>
+inline int allow_lds(K* kernel, size_t bytes) {
+  if (bytes <= 65536) return SOPHT_OK;
+  SOPHT_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)));
+  return SOPHT_OK;
+}
+
+// The largest of nb non-negative partial maxima; out may be pinned host memory. One workgroup,
+// bound by latency: 1024 threads leave few loads in turn, and the maxima meet by lane exchanges.
+template <typename T>
+__global__ void __launch_bounds__(1024) k_max_final(const T* __restrict__ partial, int nb, T* __restrict__ out) {
+  __shared__ T red[16];
+  T m = T(0);
+#pragma unroll 4
+  for (int i = threadIdx.x; i < nb; i += 1024) m = partial[i] > m ? partial[i] : m;
+  for (int k = 32; k > 0; k >>= 1) {
+    const T o = __shfl_xor(m, k, 64);
+    m = o > m ? o : m;
+  }
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  m = threadIdx.x < 16 ? red[threadIdx.x] : T(0);
+  for (int k = 8; k > 0; k >>= 1) {
+    const T o = __shfl_xor(m, k, 64);
+    m = o > m ? o : m;
+  }
+  if (threadIdx.x == 0) *out = m;
+}
+
 // Per-stage timing with HIP events recorded on the launch stream between consecutive
 // kernels of a step. Two event sets alternate between steps, so harvesting the set of
 // step k-2 before reusing it never waits on work that is still queued behind step k-1.

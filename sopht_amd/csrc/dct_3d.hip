@@ -280,15 +280,6 @@ int with_length(int64_t n, Fn&& fn) {
   return SOPHT_ERR_UNSUPPORTED;
 }
 
-// A kernel that needs more than the default 64 KB of LDS says so before its launch.
-template <typename K>
-int allow_lds(K kernel, size_t bytes) {
-  if (bytes > 65536)
-    SOPHT_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)));
-  return SOPHT_OK;
-}
-
 template <typename T, bool INV>
 int rows_pass(DctPlan* P, const T* in, T* out, int ncomp, hipStream_t s) {
   return with_length(P->n[2], [&](auto l) -> int {

@@ -378,15 +378,6 @@ __global__ void __launch_bounds__((XYPass<T, LX, LY>::NT)) kc_yx_inv(SlabGeom g,
   });
 }
 
-// Workgroups above 64 KB of LDS declare it once per kernel.
-template <typename K>
-int allow_lds(K* kernel, size_t bytes) {
-  if (bytes <= 65536) return SOPHT_OK;
-  SOPHT_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)));
-  return SOPHT_OK;
-}
-
 // fn(integral_constant<LX>, integral_constant<LY>) for the lengths of precision T.
 template <typename T, int LX, typename Fn>
 int with_xy_y(int64_t LY, Fn&& fn) {

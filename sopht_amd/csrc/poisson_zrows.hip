@@ -229,15 +229,6 @@ __global__ void __launch_bounds__((ZRowTile<T, L>::NT)) __attribute__((amdgpu_wa
   }
 }
 
-// Workgroups above 64 KB of LDS declare it once per kernel.
-template <typename K>
-int allow_lds(K* kernel, size_t bytes) {
-  if (bytes <= 65536) return SOPHT_OK;
-  SOPHT_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)));
-  return SOPHT_OK;
-}
-
 template <typename T>
 int z_rows(int64_t L, SlabGeom g, Cplx<T>* H, const T* ghat, const Cplx<T>* tw,
                    hipStream_t s, int jobs) {

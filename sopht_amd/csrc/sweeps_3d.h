@@ -907,29 +907,5 @@ __global__ void __launch_bounds__(256) k_max_abs_sum(const T* u, int64_t n, T* p
   if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
 }
 
-// The largest of nb non-negative partial maxima; out may be pinned host memory. One workgroup,
-// bound by latency: 1024 threads leave few loads in turn, and the maxima meet by lane exchanges.
-template <typename T>
-__global__ void __launch_bounds__(1024) k_max_final(const T* __restrict__ partial, int nb, T* __restrict__ out) {
-  __shared__ T red[16];
-  T m = T(0);
-#pragma unroll 4
-  for (int i = threadIdx.x; i < nb; i += 1024) m = partial[i] > m ? partial[i] : m;
-  for (int k = 32; k > 0; k >>= 1) {
-    const T o = __shfl_xor(m, k, 64);
-    m = o > m ? o : m;
-  }
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-  __syncthreads();
-  if (threadIdx.x >= 64) return;
-  m = threadIdx.x < 16 ? red[threadIdx.x] : T(0);
-  for (int k = 8; k > 0; k >>= 1) {
-    const T o = __shfl_xor(m, k, 64);
-    m = o > m ? o : m;
-  }
-  if (threadIdx.x == 0) *out = m;
-}
-
-
 }  // namespace
 }  // namespace sopht

@@ -88,29 +88,6 @@ __global__ void __launch_bounds__(256) k_abs_sum_max(const T* __restrict__ u0, c
   if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
 }
 
-// The largest of nb non-negative partial maxima; out may be pinned host memory. One workgroup,
-// bound by latency: 1024 threads leave few loads in turn, and the maxima meet by lane exchanges.
-template <typename T>
-__global__ void __launch_bounds__(1024) k_partial_max(const T* __restrict__ partial, int nb, T* __restrict__ out) {
-  __shared__ T red[16];
-  T m = T(0);
-#pragma unroll 4
-  for (int i = threadIdx.x; i < nb; i += 1024) m = partial[i] > m ? partial[i] : m;
-  for (int k = 32; k > 0; k >>= 1) {
-    const T o = __shfl_xor(m, k, 64);
-    m = o > m ? o : m;
-  }
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-  __syncthreads();
-  if (threadIdx.x >= 64) return;
-  m = threadIdx.x < 16 ? red[threadIdx.x] : T(0);
-  for (int k = 8; k > 0; k >>= 1) {
-    const T o = __shfl_xor(m, k, 64);
-    m = o > m ? o : m;
-  }
-  if (threadIdx.x == 0) *out = m;
-}
-
 template <typename T>
 int abs_sum_max(const void* const vel[3], int64_t n, void* mag, void* partial, int64_t cap, void* out,
                 hipStream_t s) {
@@ -119,7 +96,7 @@ int abs_sum_max(const void* const vel[3], int64_t n, void* mag, void* partial, i
                                       static_cast<const T*>(vel[2]), n, static_cast<T*>(mag),
                                       static_cast<T*>(partial));
   SOPHT_CHECK_LAUNCH();
-  k_partial_max<T><<<1, 1024, 0, s>>>(static_cast<const T*>(partial), nb, static_cast<T*>(out));
+  k_max_final<T><<<1, 1024, 0, s>>>(static_cast<const T*>(partial), nb, static_cast<T*>(out));
   SOPHT_CHECK_LAUNCH();
   return SOPHT_OK;
 }

@@ -130,6 +130,17 @@ def test_stretching_step_with_one_buffer_for_flux_and_midstep(dev, real_t):
     np.testing.assert_allclose(to_host(bd), buf, atol=bound, rtol=0)
 
 
+@pytest.mark.parametrize("shape", [(3, 3, 4), (9, 20, 37), (34, 5, 66)])
+def test_stretching_flux_in_place_of_the_vorticity(dev, real_t, shape):
+    # either kernel reads the vorticity at the cells it writes only
+    rng = np.random.default_rng(18)
+    w, u = rng.uniform(-1, 1, (2, 3, *shape)).astype(real_t)
+    flux = np.zeros((3, *shape))
+    S.vorticity_stretching_flux(flux, w.astype(np.float64), u.astype(np.float64), 0.25)
+    kernel = spne().gen_vorticity_stretching_flux_pyst_kernel_3d(real_t)
+    both(lambda o, i: kernel(o[0], o[0], i[0], 0.25), [w], [u], dev, [flux], 2 * 9 * float(np.finfo(real_t).eps) * 2)
+
+
 @pytest.mark.parametrize("shape", [(5, 5, 5), (6, 5, 6), (9, 7, 37), (36, 6, 66), (7, 5, 1031), (40, 12, 256)])
 def test_eno3_flux_and_step(dev, real_t, shape):
     rng = np.random.default_rng(13)
